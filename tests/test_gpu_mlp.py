@@ -78,3 +78,24 @@ def test_training_reduces_the_loss_and_params_round_trip():
     other.set_params(p)
     assert np.array_equal(other.params(), p)
     assert np.array_equal(other.forward(x[:32]), net.forward(x[:32]))
+
+
+# the smallest of every size; rows, inputs and widths that are no multiple of
+# a tile or of the unrolled steps; several blocks of rows per wavefront.  The
+# file's FP64 bar, 2e-2: a tile or a block of rows read or written wrongly
+# moves a layer's gradient by several times that.
+@pytest.mark.parametrize("n_in,width,n_hidden,n_out,B",
+                         [(1, 32, 1, 32, 1), (32, 96, 2, 64, 33), (5, 160, 4, 32, 257), (4, 256, 3, 256, 544)])
+def test_gradients_at_the_edges_of_the_tiles(n_in, width, n_hidden, n_out, B):
+    print(f"case mlp gradients {n_in}-{width}x{n_hidden}-{n_out} B={B}", flush=True)
+    net = MLP(n_in=n_in, width=width, n_hidden=n_hidden, n_out=n_out, max_batch=B, seed=3)
+    rng = np.random.default_rng(4)
+    x = rng.uniform(-1, 1, (B, n_in)).astype(np.float32)
+    t = rng.uniform(-1, 1, (B, n_out)).astype(np.float32)
+    loss, g = net.gradients(x, t)
+    Ws, bs = mlp_ref.unflatten(net.params(), n_in, width, n_hidden, n_out)
+    lp, gWp, gbp = mlp_ref.loss_and_grads(Ws, bs, x, t, emulate=False)
+    assert abs(loss - lp) <= 2e-2 * lp
+    gW, gb = mlp_ref.unflatten(g, n_in, width, n_hidden, n_out)
+    for l in range(n_hidden + 1):
+        assert _rel(gW[l], gWp[l]) <= 2e-2 and _rel(gb[l], gbp[l]) <= 2e-2, l
