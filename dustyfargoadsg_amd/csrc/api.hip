@@ -29,6 +29,13 @@
                               hipGetErrorString(e_), __FILE__, __LINE__);                   \
   } while (0)
 
+// Sub-steps per launched graph.  The kernels of one graph follow each other
+// without a gap, two graphs on a stream lie 8 us apart (measured between the
+// last kernel of a sub-step and the first of the next, 200x400 and 1024x3072):
+// a sub-step of the smaller discs takes 40-80 us, so a call's sub-steps are
+// launched in runs.  Longer runs are instantiated when a call first needs one.
+static constexpr int kRunLength[3] = {1, 4, 16};
+
 struct dfargo_ctx {
   dfargo_params p;
   int prec = DFARGO_FP64, dev = 0;
@@ -39,8 +46,12 @@ struct dfargo_ctx {
   KArgs a;
   dfargo_ctrl *d_ctrl = nullptr, *h_ctrl = nullptr;
   std::vector<int> seq; // kernel ids of one sub-step
+  // the sub-step as a graph, and executables of runs of kRunLength[k] of it
   hipGraph_t graph = nullptr;
-  hipGraphExec_t gexec = nullptr;
+  hipGraphExec_t gexec[3] = {nullptr, nullptr, nullptr};
+  // sub-steps and length of the last AlgoGas call: how many to enqueue before
+  // the next call first reads the control block back
+  double last_DT = 0.0;
   long graph_version = 0; // bumped whenever the captured sub-step is dropped
   int initialized = 0, profiling = 0;
   double kt_ms[KID_COUNT];
@@ -159,9 +170,10 @@ static int check_frame_planets(const dfargo_params &p, const dfargo_planets *s) 
 // a change of what the sub-step launches drops the graph, so that the next
 // sub-step captures it again
 static int drop_graph(dfargo_ctx *c) {
-  if (c->gexec) {
-    HIPCHK(hipGraphExecDestroy(c->gexec));
-    c->gexec = nullptr;
+  for (hipGraphExec_t &g : c->gexec) {
+    if (!g) continue;
+    HIPCHK(hipGraphExecDestroy(g));
+    g = nullptr;
   }
   if (c->graph) {
     HIPCHK(hipGraphDestroy(c->graph));
@@ -235,47 +247,75 @@ static void call_start(dfargo_ctx *c, double DT, hipStream_t s) {
   }
 }
 
-static int ensure_graph(dfargo_ctx *c);
+static int ensure_graph(dfargo_ctx *c, int level);
 
-static int run_substep(dfargo_ctx *c) {
-  if (c->profiling) {
-    // one event pair per kernel from a pool; collected once per sub-step
-    const size_t nk = c->seq.size();
-    while (c->evpool.size() < 2 * nk) {
-      hipEvent_t e;
-      HIPCHK(hipEventCreate(&e));
-      c->evpool.push_back(e);
-    }
-    for (size_t q = 0; q < nk; q++) {
-      HIPCHK(hipEventRecord(c->evpool[2 * q], c->stream));
-      launch_id(c, c->seq[q]);
-      HIPCHK(hipGetLastError());
-      HIPCHK(hipEventRecord(c->evpool[2 * q + 1], c->stream));
-    }
-    HIPCHK(hipEventSynchronize(c->evpool[2 * nk - 1]));
-    for (size_t q = 0; q < nk; q++) {
-      float ms = 0.f;
-      HIPCHK(hipEventElapsedTime(&ms, c->evpool[2 * q], c->evpool[2 * q + 1]));
-      c->kt_ms[c->seq[q]] += ms;
-      c->kt_n[c->seq[q]] += 1;
-    }
-    return DFARGO_OK;
+// one sub-step, each kernel timed
+static int profiled_substep(dfargo_ctx *c) {
+  // one event pair per kernel from a pool; collected once per sub-step
+  const size_t nk = c->seq.size();
+  while (c->evpool.size() < 2 * nk) {
+    hipEvent_t e;
+    HIPCHK(hipEventCreate(&e));
+    c->evpool.push_back(e);
   }
-  int rc = ensure_graph(c);
-  if (rc) return rc;
-  HIPCHK(hipGraphLaunch(c->gexec, c->stream));
+  for (size_t q = 0; q < nk; q++) {
+    HIPCHK(hipEventRecord(c->evpool[2 * q], c->stream));
+    launch_id(c, c->seq[q]);
+    HIPCHK(hipGetLastError());
+    HIPCHK(hipEventRecord(c->evpool[2 * q + 1], c->stream));
+  }
+  HIPCHK(hipEventSynchronize(c->evpool[2 * nk - 1]));
+  for (size_t q = 0; q < nk; q++) {
+    float ms = 0.f;
+    HIPCHK(hipEventElapsedTime(&ms, c->evpool[2 * q], c->evpool[2 * q + 1]));
+    c->kt_ms[c->seq[q]] += ms;
+    c->kt_n[c->seq[q]] += 1;
+  }
   return DFARGO_OK;
 }
 
-// The sub-step's kernel list captured once as a graph (c->graph) and
-// instantiated (c->gexec).
-static int ensure_graph(dfargo_ctx *c) {
-  if (!c->gexec) {
+// the longest run of at most n sub-steps, launched; returns how many in *done
+static int launch_run(dfargo_ctx *c, int n, int *done) {
+  int level = 2;
+  while (level > 0 && kRunLength[level] > n) level--;
+  int rc = ensure_graph(c, level);
+  if (rc) return rc;
+  HIPCHK(hipGraphLaunch(c->gexec[level], c->stream));
+  *done = kRunLength[level];
+  return DFARGO_OK;
+}
+static int run_substeps(dfargo_ctx *c, int n) {
+  int rc, done = 0;
+  while (n > 0) {
+    if (c->profiling) {
+      if ((rc = profiled_substep(c))) return rc;
+      done = 1;
+    } else if ((rc = launch_run(c, n, &done)))
+      return rc;
+    n -= done;
+  }
+  return DFARGO_OK;
+}
+
+// The sub-steps a call of length DT most likely needs at least, from the last
+// call's: one fewer, since a sub-step enqueued after the last still launches
+// its kernels (which return at once), and a missing one only costs the
+// read-back between.
+static int first_batch(const dfargo_ctx *c, double DT) {
+  const dfargo_ctrl *k = c->h_ctrl;
+  if (!(c->last_DT > 0.0) || k->substeps < 2) return 1;
+  const double n = floor((double)k->substeps * DT / c->last_DT) - 1.0;
+  return (int)std::min(std::max(n, 1.0), 4096.0);
+}
+
+// The sub-step's kernel list captured `n` times over into *graph.
+static int capture_substeps(dfargo_ctx *c, int n, hipGraph_t *graph) {
+  HIPCHK(hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
+  for (int k = 0; k < n; k++) {
     // The self-gravity transforms read only the density the sub-step starts
     // with and feed only the source kernel: in the graph they form a branch
     // of their own, beside the CFL, control and particle kernels, joined
     // before k_source.
-    HIPCHK(hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
     const bool fork = c->p.self_gravity != 0;
     if (fork) {
       HIPCHK(hipEventRecord(c->ev_fork, c->stream));
@@ -294,10 +334,23 @@ static int ensure_graph(dfargo_ctx *c) {
       }
       launch_id(c, id);
     }
-    hipError_t e = hipStreamEndCapture(c->stream, &c->graph);
-    if (e != hipSuccess) return dfargo_set_error(DFARGO_ERR_HIP, "graph capture failed: %s", hipGetErrorString(e));
-    HIPCHK(hipGraphInstantiate(&c->gexec, c->graph, nullptr, nullptr, 0));
   }
+  hipError_t e = hipStreamEndCapture(c->stream, graph);
+  if (e != hipSuccess) return dfargo_set_error(DFARGO_ERR_HIP, "graph capture failed: %s", hipGetErrorString(e));
+  return DFARGO_OK;
+}
+
+// the run of kRunLength[level] sub-steps, captured and instantiated once; the
+// single sub-step's graph is kept for the batches, which make it a child
+static int ensure_graph(dfargo_ctx *c, int level) {
+  if (c->gexec[level]) return DFARGO_OK;
+  hipGraph_t g = nullptr;
+  int rc = capture_substeps(c, kRunLength[level], &g);
+  if (rc) return rc;
+  hipError_t e = hipGraphInstantiate(&c->gexec[level], g, nullptr, nullptr, 0);
+  if (level == 0 && e == hipSuccess) c->graph = g;
+  else hipGraphDestroy(g);
+  HIPCHK(e);
   return DFARGO_OK;
 }
 
@@ -696,7 +749,8 @@ extern "C" int dfargo_destroy(dfargo_ctx *c) {
   if (!c) return DFARGO_OK;
   hipSetDevice(c->dev);
   if (c->stream) hipStreamSynchronize(c->stream);
-  if (c->gexec) hipGraphExecDestroy(c->gexec);
+  for (hipGraphExec_t g : c->gexec)
+    if (g) hipGraphExecDestroy(g);
   if (c->graph) hipGraphDestroy(c->graph);
   for (void *p : c->allocs) hipFree(p);
   if (c->h_ctrl) hipHostFree(c->h_ctrl);
@@ -954,14 +1008,14 @@ extern "C" int dfargo_algogas_device(dfargo_ctx *c, double DT) {
   call_start(c, DT, c->stream);
   HIPCHK(hipGetLastError());
   long launched = 0;
-  int batch = 1, rc;
+  int batch = first_batch(c, DT), rc;
   const long cap = 50000000L;
   for (;;) {
-    for (int b = 0; b < batch; b++)
-      if ((rc = run_substep(c))) return rc;
+    if ((rc = run_substeps(c, batch))) return rc;
     launched += batch;
     if ((rc = ctrl_pull(c))) return rc;
     const dfargo_ctrl *k = c->h_ctrl;
+    c->last_DT = DT;
     if (!(k->dtemp < 0.999999999 * DT)) break;
     if (launched > cap)
       return dfargo_set_error(DFARGO_ERR_STATE, "more than %ld sub-steps in one AlgoGas call", cap);
@@ -979,8 +1033,8 @@ extern "C" int dfargo_run_substeps(dfargo_ctx *c, double DT, int nsub) {
   call_start(c, DT, c->stream);
   HIPCHK(hipGetLastError());
   int rc;
-  for (int b = 0; b < nsub; b++)
-    if ((rc = run_substep(c))) return rc;
+  c->last_DT = 0.0; // a call left open says nothing about the next one
+  if ((rc = run_substeps(c, nsub))) return rc;
   HIPCHK(hipStreamSynchronize(c->stream));
   return DFARGO_OK;
 }
@@ -1929,7 +1983,7 @@ extern "C" int dfargo_batch_create(dfargo_ctx *const *discs, int n, dfargo_batch
   if (e == hipSuccess) e = hipGraphCreate(&b->graph, 0);
   for (int i = 0; i < n && e == hipSuccess && !rc; i++) {
     dfargo_ctx *c = b->d[i];
-    if ((rc = ensure_graph(c))) break;
+    if ((rc = ensure_graph(c, 0))) break;
     b->version.push_back(c->graph_version);
     hipGraphNode_t node;
     e = hipGraphAddChildGraphNode(&node, b->graph, nullptr, 0, c->graph);
@@ -1963,16 +2017,25 @@ static int batch_streams(dfargo_batch *b) {
     call_start(c, b->DT[i], c->stream);
   }
   HIPCHK(hipGetLastError());
-  std::vector<int> rem(n, 1);
+  std::vector<int> rem(n);
+  for (int i = 0; i < n; i++) rem[i] = first_batch(b->d[i], b->DT[i]);
   long launched = 0;
   const long cap = 50000000L;
   for (;;) {
     int most = 0;
     for (int i = 0; i < n; i++) most = std::max(most, rem[i]);
     if (most == 0) break;
-    for (int r = 0; r < most; r++)
-      for (int i = 0; i < n; i++)
-        if (rem[i] > r) HIPCHK(hipGraphLaunch(b->d[i]->gexec, b->d[i]->stream));
+    std::vector<int> left(rem);
+    for (bool more = true; more;) {
+      more = false;
+      for (int i = 0; i < n; i++) {
+        if (left[i] <= 0) continue;
+        int done = 0, rc = launch_run(b->d[i], left[i], &done);
+        if (rc) return rc;
+        left[i] -= done;
+        more = more || left[i] > 0;
+      }
+    }
     launched += most;
     for (int i = 0; i < n; i++)
       if (rem[i] > 0)
@@ -1984,6 +2047,7 @@ static int batch_streams(dfargo_batch *b) {
       if (rem[i] == 0) continue;
       const dfargo_ctrl *k = b->d[i]->h_ctrl;
       rem[i] = 0;
+      b->d[i]->last_DT = b->DT[i];
       if (k->dtemp < 0.999999999 * b->DT[i])
         rem[i] = (int)std::min(std::max(ceil((b->DT[i] - k->dtemp) / (k->dt > 0.0 ? k->dt : b->DT[i])), 1.0),
                                4096.0);
@@ -2027,6 +2091,7 @@ extern "C" int dfargo_batch_algogas(dfargo_batch *b, const double *DT) {
     double rem = 0.0;
     for (int i = 0; i < n; i++) {
       const dfargo_ctrl *k = b->d[i]->h_ctrl;
+      b->d[i]->last_DT = b->DT[i];
       if (k->dtemp < 0.999999999 * b->DT[i])
         rem = std::max(rem, ceil((b->DT[i] - k->dtemp) / (k->dt > 0.0 ? k->dt : b->DT[i])));
     }
