@@ -53,7 +53,7 @@ __device__ __forceinline__ double df_stokes_at(const KArgs &a, double lam, doubl
 // the physical viscosity always.  Like the gas's CFL kernel it multiplies
 // by the ring's reciprocal cell sizes.
 __global__ void __launch_bounds__(256) k_df_cfl(KArgs a) {
-  __shared__ double sh[1024];
+  __shared__ double sh[16];
   const dfargo_ctrl *c = a.ctrl;
   if (!c->go) return;
   const int i = blockIdx.x, ns = a.ns, tid = threadIdx.x, TB = blockDim.x;
@@ -61,7 +61,7 @@ __global__ void __launch_bounds__(256) k_df_cfl(KArgs a) {
   const double *dvr = a.dvr + base, *dvt = a.dvt + base;
   double s = 0.0;
   for (int j = tid; j < ns; j += TB) s += dvt[j];
-  s = block_sum_fast(s, sh);
+  s = block_sum(s, sh);
   const double dvmoy = s / (double)ns;
   if (tid == 0) a.dvmoy[i] = dvmoy;
   if (i < 1) {
@@ -95,20 +95,20 @@ __global__ void __launch_bounds__(256) k_df_cfl(KArgs a) {
     smax = (S > smax) ? S : smax;
   }
   // the largest sum gives the smallest dt (the map is monotone)
-  smax = -block_min_fast(-smax, sh);
+  smax = -block_min(-smax, sh);
   if (tid == 0) a.df_ring_dt[i] = DF_CFLSECURITY / sqrt(smax);
 }
 
 // ring means of SG_Accr (mpi_make1Dprofile for DUSTFEELSG Z,
 // src/sgupdate.c:26-27), one workgroup per ring
 __global__ void __launch_bounds__(256) k_df_axisg(KArgs a) {
-  __shared__ double sh[1024];
+  __shared__ double sh[16];
   const dfargo_ctrl *c = a.ctrl;
   if (!c->active) return;
   const int i = blockIdx.x, ns = a.ns;
   double s = 0.0;
   for (int j = threadIdx.x; j < ns; j += blockDim.x) s += ((const double *)a.sgr)[(long)i * ns + j];
-  s = block_sum_fast(s, sh);
+  s = block_sum(s, sh);
   if (threadIdx.x == 0) a.df_axisg[i] = s / (double)ns;
 }
 

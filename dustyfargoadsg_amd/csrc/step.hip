@@ -103,129 +103,74 @@ template <> struct TransportArith<float> {
 __device__ __forceinline__ double dmin2(double a, double b) { return (b < a) ? b : a; }
 __device__ __forceinline__ double dmax2(double a, double b) { return (b > a) ? b : a; }
 
-// the sum over a wavefront, the same in every lane (xor butterfly)
+// Sum and minimum over a wavefront, the same in every lane, in a fixed order:
+// four row shifts and two row broadcasts by DPP (VALU moves) leave the total
+// in lane 63.  A shuffle butterfly goes through the LDS crossbar twelve times
+// for a double, each step waiting for the one before.
+template <int CTRL, int ROWS> __device__ __forceinline__ double dpp_row(double v, double other) {
+  const int lo = __double2loint(v), hi = __double2hiint(v);
+  return __hiloint2double(__builtin_amdgcn_update_dpp(__double2hiint(other), hi, CTRL, ROWS, 0xf, false),
+                          __builtin_amdgcn_update_dpp(__double2loint(other), lo, CTRL, ROWS, 0xf, false));
+}
+__device__ __forceinline__ double lane63(double v) {
+  return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), 63),
+                          __builtin_amdgcn_readlane(__double2loint(v), 63));
+}
+// row_shr:1, 2, 4, 8 = 0x111, 0x112, 0x114, 0x118; row_bcast:15, :31 = 0x142,
+// 0x143 (into the rows 1 and 3, then 2 and 3); lanes without a source take
+// the neutral value
 __device__ __forceinline__ double wave_sum(double v) {
-  for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
-  return v;
+  v += dpp_row<0x111, 0xf>(v, 0.0);
+  v += dpp_row<0x112, 0xf>(v, 0.0);
+  v += dpp_row<0x114, 0xf>(v, 0.0);
+  v += dpp_row<0x118, 0xf>(v, 0.0);
+  v += dpp_row<0x142, 0xa>(v, 0.0);
+  v += dpp_row<0x143, 0xc>(v, 0.0);
+  return lane63(v);
+}
+__device__ __forceinline__ double wave_min(double v) {
+  v = dmin2(v, dpp_row<0x111, 0xf>(v, v));
+  v = dmin2(v, dpp_row<0x112, 0xf>(v, v));
+  v = dmin2(v, dpp_row<0x114, 0xf>(v, v));
+  v = dmin2(v, dpp_row<0x118, 0xf>(v, v));
+  v = dmin2(v, dpp_row<0x142, 0xa>(v, v));
+  v = dmin2(v, dpp_row<0x143, 0xc>(v, v));
+  return lane63(v);
 }
 
-// deterministic block reductions (fixed tree for a given blockDim)
-__device__ double block_sum(double v, double *sh) {
-  int t = threadIdx.x, TB = blockDim.x, P = 1;
-  while (P * 2 <= TB) P *= 2;
-  sh[t] = v;
-  __syncthreads();
-  if (t < TB - P) sh[t] += sh[t + P];
-  __syncthreads();
-  for (int s = P / 2; s > 0; s >>= 1) {
-    if (t < s) sh[t] += sh[t + s];
-    __syncthreads();
-  }
-  double r = sh[0];
-  __syncthreads();
-  return r;
-}
-__device__ double block_min(double v, double *sh) {
-  int t = threadIdx.x, TB = blockDim.x, P = 1;
-  while (P * 2 <= TB) P *= 2;
-  sh[t] = v;
-  __syncthreads();
-  if (t < TB - P) sh[t] = dmin2(sh[t], sh[t + P]);
-  __syncthreads();
-  for (int s = P / 2; s > 0; s >>= 1) {
-    if (t < s) sh[t] = dmin2(sh[t], sh[t + s]);
-    __syncthreads();
-  }
-  double r = sh[0];
-  __syncthreads();
-  return r;
-}
-// N sums at once: wavefront shuffle trees, then one pass over the wave
-// partials (blocks that are whole wavefronts), else the LDS tree.  sh must
-// hold 17*N doubles (and blockDim doubles for the fallback).
-template <int N> __device__ void block_sum_n(double (&v)[N], double *sh) {
-  const int TB = blockDim.x;
-  if (TB % 64 != 0) {
+// The same over a block of whole wavefronts, the wavefronts' values in
+// wavefront order; every thread gets the results.  sh holds 16 N doubles and
+// may be used again after the return.
+template <int N> __device__ __forceinline__ void block_sum_n(double (&v)[N], double *sh) {
+  const int wave = threadIdx.x >> 6, nw = blockDim.x >> 6;
 #pragma unroll
-    for (int k = 0; k < N; k++) v[k] = block_sum(v[k], sh);
-    return;
+  for (int k = 0; k < N; k++) {
+    const double s = wave_sum(v[k]);
+    if ((threadIdx.x & 63) == 0) sh[wave * N + k] = s;
   }
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nw = TB >> 6;
-#pragma unroll
-  for (int k = 0; k < N; k++)
-    for (int off = 32; off > 0; off >>= 1) v[k] += __shfl_down(v[k], off, 64);
-  if (lane == 0)
-#pragma unroll
-    for (int k = 0; k < N; k++) sh[wave * N + k] = v[k];
   __syncthreads();
-  if (threadIdx.x < N) {
+#pragma unroll
+  for (int k = 0; k < N; k++) {
     double s = 0.0;
-    for (int w = 0; w < nw; w++) s += sh[w * N + threadIdx.x];
-    sh[16 * N + threadIdx.x] = s;
+    for (int w = 0; w < nw; w++) s += sh[w * N + k];
+    v[k] = s;
   }
   __syncthreads();
-#pragma unroll
-  for (int k = 0; k < N; k++) v[k] = sh[16 * N + k];
-  __syncthreads();
 }
-__device__ double block_sum_fast(double v, double *sh) {
+__device__ __forceinline__ double block_sum(double v, double *sh) {
   double w[1] = {v};
   block_sum_n<1>(w, sh);
   return w[0];
 }
-__device__ double block_min_fast(double v, double *sh) {
-  const int TB = blockDim.x;
-  if (TB % 64 != 0) return block_min(v, sh);
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nw = TB >> 6;
-  for (int off = 32; off > 0; off >>= 1) v = dmin2(v, __shfl_down(v, off, 64));
-  if (lane == 0) sh[wave] = v;
+__device__ __forceinline__ double block_min(double v, double *sh) {
+  const int nw = blockDim.x >> 6;
+  v = wave_min(v);
+  if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = v;
   __syncthreads();
-  if (threadIdx.x == 0) {
-    double m = sh[0];
-    for (int w = 1; w < nw; w++) m = dmin2(m, sh[w]);
-    sh[16] = m;
-  }
+  double m = sh[0];
+  for (int w = 1; w < nw; w++) m = dmin2(m, sh[w]);
   __syncthreads();
-  double r = sh[16];
-  __syncthreads();
-  return r;
-}
-
-// N sums and one minimum in one pass (same scheme as block_sum_n); sh
-// must hold 17*(N+1) doubles (and blockDim doubles for the fallback).
-template <int N> __device__ void block_sum_min_n(double (&v)[N], double &mn, double *sh) {
-  const int TB = blockDim.x;
-  if (TB % 64 != 0) {
-#pragma unroll
-    for (int k = 0; k < N; k++) v[k] = block_sum(v[k], sh);
-    mn = block_min(mn, sh);
-    return;
-  }
-  const int M = N + 1, lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nw = TB >> 6;
-#pragma unroll
-  for (int k = 0; k < N; k++)
-    for (int off = 32; off > 0; off >>= 1) v[k] += __shfl_down(v[k], off, 64);
-  for (int off = 32; off > 0; off >>= 1) mn = dmin2(mn, __shfl_down(mn, off, 64));
-  if (lane == 0) {
-#pragma unroll
-    for (int k = 0; k < N; k++) sh[wave * M + k] = v[k];
-    sh[wave * M + N] = mn;
-  }
-  __syncthreads();
-  if (threadIdx.x < N) {
-    double s = 0.0;
-    for (int w = 0; w < nw; w++) s += sh[w * M + threadIdx.x];
-    sh[16 * M + threadIdx.x] = s;
-  } else if (threadIdx.x == N) {
-    double m = sh[N];
-    for (int w = 1; w < nw; w++) m = dmin2(m, sh[w * M + N]);
-    sh[16 * M + N] = m;
-  }
-  __syncthreads();
-#pragma unroll
-  for (int k = 0; k < N; k++) v[k] = sh[16 * M + k];
-  mn = sh[16 * M + N];
-  __syncthreads();
+  return m;
 }
 
 // Neumaier-compensated running sum
@@ -428,149 +373,215 @@ __global__ void k_algogas_begin(KArgs a, double DT) {
 // per-ring partial sums of ComputeForce (src/Force.c:155-214), GasTotalMass
 // and the barycentre (src/SideEuler.c:15-77) and DetectCrash
 // (src/SourceEuler.c:51-69): one read of rho, vr, vt (and cs, e).
+//
+// Bound by the chain load - sum of vt - CFL terms - minimum, a few
+// microseconds on its own whatever the grid, so everything the ring mean of
+// vt does not enter shares the first reduction with it and the fields are
+// loaded before that reduction waits (up to six cells per thread; beyond, the
+// registers do not hold them).  The star's force needs no sum of its own: its
+// cells lie at one distance from it, so it is the barycentre sum times a
+// factor of the ring.
 template <typename T, int K> __global__ void __launch_bounds__(RING_LB(K)) k_cfl_ring(KArgs a) {
-  __shared__ double sh[1024];
+  constexpr int M = 7;
+  __shared__ double sh[16 * M];
+  __shared__ double shmin[16], shf[16 * 4];
   const dfargo_ctrl *c = a.ctrl;
   if (!c->go) return;
-  const int i = ring_of_block(a), ns = a.ns, nr = a.nr, t = threadIdx.x, TB = blockDim.x;
+  const int i = ring_of_block(a), ns = a.ns, nr = a.nr, t = threadIdx.x, TB = ns / K, nw = blockDim.x >> 6;
+  const bool on = t < TB; // the block is the ring's threads rounded up to whole wavefronts
+  const int t0 = on ? t : 0;
   const long base = (long)i * ns;
   // the CFL arithmetic is FP64 whatever the storage type: the sub-step
   // count ceil(DT / dt_min) then follows the FP64 run's, and FP32 storage
   // changes the solution, not the time discretisation
-  using R = double;
-  const T *vt = (const T *)a.vt + base, *vr = (const T *)a.vr + base;
-  R vt_own[K];
-  double s = 0.0;
+  const T *vt = (const T *)a.vt + base, *vr = (const T *)a.vr + base, *rho = (const T *)a.rho + base;
+  constexpr bool AHEAD = K <= 6;
+  constexpr int KA = AHEAD ? K : 1;
+  T vt_own[K], vt_next[KA], vr_in[KA], vr_out[KA], cs_prev[KA];
 #pragma unroll
   for (int k = 0; k < K; k++) {
-    vt_own[k] = (R)vt[t + k * TB];
-    s += (double)vt_own[k];
-  }
-  s = block_sum_fast(s, sh);
-  const double vmoy = s / (double)ns;
-  if (t == 0) a.vmoy[i] = vmoy;
-  double dtmin = 1e30;
-  if (i >= 1) {
-    const R viscosity = (R)a.nu_ring[i];
-    const R dxrad = (R)(a.Rsup[i] - a.Rinf[i]);
-    const R dxtheta = (R)(a.Rmed[i] * a.pm / (double)ns);
-    const R vm = (R)vmoy, dxmin = (dxrad < dxtheta) ? dxrad : dxtheta;
-    const R invdt5 = (viscosity != R(0)) ? viscosity * R(4) / (R)a.powmin2[i] : R(1e-10);
-    // the ring's cell sizes divide every cell's terms: one reciprocal each
-    // (within an ulp of the quotients, which only moves dt by as much)
-    const R idxmin = R(1) / dxmin, idxrad = R(1) / dxrad, idxtheta = R(1) / dxtheta;
-    R smax = R(0);
-#pragma unroll
-    for (int k = 0; k < K; k++) {
-      const int j = t + k * TB, jp = (j == ns - 1) ? 0 : j + 1;
-      const R cs = a.energy ? (R)((const T *)a.cs)[base + j] : (R)a.cs_iso[i];
-      const R vres = a.fast ? vt_own[k] - vm : vt_own[k];
-      const R vrl = (R)vr[j];
-      const R invdt1 = cs * idxmin;
-      const R invdt2 = fabs(vrl) * idxrad;
-      const R invdt3 = fabs(vres) * idxtheta;
-      R dvr = (R)vr[j + ns] - vrl;
-      R dvt = (R)vt[jp] - vt_own[k];
-      if (dvr >= R(0)) dvr = R(1e-10); else dvr = -dvr;
-      if (dvt >= R(0)) dvt = R(1e-10); else dvt = -dvt;
-      const R q4 = dvr * idxrad, q5 = dvt * idxtheta;
-      R invdt4 = (q5 > q4) ? q5 : q4;
-      invdt4 *= R(4.0 * DF_CVNR * DF_CVNR);
-      const R invdt6 = R(1e-10);
-      // dt = CFLSECURITY / sqrt(S) decreases with S, and rounding keeps
-      // that order: the smallest dt of the ring is that of its largest S
-      const R S = invdt1 * invdt1 + invdt2 * invdt2 + invdt3 * invdt3 + invdt4 * invdt4 + invdt5 * invdt5 +
-                  invdt6 * invdt6;
-      smax = (S > smax) ? S : smax;
+    const int j = t0 + k * TB;
+    vt_own[k] = vt[j];
+    if constexpr (AHEAD) {
+      vt_next[k] = vt[(j == ns - 1) ? 0 : j + 1];
+      vr_in[k] = vr[j];
+      vr_out[k] = vr[j + ns];
+      cs_prev[k] = a.energy ? ((const T *)a.cs)[base + j] : (T)0;
     }
-    dtmin = R(DF_CFLSECURITY) / sqrt(smax);
   }
   // per-ring partials, stored partial-major (ring_part[p * nr + i]):
   // negative-density and negative-energy counts, disc mass, barycentre.
   // With the energy equation the same pass is ComputeSoundSpeed
-  // (src/SourceEuler.c:2340, after the CFL above read the previous cs) and
+  // (src/SourceEuler.c:2340; the CFL below reads the previous cs) and
   // the ring mean of cs that mpi_make1Dprofile feeds to FViscosity
   // (src/Viscosity.c:30-35) for the kernels after this one.
   double *part = a.ring_part + i;
+  T cs_new[K];
   {
     CSum m = {0, 0}, xb = {0, 0}, yb = {0, 0};
-    double crd = 0.0, cre = 0.0, css = 0.0;
+    double s = 0.0, css = 0.0;
+    int crd = 0, cre = 0;
     const double g = a.gamma;
 #pragma unroll
     for (int k = 0; k < K; k++) {
-      const int j = t + k * TB;
-      double dens = ld<T>(a.rho, base + j);
-      if (dens < 0.0) crd += 1.0;
+      const int j = t0 + k * TB;
+      const double dens = (double)rho[j];
+      s += (double)vt_own[k];
+      crd += dens < 0.0;
+      cs_new[k] = (T)0;
       if (a.energy) {
         const double en = ld<T>(a.en, base + j);
-        if (en < 0.0) cre += 1.0;
-        const double cs = sqrt(g * (g - 1.0) * en / dens);
-        // the particles of this sub-step still read the previous cs
-        if (a.d_on) ((T *)a.cs_old)[base + j] = ((const T *)a.cs)[base + j];
-        st<T>(a.cs, base + j, cs);
-        css += (double)(T)cs;
+        cre += en < 0.0;
+        cs_new[k] = (T)sqrt(g * (g - 1.0) * en / dens);
+        css += (double)cs_new[k];
       }
-      // the particle buckets of this sub-step start empty
-      if (a.d_on) a.cell_count[base + j] = 0;
-      double cm = a.Surf[i] * dens;
+      const double cm = a.Surf[i] * dens;
       m.add(cm);
       xb.add(cm * (a.Rmed[i] * a.CosAz[j]));
       yb.add(cm * (a.Rmed[i] * a.SinAz[j]));
     }
-    double v[6] = {crd, cre, m.value(), xb.value(), yb.value(), css};
-    block_sum_min_n<6>(v, dtmin, sh);
-    if (t == 0) {
+    double v[M] = {s, (double)crd, (double)cre, m.value(), xb.value(), yb.value(), css};
 #pragma unroll
-      for (int k = 0; k < 5; k++) part[(long)k * nr] = v[k];
-      a.ring_dt[i] = dtmin;
-      if (a.energy) {
-        const double gcs = v[5] / (double)ns;
-        a.gcs[i] = gcs;
-        double nu = a.visc_const;
-        if (a.alpha_on) nu = a.alpha * gcs * gcs * a.r15[i];
-        a.nu_ring[i] = a.visc_on ? nu * a.visc_mult[i] : 0.0;
-      }
+    for (int q = 0; q < M; q++) {
+      if ((q == 2 || q == 6) && !a.energy) continue;
+      const double w = wave_sum(on ? v[q] : 0.0);
+      if ((t & 63) == 0) sh[(t >> 6) * M + q] = w;
     }
   }
-  // then fx, fx (Hill-cut), fy, fy (Hill-cut) per force target; the
-  // inner/outer split of GlobalForce is only ever summed, so it is not kept
+  __syncthreads();
+  double vsum = 0.0;
+  for (int w = 0; w < nw; w++) vsum += sh[w * M];
+  const double vmoy = vsum / (double)ns;
+  double dtmin = 1e30;
+  if (i >= 1) {
+    const double viscosity = a.nu_ring[i];
+    const double dxrad = a.Rsup[i] - a.Rinf[i];
+    const double dxtheta = a.Rmed[i] * a.pm / (double)ns;
+    const double dxmin = (dxrad < dxtheta) ? dxrad : dxtheta;
+    const double invdt5 = (viscosity != 0.0) ? viscosity * 4.0 / a.powmin2[i] : 1e-10;
+    // the ring's cell sizes divide every cell's terms: one reciprocal each
+    // (within an ulp of the quotients, which only moves dt by as much)
+    const double idxmin = 1.0 / dxmin, idxrad = 1.0 / dxrad, idxtheta = 1.0 / dxtheta;
+    double smax = 0.0;
+#pragma unroll
+    for (int k = 0; k < K; k++) {
+      const int j = t0 + k * TB;
+      double vtn, vrl, vro, cs;
+      if constexpr (AHEAD) {
+        vtn = (double)vt_next[k];
+        vrl = (double)vr_in[k];
+        vro = (double)vr_out[k];
+        cs = a.energy ? (double)cs_prev[k] : a.cs_iso[i];
+      } else {
+        vtn = (double)vt[(j == ns - 1) ? 0 : j + 1];
+        vrl = (double)vr[j];
+        vro = (double)vr[j + ns];
+        cs = a.energy ? ld<T>(a.cs, base + j) : a.cs_iso[i];
+      }
+      const double vtl = (double)vt_own[k];
+      const double vres = a.fast ? vtl - vmoy : vtl;
+      const double invdt1 = cs * idxmin;
+      const double invdt2 = fabs(vrl) * idxrad;
+      const double invdt3 = fabs(vres) * idxtheta;
+      double dvr = vro - vrl, dvt = vtn - vtl;
+      if (dvr >= 0.0) dvr = 1e-10; else dvr = -dvr;
+      if (dvt >= 0.0) dvt = 1e-10; else dvt = -dvt;
+      const double q4 = dvr * idxrad, q5 = dvt * idxtheta;
+      double invdt4 = (q5 > q4) ? q5 : q4;
+      invdt4 *= 4.0 * DF_CVNR * DF_CVNR;
+      const double invdt6 = 1e-10;
+      // dt = CFLSECURITY / sqrt(S) decreases with S, and rounding keeps
+      // that order: the smallest dt of the ring is that of its largest S
+      const double S = invdt1 * invdt1 + invdt2 * invdt2 + invdt3 * invdt3 + invdt4 * invdt4 + invdt5 * invdt5 +
+                       invdt6 * invdt6;
+      smax = (S > smax) ? S : smax;
+    }
+    // threads past the ring repeat its first cell, which changes no minimum
+    dtmin = DF_CFLSECURITY / sqrt(smax);
+  }
+  dtmin = wave_min(dtmin);
+  if ((t & 63) == 0) shmin[t >> 6] = dtmin;
+  if (on) {
+#pragma unroll
+    for (int k = 0; k < K; k++) {
+      const long l = base + t + k * TB;
+      if (a.energy) {
+        // the particles of this sub-step still read the previous cs
+        if (a.d_on) ((T *)a.cs_old)[l] = ((const T *)a.cs)[l];
+        ((T *)a.cs)[l] = cs_new[k];
+      }
+      // the particle buckets of this sub-step start empty
+      if (a.d_on) a.cell_count[l] = 0;
+    }
+  }
+  __syncthreads();
   const bool hill = a.exclude_hill;
-  for (int tg = 0; tg < c->ntarget; tg++) {
+  if (t < M && !((t == 2 || t == 6) && !a.energy)) {
+    double s = 0.0;
+    for (int w = 0; w < nw; w++) s += sh[w * M + t];
+    if (t == 0) {
+      a.vmoy[i] = vmoy;
+      double d = shmin[0];
+      for (int w = 1; w < nw; w++) d = dmin2(d, shmin[w]);
+      a.ring_dt[i] = d;
+    } else if (t < 6) {
+      part[(long)(t - 1) * nr] = s;
+      if (t >= 4) {
+        // target 0, the star: G cellmass dx / d^3 with d one value on the ring
+        // (no cell lies in its Hill radius, 1e-15)
+        const double rsm = c->tg_rsm[0], dist2 = a.Rmed[i] * a.Rmed[i] + rsm * rsm;
+        const double f = DF_G * s * (1.0 / dist2 / sqrt(dist2));
+        double *g = part + (long)(5 + 2 * (t - 4)) * nr;
+        g[0] = f;
+        if (hill) g[nr] = f;
+      }
+    } else {
+      const double gcs = s / (double)ns;
+      a.gcs[i] = gcs;
+      double nu = a.visc_const;
+      if (a.alpha_on) nu = a.alpha * gcs * gcs * a.r15[i];
+      a.nu_ring[i] = a.visc_on ? nu * a.visc_mult[i] : 0.0;
+    }
+  }
+  // then fx, fx (Hill-cut), fy, fy (Hill-cut) per planet that feels the disc;
+  // the inner/outer split of GlobalForce is only ever summed, so it is not kept
+  for (int tg = 1; tg < c->ntarget; tg++) {
     const double x = c->tg_x[tg], y = c->tg_y[tg], rsm = c->tg_rsm[tg];
     const double rh = c->tg_rh[tg];
     CSum fx[2] = {{0, 0}, {0, 0}}, fy[2] = {{0, 0}, {0, 0}};
+    if (on)
 #pragma unroll
-    for (int k = 0; k < K; k++) {
-      const int j = t + k * TB;
-      double xc = a.Rmed[i] * a.CosAz[j], yc = a.Rmed[i] * a.SinAz[j];
-      double cellmass = a.Surf[i] * ld<T>(a.rho, base + j);
-      double dx = xc - x, dy = yc - y;
-      double d2 = dx * dx + dy * dy;
-      double dist2 = d2 + rsm * rsm;
-      double distance = sqrt(dist2);
-      double InvDist3 = 1.0 / dist2 / distance;
-      fx[0].add(DF_G * cellmass * dx * InvDist3 * 1.0);
-      fy[0].add(DF_G * cellmass * dy * InvDist3 * 1.0);
-      if (hill) {
-        double planet_distance = sqrt(d2);
-        double cutoff = a.exclude_hill_factor * rh, hill_cut;
-        if (planet_distance / cutoff < 0.5) hill_cut = 0.0;
-        else if (planet_distance > cutoff) hill_cut = 1.0;
-        else hill_cut = pow(sin((planet_distance / cutoff - .5) * DF_PI), 2.);
-        fx[1].add(DF_G * cellmass * dx * InvDist3 * hill_cut);
-        fy[1].add(DF_G * cellmass * dy * InvDist3 * hill_cut);
+      for (int k = 0; k < K; k++) {
+        const int j = t + k * TB;
+        double xc = a.Rmed[i] * a.CosAz[j], yc = a.Rmed[i] * a.SinAz[j];
+        double cellmass = a.Surf[i] * (double)rho[j];
+        double dx = xc - x, dy = yc - y;
+        double d2 = dx * dx + dy * dy;
+        double dist2 = d2 + rsm * rsm;
+        double distance = sqrt(dist2);
+        double InvDist3 = 1.0 / dist2 / distance;
+        fx[0].add(DF_G * cellmass * dx * InvDist3 * 1.0);
+        fy[0].add(DF_G * cellmass * dy * InvDist3 * 1.0);
+        if (hill) {
+          double planet_distance = sqrt(d2);
+          double cutoff = a.exclude_hill_factor * rh, hill_cut;
+          if (planet_distance / cutoff < 0.5) hill_cut = 0.0;
+          else if (planet_distance > cutoff) hill_cut = 1.0;
+          else hill_cut = pow(sin((planet_distance / cutoff - .5) * DF_PI), 2.);
+          fx[1].add(DF_G * cellmass * dx * InvDist3 * hill_cut);
+          fy[1].add(DF_G * cellmass * dy * InvDist3 * hill_cut);
+        }
       }
-    }
     double *g = part + (long)(5 + 4 * tg) * nr;
     if (hill) {
       double v[4] = {fx[0].value(), fx[1].value(), fy[0].value(), fy[1].value()};
-      block_sum_n<4>(v, sh);
+      block_sum_n<4>(v, shf);
       if (t == 0)
 #pragma unroll
         for (int k = 0; k < 4; k++) g[(long)k * nr] = v[k];
     } else {
       double v[2] = {fx[0].value(), fy[0].value()};
-      block_sum_n<2>(v, sh);
+      block_sum_n<2>(v, shf);
       if (t == 0) { g[0] = v[0]; g[2 * (long)nr] = v[1]; }
     }
   }
@@ -810,7 +821,7 @@ template <typename T, bool ACC> __global__ void __launch_bounds__(CtrlBlock<ACC>
       nd = dmin2(nd, dt);
     }
   }
-  nd = block_min_fast(nd, sh);
+  nd = block_min(nd, sh);
   // minimum stopping time of the last particle interpolation (reset to 1e6
   // at each interpolation, src/Dsys.c:300): the minimum of the per-block
   // minima, compared as bit patterns of positive doubles
@@ -1033,7 +1044,8 @@ __device__ void control_serial(const KArgs &a, dfargo_ctrl *c, const double *sum
 // ComputeSoundSpeed at the start of AlgoGas (src/SourceEuler.c:2340); in
 // the sub-steps the CFL kernel recomputes cs with its ring means
 template <typename T, int K> __global__ void __launch_bounds__(RING_LB(K)) k_eos(KArgs a) {
-  const int i = ring_of_block(a), ns = a.ns, t = threadIdx.x, TB = blockDim.x;
+  const int i = ring_of_block(a), ns = a.ns, t = threadIdx.x, TB = ns / K;
+  if (t >= TB) return;
   const long base = (long)i * ns;
   const double g = a.gamma;
 #pragma unroll
@@ -1445,10 +1457,14 @@ __device__ double vischeat_cell(const KArgs &a, int i, int j, double *trr, doubl
 }
 
 template <typename T, int K> __global__ void __launch_bounds__(RING_LB(K)) k_energy(KArgs a) {
-  __shared__ double sh[1024];
+  __shared__ double sh[16];
   const dfargo_ctrl *c = a.ctrl;
   if (!c->active) return;
-  const int i = ring_of_block(a), ns = a.ns, nr = a.nr, t = threadIdx.x, TB = blockDim.x;
+  const int i = ring_of_block(a), ns = a.ns, nr = a.nr, TB = ns / K;
+  // threads past the ring (the block is whole wavefronts) repeat its first
+  // cells, outside the sum, and store nothing
+  const bool on = (int)threadIdx.x < TB;
+  const int t = on ? threadIdx.x : 0;
   const long base = (long)i * ns;
   const double dt = c->dt;
   // the stresses, divergence and heating are diagnostics read between
@@ -1474,7 +1490,7 @@ template <typename T, int K> __global__ void __launch_bounds__(RING_LB(K)) k_ene
       vh[k] = (a.nu_ring[nr - 1] != 0.0) ? q1 * exp(log(q1 / q2) * a.vh_lr1 / a.vh_lr2) : 0.0;
     }
     dv[k] = d;
-    if (last) {
+    if (last && on) {
       st<T>(a.trr, base + j, trr);
       st<T>(a.tpp, base + j, tpp);
       st<T>(a.trp, base + j, trp);
@@ -1494,7 +1510,7 @@ template <typename T, int K> __global__ void __launch_bounds__(RING_LB(K)) k_ene
     double s = 0.0;
 #pragma unroll
     for (int k = 0; k < K; k++) s += (ld<T>(a.vti, base + t + k * TB) + a.Rmed[i] * c->omega_frame);
-    s = block_sum_fast(s, sh);
+    s = block_sum(on ? s : 0.0, sh);
     double omega = s / (double)ns;
     omega /= a.Rmed[i];
     double coolingtime = a.beta[i] / omega;
@@ -1509,8 +1525,9 @@ template <typename T, int K> __global__ void __launch_bounds__(RING_LB(K)) k_ene
 #pragma unroll
     for (int k = 0; k < K; k++) enew[k] += ld<T>(a.fbedot, base + t + k * TB) * dt;
   }
+  if (on)
 #pragma unroll
-  for (int k = 0; k < K; k++) st_sr<T>(a.en, base + t + k * TB, enew[k], sr_key(c, base + t + k * TB, SR_EN));
+    for (int k = 0; k < K; k++) st_sr<T>(a.en, base + t + k * TB, enew[k], sr_key(c, base + t + k * TB, SR_EN));
 }
 
 // ------------------------------------------------------------------------
@@ -2279,7 +2296,8 @@ template <typename T> __global__ void __launch_bounds__(NR_TB) k_nonreflecting(K
 // sub-step's CFL condition read
 template <typename T, int K> __global__ void __launch_bounds__(RING_LB(K)) k_eos_step(KArgs a) {
   if (!a.ctrl->active) return;
-  const int i = ring_of_block(a), ns = a.ns, t = threadIdx.x, TB = blockDim.x;
+  const int i = ring_of_block(a), ns = a.ns, t = threadIdx.x, TB = ns / K;
+  if (t >= TB) return;
   const long base = (long)i * ns;
   const double g = a.gamma;
 #pragma unroll
@@ -2322,7 +2340,8 @@ static int wide_k(int ns) {
 #define RING_DISPATCH_K(KSEL, KERNEL, T, a, s, lds, ...)                                    \
   do {                                                                                      \
     int K_ = (KSEL);                                                                        \
-    dim3 g_((a).nr), b_((a).ns / K_);                                                       \
+    /* whole wavefronts: the reductions need them */                                        \
+    dim3 g_((a).nr), b_(((a).ns / K_ + 63) / 64 * 64);                                      \
     switch (K_) {                                                                           \
       case 1: hipLaunchKernelGGL((KERNEL<T, 1>), g_, b_, lds, s, a, ##__VA_ARGS__); break;  \
       case 2: hipLaunchKernelGGL((KERNEL<T, 2>), g_, b_, lds, s, a, ##__VA_ARGS__); break;  \
@@ -2460,14 +2479,15 @@ template void launch_visc_stress_state<float>(const KArgs &, hipStream_t);
 // reduction order.
 template <typename T, int K> __global__ void __launch_bounds__(RING_LB(K)) k_diag_ring(KArgs a, DiagBodies b,
                                                                                        double *part) {
-  __shared__ double sh[1024];
+  __shared__ double sh[16 * 4];
   const dfargo_ctrl *c = a.ctrl;
-  const int i = blockIdx.x, ns = a.ns, nr = a.nr, t = threadIdx.x, TB = blockDim.x;
+  const int i = blockIdx.x, ns = a.ns, nr = a.nr, t = threadIdx.x, TB = ns / K;
+  const bool on = t < TB; // the block is whole wavefronts
   const long base = (long)i * ns;
   const double Rm = a.Rmed[i], S = a.Surf[i], Of = c->omega_frame;
   const double wr = (a.Rsup[i] - a.Rinf[i]);
   CSum m = {0, 0}, mom = {0, 0}, en = {0, 0};
-  for (int k = 0; k < K; k++) {
+  for (int k = 0; on && k < K; k++) {
     const int j = t + k * TB;
     const long l = base + j;
     const double d = ld<T>(a.rho, l);
@@ -2487,7 +2507,7 @@ template <typename T, int K> __global__ void __launch_bounds__(RING_LB(K)) k_dia
   for (int bd = 0; bd < b.n; bd++) {
     const double x = b.x[bd], y = b.y[bd], rsm = b.rsm[bd], cutoff = a.exclude_hill_factor * b.rh[bd];
     CSum f[4] = {{0, 0}, {0, 0}, {0, 0}, {0, 0}};
-    for (int k = 0; k < K; k++) {
+    for (int k = 0; on && k < K; k++) {
       const int j = t + k * TB;
       const double xc = Rm * a.CosAz[j], yc = Rm * a.SinAz[j];
       const double cellmass = S * ld<T>(a.rho, base + j);
