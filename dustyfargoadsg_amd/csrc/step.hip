@@ -203,7 +203,8 @@ __device__ double d_aspect_ratio(const KArgs &a, double rad) {
   return ar;
 }
 __device__ double d_smoothing(const KArgs &a, double r) {
-  return a.thickness_smoothing * d_aspect_ratio(a, r) * pow(r, 1.0 + a.flaring);
+  // pow(r, 1) is r
+  return a.thickness_smoothing * d_aspect_ratio(a, r) * (a.flaring == 0.0 ? r : pow(r, 1.0 + a.flaring));
 }
 
 // gravitational potential at cell (i, j): FillForcesArrays
@@ -291,56 +292,71 @@ __device__ double psys_info(const KArgs &a, dfargo_ctrl *c, int get) {
   return asin(cross / (d1 * d2));
 }
 
+// The planets as the control wavefront holds them: planet k in lane k
+// (k < nb; the other lanes hold zeros), other planets' values by lane moves.
+struct Body {
+  double x, y, vx, vy, m;
+};
+__device__ __forceinline__ Body load_body(const dfargo_ctrl *c, int lane) {
+  Body b = {0.0, 0.0, 0.0, 0.0, 0.0};
+  if (lane < c->nb) b = {c->pl_x[lane], c->pl_y[lane], c->pl_vx[lane], c->pl_vy[lane], c->pl_m[lane]};
+  return b;
+}
+
 // start of a sub-step: mass taper, n-body limit and the force-sum targets
-// (src/SourceEuler.c:398-440, src/Pframeforce.c:131-161); one thread, run
-// once the loop condition holds
-__device__ void begin_substep(const KArgs &a, dfargo_ctrl *c) {
-  int nb = c->nb;
+// (src/SourceEuler.c:398-440, src/Pframeforce.c:131-161); one wavefront, run
+// once the loop condition holds.  c lies in LDS.
+__device__ void begin_substep(const KArgs &a, dfargo_ctrl *c, Body b, double time, int lane) {
+  const int nb = c->nb;
+  const bool planet = lane < nb;
+  double pmass = c->particles_mass0;
   if (a.mass_taper_param > 1e-2) {
-    double mt = (c->time - c->time0) / (a.mass_taper_param * 2.0 * DF_PI);
+    double mt = (time - c->time0) / (a.mass_taper_param * 2.0 * DF_PI);
     mt = (mt > 1.0 ? 1.0 : pow(sin(mt * DF_PI / 2.0), 2.0));
-    c->mass_taper = mt;
-    if (mt < 1.0)
-      for (int k = 0; k < nb; k++) c->pl_m[k] = c->pl_m0[k] + (c->pl_m1[k] - c->pl_m0[k]) * mt;
-    c->particles_mass = c->particles_mass0 * mt;
-  } else {
-    for (int k = 0; k < nb; k++)
-      if (c->pl_acc[k] < 1e-10) c->pl_m[k] = c->pl_m1[k];
-    c->particles_mass = c->particles_mass0;
+    if (planet && mt < 1.0) b.m = c->pl_m0[lane] + (c->pl_m1[lane] - c->pl_m0[lane]) * mt;
+    pmass = pmass * mt;
+    if (lane == 0) c->mass_taper = mt;
+  } else if (planet && c->pl_acc[lane] < 1e-10) {
+    b.m = c->pl_m1[lane];
   }
+  if (planet) c->pl_m[lane] = b.m;
   double dtnbody = 100.0;
   if (nb > 1) {
     dtnbody = 1e5;
-    for (int k = 0; k < nb; k++)
-      for (int j = k + 1; j < nb; j++) {
-        double dx = c->pl_x[k] - c->pl_x[j], dy = c->pl_y[k] - c->pl_y[j];
-        double dist = sqrt(dx * dx + dy * dy);
-        double buf = 2.0 * DF_PI * sqrt(dist * dist * dist / (c->pl_m[k] + c->pl_m[j] + 1e-8)) / 100.0;
-        dtnbody = dmin2(dtnbody, buf);
-      }
+    for (int j = 1; j < nb; j++) {
+      const double dx = b.x - __shfl(b.x, j, 64), dy = b.y - __shfl(b.y, j, 64), mj = __shfl(b.m, j, 64);
+      const double dist = sqrt(dx * dx + dy * dy);
+      const double buf = 2.0 * DF_PI * sqrt(dist * dist * dist / (b.m + mj + 1e-8)) / 100.0;
+      if (lane < j) dtnbody = dmin2(dtnbody, buf);
+    }
+    dtnbody = wave_min(dtnbody);
   }
-  c->dtnbody = dtnbody;
-  // target 0: the star (ComputeAccel at 0,0, src/SourceEuler.c:482)
-  c->tg_x[0] = 0.0;
-  c->tg_y[0] = 0.0;
-  c->tg_rsm[0] = a.indirect_smoothing;
-  c->tg_a[0] = sqrt(0.0 * 0.0 + 0.0 * 0.0);
-  c->tg_rh[0] = pow(0.0 / 3., 1. / 3.) * c->tg_a[0] + 1e-15;
-  c->tg_planet[0] = -1;
-  int nt = 1;
-  for (int k = 0; k < nb; k++) {
-    if (!c->pl_feel_disk[k]) continue;
-    double m = c->pl_m[k], x = c->pl_x[k], y = c->pl_y[k], r = sqrt(x * x + y * y);
-    double sm = a.roche ? r * pow(m / 3., 1. / 3.) * a.roche_smoothing : d_smoothing(a, r);
-    c->tg_x[nt] = x;
-    c->tg_y[nt] = y;
-    c->tg_rsm[nt] = sm;
-    c->tg_a[nt] = sqrt(x * x + y * y);
-    c->tg_rh[nt] = pow(m / 3., 1. / 3.) * c->tg_a[nt] + 1e-15;
-    c->tg_planet[nt] = k;
-    nt++;
+  // target 0: the star (ComputeAccel at 0,0, src/SourceEuler.c:482); then
+  // the planets that feel the disc, in order
+  const bool feels = planet && c->pl_feel_disk[lane];
+  const unsigned long long who = __ballot(feels);
+  if (lane == 0) {
+    c->particles_mass = pmass;
+    c->dtnbody = dtnbody;
+    c->tg_x[0] = 0.0;
+    c->tg_y[0] = 0.0;
+    c->tg_rsm[0] = a.indirect_smoothing;
+    c->tg_a[0] = 0.0;
+    c->tg_rh[0] = 1e-15;
+    c->tg_planet[0] = -1;
+    c->ntarget = 1 + __popcll(who);
   }
-  c->ntarget = nt;
+  if (feels) {
+    const int nt = 1 + __popcll(who & ((1ull << lane) - 1ull));
+    const double r = sqrt(b.x * b.x + b.y * b.y);
+    c->tg_x[nt] = b.x;
+    c->tg_y[nt] = b.y;
+    c->tg_rsm[nt] = a.roche ? r * pow(b.m / 3., 1. / 3.) * a.roche_smoothing : d_smoothing(a, r);
+    c->tg_a[nt] = r;
+    // the Hill radius enters only the cut of EXCLUDEHILL
+    c->tg_rh[nt] = a.exclude_hill ? pow(b.m / 3., 1. / 3.) * r + 1e-15 : 0.0;
+    c->tg_planet[nt] = lane;
+  }
 }
 
 // AlgoGas entry: loop variables, and the first sub-step's start.  The
@@ -354,19 +370,26 @@ __device__ void begin_substep(const KArgs &a, dfargo_ctrl *c) {
 // call).  The last kernel of a sub-step copies go_next into go, so no flag
 // changes under a kernel that reads it, even with the self-gravity kernels
 // running concurrently with the control kernel.
-__global__ void k_algogas_begin(KArgs a, double DT) {
-  if (threadIdx.x == 0 && blockIdx.x == 0) {
-    dfargo_ctrl *c = a.ctrl;
-    c->DT = DT;
-    c->dtemp = 0.0;
-    c->substeps = 0;
-    c->gas_timesteps_cfl = 1;
-    c->active = 0;
-    c->go = c->dtemp < 0.999999999 * c->DT;
-    c->go_next = c->go;
-    c->fargo_margin_bits = 0x3FE0000000000000ULL; // 0.5
-    if (c->go) begin_substep(a, c);
+__global__ void __launch_bounds__(64) k_algogas_begin(KArgs a, double DT) {
+  __shared__ dfargo_ctrl cs;
+  constexpr int NW = (int)(sizeof(dfargo_ctrl) / 8);
+  const int t = threadIdx.x;
+  for (int w = t; w < NW; w += 64) ((unsigned long long *)&cs)[w] = ((const unsigned long long *)a.ctrl)[w];
+  __syncthreads();
+  if (t == 0) {
+    cs.DT = DT;
+    cs.dtemp = 0.0;
+    cs.substeps = 0;
+    cs.gas_timesteps_cfl = 1;
+    cs.active = 0;
+    cs.go = 0.0 < 0.999999999 * DT;
+    cs.go_next = cs.go;
+    cs.fargo_margin_bits = 0x3FE0000000000000ULL; // 0.5
   }
+  __syncthreads();
+  if (cs.go) begin_substep(a, &cs, load_body(&cs, t), cs.time, t);
+  __syncthreads();
+  for (int w = t; w < NW; w += 64) ((unsigned long long *)a.ctrl)[w] = ((const unsigned long long *)&cs)[w];
 }
 
 // ConditionCFL per ring (src/SourceEuler.c:1340-1484) fused with the
@@ -587,61 +610,56 @@ template <typename T, int K> __global__ void __launch_bounds__(RING_LB(K)) k_cfl
   }
 }
 
-// Cash-Karp RK5 of the star+planet problem (src/RungeKunta.c:14-91)
-__device__ void d_deriv_rk5(const double *q, const double *masses, double *deriv, int n, double dt,
-                            const int *feelothers, int indirect) {
-  const double *x = q, *y = q + n, *vx = y + n, *vy = vx + n;
-  double *dx = deriv, *dy = deriv + n, *dvx = dy + n, *dvy = dvx + n;
-  for (int i = 0; i < n; i++) {
-    const double Di = sqrt(x[i] * x[i] + y[i] * y[i]);
-    dx[i] = vx[i];
-    dy[i] = vy[i];
-    dvx[i] = -DF_G * 1.0 / Di / Di / Di * x[i];
-    dvy[i] = -DF_G * 1.0 / Di / Di / Di * y[i];
-    for (int j = 0; j < n; j++) {
-      if (indirect) {
-        const double Dj = sqrt(x[j] * x[j] + y[j] * y[j]);
-        dvx[i] -= DF_G * masses[j] / Dj / Dj / Dj * x[j];
-        dvy[i] -= DF_G * masses[j] / Dj / Dj / Dj * y[j];
-      }
-      if ((j != i) && feelothers[i]) {
-        double dist = (x[i] - x[j]) * (x[i] - x[j]) + (y[i] - y[j]) * (y[i] - y[j]);
-        dist = sqrt(dist);
-        dvx[i] += DF_G * masses[j] / dist / dist / dist * (x[j] - x[i]);
-        dvy[i] += DF_G * masses[j] / dist / dist / dist * (y[j] - y[i]);
-      }
+// Cash-Karp RK5 of the star+planet problem (src/RungeKunta.c:14-91), a planet
+// per lane with its six stages in registers
+__device__ __forceinline__ Body d_deriv_rk5(const Body &q, double dt, int n, int lane, bool feels_others,
+                                            int indirect) {
+  const double Di = sqrt(q.x * q.x + q.y * q.y);
+  const double self = -DF_G * 1.0 / Di / Di / Di;
+  Body d = {q.vx, q.vy, self * q.x, self * q.y, 0.0};
+  for (int j = 0; j < n; j++) {
+    const double xj = __shfl(q.x, j, 64), yj = __shfl(q.y, j, 64), mj = __shfl(q.m, j, 64);
+    if (indirect) {
+      const double Dj = __shfl(Di, j, 64), w = DF_G * mj / Dj / Dj / Dj;
+      d.vx -= w * xj;
+      d.vy -= w * yj;
+    }
+    if (n > 1 && j != lane && feels_others) {
+      const double dist = sqrt((q.x - xj) * (q.x - xj) + (q.y - yj) * (q.y - yj));
+      const double w = DF_G * mj / dist / dist / dist;
+      d.vx += w * (xj - q.x);
+      d.vy += w * (yj - q.y);
     }
   }
-  for (int i = 0; i < 4 * n; i++) deriv[i] *= dt;
+  return {d.x * dt, d.y * dt, d.vx * dt, d.vy * dt, 0.0};
 }
-__device__ void d_translate(const double *q0, const double *k1, const double *k2, const double *k3,
-                            const double *k4, const double *k5, double c1, double c2, double c3,
-                            double c4, double c5, double *q1, int n) {
-  for (int i = 0; i < 4 * n; i++)
-    q1[i] = q0[i] + c1 * k1[i] + c2 * k2[i] + c3 * k3[i] + c4 * k4[i] + c5 * k5[i];
+template <int N> __device__ __forceinline__ Body d_translate(const Body &q, const Body (&k)[6], const double (&c)[N]) {
+  Body r = q;
+#pragma unroll
+  for (int s = 0; s < N; s++) {
+    if (c[s] == 0.0) continue;
+    r.x += c[s] * k[s].x;
+    r.y += c[s] * k[s].y;
+    r.vx += c[s] * k[s].vx;
+    r.vy += c[s] * k[s].vy;
+  }
+  return r;
 }
-// k holds the six stages, 6 x 4*DF_MAXPL doubles (LDS: the control kernel
-// keeps per-thread arrays out of scratch memory)
-__device__ void d_rk5(const double *q0, double dt, const double *m, double *q1, int n,
-                      const int *fo, int ind, double *k) {
-  double *k1 = k, *k2 = k1 + 4 * DF_MAXPL, *k3 = k2 + 4 * DF_MAXPL, *k4 = k3 + 4 * DF_MAXPL,
-         *k5 = k4 + 4 * DF_MAXPL, *k6 = k5 + 4 * DF_MAXPL;
-  for (int i = 0; i < 4 * DF_MAXPL; i++) k1[i] = k2[i] = k3[i] = k4[i] = k5[i] = k6[i] = 0.0;
-  d_deriv_rk5(q0, m, k1, n, dt, fo, ind);
-  d_translate(q0, k1, k2, k3, k4, k5, 0.2, 0.0, 0.0, 0.0, 0.0, q1, n);
-  d_deriv_rk5(q1, m, k2, n, dt, fo, ind);
-  d_translate(q0, k1, k2, k3, k4, k5, 0.075, 0.225, 0.0, 0.0, 0.0, q1, n);
-  d_deriv_rk5(q1, m, k3, n, dt, fo, ind);
-  d_translate(q0, k1, k2, k3, k4, k5, 0.3, -0.9, 1.2, 0.0, 0.0, q1, n);
-  d_deriv_rk5(q1, m, k4, n, dt, fo, ind);
-  d_translate(q0, k1, k2, k3, k4, k5, -11.0 / 54.0, 2.5, -70.0 / 27.0, 35.0 / 27.0, 0.0, q1, n);
-  d_deriv_rk5(q1, m, k5, n, dt, fo, ind);
-  d_translate(q0, k1, k2, k3, k4, k5, 1631.0 / 55296.0, 175.0 / 512.0, 575.0 / 13824.0,
-              44275.0 / 110592.0, 253.0 / 4096.0, q1, n);
-  d_deriv_rk5(q1, m, k6, n, dt, fo, ind);
-  for (int i = 0; i < 4 * n; i++)
-    q1[i] = q0[i] + 37.0 / 378.0 * k1[i] + 250.0 / 621.0 * k3[i] + 125.0 / 594.0 * k4[i] +
-            512.0 / 1771.0 * k6[i];
+__device__ Body d_rk5(const Body &q, double dt, int n, int lane, bool fo, int ind) {
+  Body k[6];
+  k[0] = d_deriv_rk5(q, dt, n, lane, fo, ind);
+  const double c1[1] = {0.2};
+  k[1] = d_deriv_rk5(d_translate<1>(q, k, c1), dt, n, lane, fo, ind);
+  const double c2[2] = {0.075, 0.225};
+  k[2] = d_deriv_rk5(d_translate<2>(q, k, c2), dt, n, lane, fo, ind);
+  const double c3[3] = {0.3, -0.9, 1.2};
+  k[3] = d_deriv_rk5(d_translate<3>(q, k, c3), dt, n, lane, fo, ind);
+  const double c4[4] = {-11.0 / 54.0, 2.5, -70.0 / 27.0, 35.0 / 27.0};
+  k[4] = d_deriv_rk5(d_translate<4>(q, k, c4), dt, n, lane, fo, ind);
+  const double c5[5] = {1631.0 / 55296.0, 175.0 / 512.0, 575.0 / 13824.0, 44275.0 / 110592.0, 253.0 / 4096.0};
+  k[5] = d_deriv_rk5(d_translate<5>(q, k, c5), dt, n, lane, fo, ind);
+  const double c6[6] = {37.0 / 378.0, 0.0, 250.0 / 621.0, 125.0 / 594.0, 0.0, 512.0 / 1771.0};
+  return d_translate<6>(q, k, c6);
 }
 
 // Scalar part of a sub-step, one block: the CFL reduction and sub-step dt
@@ -774,271 +792,318 @@ __device__ void accrete_planets(const KArgs &a, dfargo_ctrl *c, double dt, doubl
   }
 }
 
-template <typename T>
-__device__ void control_serial(const KArgs &a, dfargo_ctrl *c, const double *sums, double *sh, double s_dt);
+__device__ void control_wave(const KArgs &a, dfargo_ctrl *c, const double *sums, double dt, double dtemp, int lane);
 
 // Two builds: without accretion, 1024 threads; with it, 512, whose larger
-// register budget keeps the accretion path and the one-thread n-body code
-// free of spills.
+// register budget keeps the accretion path and the n-body code free of spills.
+//
+// One workgroup between two grids: bound by its own latency.  All of its
+// global reads (the control block, the rings' limits, the partials in batches
+// of eight per lane) are issued before the loop condition is looked at, they
+// meet in one barrier, and one wavefront does the rest with a planet per lane
+// and its n-body stages in registers.  One thread with the stages in LDS and a
+// load, an add and a wait per ring took 24 us at 200x400 with a free planet
+// and 23 us at 1024 rings.
 template <bool ACC> struct CtrlBlock { static constexpr int n = 1024; };
 template <> struct CtrlBlock<true> { static constexpr int n = 512; };
 template <typename T, bool ACC> __global__ void __launch_bounds__(CtrlBlock<ACC>::n) k_control(KArgs a) {
-  __shared__ double sh[1024];
+  constexpr int TB = CtrlBlock<ACC>::n, NWV = TB / 64;
   __shared__ double sums[DF_NPART(DF_MAXTG)];
-  // The control block is staged in LDS for the kernel's run: the one-thread
-  // part below reads and writes dozens of its fields in dependent order,
-  // which from global memory costs a memory latency each.  It is copied in
-  // and back by all threads; no kernel that may run beside this one writes
-  // the block (the self-gravity transforms only read its go flag, which
-  // this kernel leaves as it is).
+  __shared__ double smin[NWV];
+  __shared__ unsigned long long tsw[NWV];
+  // The control block is staged in LDS for the kernel's run: the part below
+  // reads and writes dozens of its fields in dependent order, which from
+  // global memory costs a memory latency each.  It is copied in and back by
+  // all threads; no kernel that may run beside this one writes the block
+  // (the self-gravity transforms only read its go flag, which this kernel
+  // leaves as it is).
   __shared__ dfargo_ctrl cs;
-  static_assert(sizeof(dfargo_ctrl) % 8 == 0, "the control block is copied as 8-byte words");
   constexpr int NW = (int)(sizeof(dfargo_ctrl) / 8);
+  static_assert(sizeof(dfargo_ctrl) % 8 == 0 && NW <= TB, "the control block is copied as 8-byte words, one a thread");
   dfargo_ctrl *const cg = a.ctrl;
-  const int t = threadIdx.x, TB = blockDim.x, nr = a.nr, ns = a.ns;
-  if (!cg->go) {
-    if (t == 0) cg->active = 0;
-    return;
-  }
-  for (int w = t; w < NW; w += TB) ((unsigned long long *)&cs)[w] = ((const unsigned long long *)cg)[w];
-  __syncthreads();
-  dfargo_ctrl *c = &cs;
+  const int t = threadIdx.x, lane = t & 63, wave = t >> 6, nr = a.nr, ns = a.ns;
+  const int go = cg->go, NP = DF_NPART(cg->ntarget);
+  const unsigned long long word = t < NW ? ((const unsigned long long *)cg)[t] : 0ull;
   double nd = 1e30;
-  for (int i = 1 + t; i < nr; i += TB) {
-    double v = a.ring_dt[i];
+  for (int i = t; i < nr; i += TB) {
+    double v = i > 0 ? a.ring_dt[i] : 1e30;
     // with the dust fluid each cell's limit is max2(min2(dtg, dtd), 1e-10)
     // (src/SourceEuler.c:1462-1465); both maps are monotone, so per ring
-    if (a.df_on) v = dmax2(dmin2(v, a.df_ring_dt[i]), 1.e-10);
+    if (a.df_on && i > 0) v = dmax2(dmin2(v, a.df_ring_dt[i]), 1.e-10);
     nd = dmin2(nd, v);
-  }
-  for (int i = t; i < nr - 1; i += TB) {
-    double dt = a.pm * DF_CFLSECURITY / (double)ns /
-                fabs(a.vmoy[i] * a.InvRmed[i] - a.vmoy[i + 1] * a.InvRmed[i + 1]);
-    nd = dmin2(nd, dt);
-    // the dust fluid's shear limit (src/SourceEuler.c:1486-1491)
-    if (a.df_on && !a.df_sfta) {
-      dt = a.pm * DF_CFLSECURITY / (double)ns / fabs(a.dvmoy[i] * a.InvRmed[i] - a.dvmoy[i + 1] * a.InvRmed[i + 1]);
-      nd = dmin2(nd, dt);
+    if (i < nr - 1) {
+      const double w0 = a.InvRmed[i], w1 = a.InvRmed[i + 1];
+      v = a.pm * DF_CFLSECURITY / (double)ns / fabs(a.vmoy[i] * w0 - a.vmoy[i + 1] * w1);
+      nd = dmin2(nd, v);
+      // the dust fluid's shear limit (src/SourceEuler.c:1486-1491)
+      if (a.df_on && !a.df_sfta) {
+        v = a.pm * DF_CFLSECURITY / (double)ns / fabs(a.dvmoy[i] * w0 - a.dvmoy[i + 1] * w1);
+        nd = dmin2(nd, v);
+      }
     }
   }
-  nd = block_min(nd, sh);
   // minimum stopping time of the last particle interpolation (reset to 1e6
   // at each interpolation, src/Dsys.c:300): the minimum of the per-block
   // minima, compared as bit patterns of positive doubles
-  double dust_min_ts = 1e6;
-  if (a.d_on && a.d_np > 0 && a.d_feedback) {
-    unsigned long long m = (unsigned long long)__double_as_longlong(1e6);
-    const int nb = (a.d_np + 255) / 256;
-    for (int b = t; b < nb; b += TB) m = (a.p_tsmin[b] < m) ? a.p_tsmin[b] : m;
-    for (int off = 32; off > 0; off >>= 1) {
-      const unsigned long long o = (unsigned long long)__shfl_xor((long)m, off, 64);
-      m = (o < m) ? o : m;
-    }
-    __shared__ unsigned long long tsw[16];
-    if ((t & 63) == 0) tsw[t >> 6] = m;
-    __syncthreads();
-    m = tsw[0];
-    for (int w = 1; w < TB / 64; w++) m = (tsw[w] < m) ? tsw[w] : m;
-    dust_min_ts = __longlong_as_double((long long)m);
+  const bool ts_limit = a.d_on && a.d_np > 0 && a.d_feedback;
+  unsigned long long ts = (unsigned long long)__double_as_longlong(1e6);
+  if (ts_limit) {
+    const int nblk = (a.d_np + 255) / 256;
+    for (int b = t; b < nblk; b += TB) ts = (a.p_tsmin[b] < ts) ? a.p_tsmin[b] : ts;
   }
   // each wavefront sums whole partials: lanes stride the rings with a
-  // compensated sum, then a fixed shuffle tree (deterministic)
-  const int NP = DF_NPART(c->ntarget), lane = t & 63, nw = TB >> 6;
-  for (int p = t >> 6; p < NP; p += nw) {
+  // compensated sum, then a fixed tree (deterministic)
+  double psum[(DF_NPART(DF_MAXTG) + NWV - 1) / NWV];
+#pragma unroll
+  for (int r = 0; r < (DF_NPART(DF_MAXTG) + NWV - 1) / NWV; r++) {
+    const int p = wave + r * NWV;
+    psum[r] = 0.0;
+    if (p >= NP) continue;
     const double *src = a.ring_part + (long)p * nr;
     CSum s = {0, 0};
-    for (int i = lane; i < nr; i += 64) s.add(src[i]);
-    double v = s.value();
-    for (int off = 32; off > 0; off >>= 1) v += __shfl_down(v, off, 64);
+    for (int i0 = 0; i0 < nr; i0 += 8 * 64) {
+      double x[8];
+#pragma unroll
+      for (int q = 0; q < 8; q++) x[q] = (i0 + q * 64 + lane < nr) ? src[i0 + q * 64 + lane] : 0.0;
+#pragma unroll
+      for (int q = 0; q < 8; q++) s.add(x[q]);
+    }
+    psum[r] = s.value();
+  }
+  if (!go) {
+    if (t == 0) cg->active = 0;
+    return;
+  }
+  if (t < NW) ((unsigned long long *)&cs)[t] = word;
+  nd = wave_min(nd);
+  if (lane == 0) smin[wave] = nd;
+  if (ts_limit) {
+    for (int off = 32; off > 0; off >>= 1) {
+      const unsigned long long o = (unsigned long long)__shfl_xor((long)ts, off, 64);
+      ts = (o < ts) ? o : ts;
+    }
+    if (lane == 0) tsw[wave] = ts;
+  }
+#pragma unroll
+  for (int r = 0; r < (DF_NPART(DF_MAXTG) + NWV - 1) / NWV; r++) {
+    const int p = wave + r * NWV;
+    if (p >= NP) continue;
+    const double v = wave_sum(psum[r]);
     if (lane == 0) sums[p] = v;
   }
   __syncthreads();
-  // sub-step dt
+  dfargo_ctrl *const c = &cs;
   __shared__ double s_dt;
-  if (t == 0) {
+  if (wave == 0) {
+    // sub-step dt
     double dt;
+    int gts = c->gas_timesteps_cfl;
     if (!a.d_fixed_dt) {
-      double deltaT = c->DT - c->dtemp;
+      nd = wave_min(lane < NWV ? smin[lane] : 1e30);
+      const double deltaT = c->DT - c->dtemp;
       // the minimum stopping time of the last interpolation, resolved by two
       // steps (src/SourceEuler.c:1501-1507)
-      if (a.d_on && a.d_np > 0 && a.d_feedback) {
-        double dt_fb = 0.5 * dust_min_ts;
+      if (ts_limit) {
+        unsigned long long m = tsw[0];
+        for (int w = 1; w < NWV; w++) m = (tsw[w] < m) ? tsw[w] : m;
+        double dt_fb = 0.5 * __longlong_as_double((long long)m);
         if (dt_fb == 0.0) dt_fb = 1e10;
         if (dt_fb < nd) nd = dt_fb;
       }
       if (deltaT < nd) nd = deltaT;
-      int gts = (int)(ceil(deltaT / nd));
-      double dthydro = deltaT / (double)gts;
+      gts = (int)(ceil(deltaT / nd));
+      const double dthydro = deltaT / (double)gts;
       dt = dmin2(dthydro, c->dtnbody);
-      c->gas_timesteps_cfl = gts;
     } else {
       // the particles' fixed time step (src/SourceEuler.c:457-463)
       dt = a.d_dust_timestep;
-      c->mindt = a.d_dust_timestep;
-      c->maxdt = a.d_dust_timestep;
     }
-    c->dtemp += dt;
-    if (dt < c->mindt) c->mindt = dt;
-    if (dt > c->maxdt) c->maxdt = dt;
-    c->dt = dt;
-    s_dt = dt;
+    const double dtemp = c->dtemp + dt;
+    if (lane == 0) {
+      c->gas_timesteps_cfl = gts;
+      if (a.d_fixed_dt) c->mindt = c->maxdt = dt;
+      c->dtemp = dtemp;
+      if (dt < c->mindt) c->mindt = dt;
+      if (dt > c->maxdt) c->maxdt = dt;
+      c->dt = dt;
+      s_dt = dt;
+    }
+    if constexpr (!ACC) control_wave(a, c, sums, dt, dtemp, lane);
   }
   if constexpr (ACC) {
     // AccreteOntoPlanets right after dt (src/SourceEuler.c:454)
+    __shared__ double red[(6 + 2 * DF_MAXTG) * 16];
     __syncthreads();
-    accrete_planets<T>(a, c, s_dt, sums, sh);
+    accrete_planets<T>(a, c, s_dt, sums, red);
+    __syncthreads();
+    if (wave == 0) control_wave(a, c, sums, s_dt, c->dtemp, lane);
   }
   __syncthreads();
-  if (t == 0) control_serial<T>(a, c, sums, sh, s_dt);
-  __syncthreads();
-  for (int w = t; w < NW; w += TB) ((unsigned long long *)cg)[w] = ((const unsigned long long *)&cs)[w];
+  if (t < NW) ((unsigned long long *)cg)[t] = ((const unsigned long long *)&cs)[t];
 }
 
-// The one-thread part of the control kernel on the LDS copy c of the
-// control block: crash flags, indirect terms, barycentre, FillForcesArrays'
-// parameters, AdvanceSystemFromDisk, AdvanceSystemRK5, the frame and the
-// loop condition.
-template <typename T>
-__device__ void control_serial(const KArgs &a, dfargo_ctrl *c, const double *sums, double *sh, double s_dt) {
-  const double dt = s_dt;
-  c->omega_prev = c->omega_frame;
-  c->crashed_d = sums[0] > 0.0;
-  c->crashed_e = sums[1] > 0.0;
+// The part of the control kernel one wavefront does on the LDS copy c of the
+// control block, a planet per lane: crash flags, indirect terms, barycentre,
+// FillForcesArrays' parameters, AdvanceSystemFromDisk, AdvanceSystemRK5, the
+// frame and the loop condition.  What is not a planet's is formed by every
+// lane and stored by lane 0.
+// The call's time dtemp after this sub-step comes as an argument: a lane must
+// not read back what lane 0 stores here.
+__device__ void control_wave(const KArgs &a, dfargo_ctrl *c, const double *sums, double dt, double dtemp, int lane) {
+  const int nb = c->nb;
+  const bool planet = lane < nb;
+  const double time = c->time;
   // gas indirect term: ComputeAccel(star), src/SideEuler.c:282-298
   const double *g0 = sums + 5;
-  c->dop_x = a.exclude_hill ? g0[1] : g0[0];
-  c->dop_y = a.exclude_hill ? g0[3] : g0[2];
+  const double dop_x = a.exclude_hill ? g0[1] : g0[0], dop_y = a.exclude_hill ? g0[3] : g0[2];
   // barycentre (src/SideEuler.c:42-112)
-  double total = sums[2];
-  c->barx[2] = sums[3] / (1.0 + total);
-  c->bary[2] = sums[4] / (1.0 + total);
-  c->dopalt_x = -(c->barx[2] - 2.0 * c->barx[1] + c->barx[0]) / (dt * dt);
-  c->dopalt_y = -(c->bary[2] - 2.0 * c->bary[1] + c->bary[0]) / (dt * dt);
-  c->barx[0] = c->barx[1]; c->barx[1] = c->barx[2];
-  c->bary[0] = c->bary[1]; c->bary[1] = c->bary[2];
+  const double total = sums[2];
+  const double bx = sums[3] / (1.0 + total), by = sums[4] / (1.0 + total);
+  const double dopalt_x = -(bx - 2.0 * c->barx[1] + c->barx[0]) / (dt * dt);
+  const double dopalt_y = -(by - 2.0 * c->bary[1] + c->bary[0]) / (dt * dt);
+  double ind_x = -dop_x, ind_y = -dop_y;
+  if (a.alt_indirect) {
+    ind_x = -dopalt_x;
+    ind_y = -dopalt_y;
+  }
+  if (!a.indirect_term) {
+    ind_x = 0.0;
+    ind_y = 0.0;
+  }
+  if (lane == 0) {
+    c->omega_prev = c->omega_frame;
+    c->crashed_d = sums[0] > 0.0;
+    // an isothermal disc has no energy to scan (its partials are not formed)
+    c->crashed_e = a.energy && sums[1] > 0.0;
+    c->dop_x = dop_x;
+    c->dop_y = dop_y;
+    c->dopalt_x = dopalt_x;
+    c->dopalt_y = dopalt_y;
+    c->barx[0] = c->barx[1]; c->barx[1] = bx; c->barx[2] = bx;
+    c->bary[0] = c->bary[1]; c->bary[1] = by; c->bary[2] = by;
+    c->ind_x = ind_x;
+    c->ind_y = ind_y;
+  }
   // FillForcesArrays parameters
   double planetmass_taper = 1.0;
   if (a.mass_taper_param > 1e-2) {
-    double mt = (c->time - c->time0) / (a.mass_taper_param * 2.0 * DF_PI);
+    const double mt = (time - c->time0) / (a.mass_taper_param * 2.0 * DF_PI);
     planetmass_taper = (mt > 1.0 ? 1.0 : .5 * (1.0 - cos(DF_PI * mt)));
   }
-  c->ind_x = -c->dop_x;
-  c->ind_y = -c->dop_y;
-  if (a.alt_indirect) {
-    c->ind_x = -c->dopalt_x;
-    c->ind_y = -c->dopalt_y;
-  }
-  if (!a.indirect_term) {
-    c->ind_x = 0.0;
-    c->ind_y = 0.0;
-  }
-  const int nb = c->nb;
-  for (int k = 0; k < nb; k++) {
-    double xp = c->pl_x[k], yp = c->pl_y[k], mp = c->pl_m[k] * planetmass_taper;
-    double PlanetDistance = sqrt(xp * xp + yp * yp);
-    double invd3 = 1.0 / PlanetDistance / PlanetDistance / PlanetDistance;
-    double RRoche = PlanetDistance * pow((1.0 / 3.0 * mp), 1.0 / 3.0);
-    double sm = a.roche ? RRoche * a.roche_smoothing : d_smoothing(a, PlanetDistance);
-    c->pot_x[k] = xp;
-    c->pot_y[k] = yp;
-    c->pot_m[k] = mp;
-    c->pot_invd3[k] = invd3;
-    c->pot_smooth[k] = sm * sm;
+  Body b = load_body(c, lane);
+  if (planet) {
+    const double mp = b.m * planetmass_taper, PlanetDistance = sqrt(b.x * b.x + b.y * b.y);
+    const double sm = a.roche ? PlanetDistance * pow((1.0 / 3.0 * mp), 1.0 / 3.0) * a.roche_smoothing
+                              : d_smoothing(a, PlanetDistance);
+    c->pot_x[lane] = b.x;
+    c->pot_y[lane] = b.y;
+    c->pot_m[lane] = mp;
+    c->pot_invd3[lane] = 1.0 / PlanetDistance / PlanetDistance / PlanetDistance;
+    c->pot_smooth[lane] = sm * sm;
   }
   // the corotating frame's mark (src/SourceEuler.c:476), before the
   // disc's kick changes the velocities
-  if (a.frame) psys_info(a, c, 0);
+  if (a.frame && lane == 0) psys_info(a, c, 0);
+  double omega_frame = c->omega_frame;
   // AdvanceSystemFromDisk (src/Pframeforce.c:131-161)
   for (int tg = 1; tg < c->ntarget; tg++) {
-    int k = c->tg_planet[tg];
+    if (c->tg_planet[tg] != lane) continue;
     const double *g = sums + 5 + 4 * tg;
-    double gx = a.exclude_hill ? g[1] : g[0];
-    double gy = a.exclude_hill ? g[3] : g[2];
-    c->pl_vx[k] += dt * gx;
-    c->pl_vy[k] += dt * gy;
-    c->pl_vx[k] += dt * c->ind_x;
-    c->pl_vy[k] += dt * c->ind_y;
+    const double gx = a.exclude_hill ? g[1] : g[0], gy = a.exclude_hill ? g[3] : g[2];
+    b.vx += dt * gx;
+    b.vy += dt * gy;
+    b.vx += dt * ind_x;
+    b.vy += dt * ind_y;
   }
   // AdvanceSystemRK5 (src/Pframeforce.c:163-266)
   if (nb > 0) {
-    double *q0 = sh, *q1 = q0 + 4 * DF_MAXPL, *m = q1 + 4 * DF_MAXPL, *kst = m + DF_MAXPL;
+    const bool moves = planet && lane >= 1 - (time >= a.release_date);
     if (!a.forced_circular) {
-      for (int i = 0; i < nb; i++) {
-        q0[i] = c->pl_x[i]; q0[i + nb] = c->pl_y[i];
-        q0[i + 2 * nb] = c->pl_vx[i]; q0[i + 3 * nb] = c->pl_vy[i];
-        m[i] = c->pl_m[i];
-      }
-      d_rk5(q0, dt, m, q1, nb, c->pl_feel_others, a.indirect_term, kst);
+      const Body q = d_rk5(b, dt, nb, lane, planet && c->pl_feel_others[lane], a.indirect_term);
+      if (moves) b = q;
+    } else if (moves) {
+      const double theta = atan2(b.y, b.x);
+      const double r = sqrt(b.x * b.x + b.y * b.y), v = sqrt(b.vx * b.vx + b.vy * b.vy);
+      const double omega = (-b.y * b.vx + b.x * b.vy) / r / r, dtheta = omega * dt;
+      double sn, cn;
+      sincos(theta + dtheta, &sn, &cn);
+      b.x = r * cn;
+      b.y = r * sn;
+      b.vx = -v * sn;
+      b.vy = v * cn;
     }
-    for (int i = 1 - (c->time >= a.release_date); i < nb; i++) {
-      if (!a.forced_circular) {
-        c->pl_x[i] = q1[i]; c->pl_y[i] = q1[i + nb];
-        c->pl_vx[i] = q1[i + 2 * nb]; c->pl_vy[i] = q1[i + 3 * nb];
-      } else {
-        double x = c->pl_x[i], y = c->pl_y[i], theta = atan2(y, x);
-        double vx = c->pl_vx[i], vy = c->pl_vy[i];
-        double r = sqrt(x * x + y * y), v = sqrt(vx * vx + vy * vy);
-        double omega = (-y * vx + x * vy) / r / r, dtheta = omega * dt;
-        c->pl_x[i] = r * cos(theta + dtheta);
-        c->pl_y[i] = r * sin(theta + dtheta);
-        c->pl_vx[i] = -v * sin(theta + dtheta);
-        c->pl_vy[i] = v * cos(theta + dtheta);
-      }
-    }
-    if (c->time < a.release_date) {
-      double x = c->pl_x[0], y = c->pl_y[0], r = sqrt(x * x + y * y), theta = atan2(y, x);
-      double rdot = (a.release_radius - r) / (a.release_date - c->time);
-      double omega = sqrt((1. + c->pl_m[0]) / r / r / r), new_r = r + rdot * dt, denom = r - new_r;
-      double dtheta = (denom != 0.0) ? 2. * dt * r * omega / denom * (sqrt(r / new_r) - 1.) : omega * dt;
-      double vx = rdot, vy = new_r * sqrt((1. + c->pl_m[0]) / new_r / new_r / new_r);
-      c->pl_x[0] = new_r * cos(dtheta + theta);
-      c->pl_y[0] = new_r * sin(dtheta + theta);
-      c->pl_vx[0] = vx * cos(dtheta + theta) - vy * sin(dtheta + theta);
-      c->pl_vy[0] = vx * sin(dtheta + theta) + vy * cos(dtheta + theta);
+    if (lane == 0 && time < a.release_date) {
+      const double x = b.x, y = b.y, r = sqrt(x * x + y * y), theta = atan2(y, x);
+      const double rdot = (a.release_radius - r) / (a.release_date - time);
+      const double omega = sqrt((1. + b.m) / r / r / r), new_r = r + rdot * dt, denom = r - new_r;
+      const double dtheta = (denom != 0.0) ? 2. * dt * r * omega / denom * (sqrt(r / new_r) - 1.) : omega * dt;
+      const double vx = rdot, vy = new_r * sqrt((1. + b.m) / new_r / new_r / new_r);
+      const double cn = cos(dtheta + theta), sn = sin(dtheta + theta);
+      b.x = new_r * cn;
+      b.y = new_r * sn;
+      b.vx = vx * cn - vy * sn;
+      b.vy = vx * sn + vy * cn;
     }
     // the frame follows its centre (src/SourceEuler.c:516-524); the
     // source kernel applies CorrectVtheta (vt -= domega Rmed) where it
     // reads vt
     if (a.frame) {
-      const double omega_new = psys_info(a, c, 1) / dt;
-      c->domega = omega_new - c->omega_frame;
-      c->omega_frame = omega_new;
-    }
-    // the particles of this sub-step feel the planets where the n-body
-    // step left them (src/SourceEuler.c:504-513 come before RotatePsys)
-    if (a.d_on)
-      for (int i = 0; i < nb; i++) {
-        c->dust_pl_x[i] = c->pl_x[i];
-        c->dust_pl_y[i] = c->pl_y[i];
+      if (planet) {
+        c->pl_x[lane] = b.x; c->pl_y[lane] = b.y;
+        c->pl_vx[lane] = b.vx; c->pl_vy[lane] = b.vy;
       }
-    // RotatePsys (src/Psys.c:352-370)
-    double angle = c->omega_frame * dt, sint = sin(angle), cost = cos(angle);
-    for (int i = 0; i < nb; i++) {
-      double xt = c->pl_x[i], yt = c->pl_y[i];
-      c->pl_x[i] = xt * cost + yt * sint;
-      c->pl_y[i] = -xt * sint + yt * cost;
-      xt = c->pl_vx[i];
-      yt = c->pl_vy[i];
-      c->pl_vx[i] = xt * cost + yt * sint;
-      c->pl_vy[i] = -xt * sint + yt * cost;
+      __threadfence_block();
+      double omega_new = 0.0;
+      if (lane == 0) {
+        omega_new = psys_info(a, c, 1) / dt;
+        c->domega = omega_new - omega_frame;
+        c->omega_frame = omega_new;
+      }
+      omega_frame = __shfl(omega_new, 0, 64);
+    }
+    if (planet) {
+      // the particles of this sub-step feel the planets where the n-body
+      // step left them (src/SourceEuler.c:504-513 come before RotatePsys)
+      if (a.d_on) {
+        c->dust_pl_x[lane] = b.x;
+        c->dust_pl_y[lane] = b.y;
+      }
+      // RotatePsys (src/Psys.c:352-370)
+      const double angle = omega_frame * dt;
+      if (angle != 0.0) {
+        double sint, cost;
+        sincos(angle, &sint, &cost);
+        double xt = b.x, yt = b.y;
+        b.x = xt * cost + yt * sint;
+        b.y = -xt * sint + yt * cost;
+        xt = b.vx;
+        yt = b.vy;
+        b.vx = xt * cost + yt * sint;
+        b.vy = -xt * sint + yt * cost;
+      }
+      c->pl_x[lane] = b.x; c->pl_y[lane] = b.y;
+      c->pl_vx[lane] = b.vx; c->pl_vy[lane] = b.vy;
+      // masses of this sub-step for the particle kernels
+      if (a.d_on) c->dust_pl_m[lane] = b.m;
     }
   }
   // PhysicalTime += dt closes the sub-step (src/SourceEuler.c:714); every
   // other use of PhysicalTime in the sub-step is above
-  c->time += dt;
-  c->substeps += 1;
-  c->substeps_total += 1;
-  c->active = 1;
-  if (a.d_on) {
-    // masses of this sub-step for the particle kernels, and a fresh
-    // minimum for their interpolation (src/Dsys.c:300)
-    c->dust_mp = c->particles_mass;
-    for (int k = 0; k < nb; k++) c->dust_pl_m[k] = c->pl_m[k];
-    c->out_count = 0;
+  const int go_next = dtemp < 0.999999999 * c->DT;
+  if (lane == 0) {
+    c->time = time + dt;
+    c->substeps += 1;
+    c->substeps_total += 1;
+    c->active = 1;
+    if (a.d_on) {
+      // ... and a fresh minimum for their interpolation (src/Dsys.c:300)
+      c->dust_mp = c->particles_mass;
+      c->out_count = 0;
+    }
+    // loop condition and start of the next sub-step
+    c->go_next = go_next;
   }
-  // loop condition and start of the next sub-step
-  c->go_next = c->dtemp < 0.999999999 * c->DT;
-  if (c->go_next) begin_substep(a, c);
+  if (go_next) begin_substep(a, c, b, time + dt, lane);
 }
 
 // ComputeSoundSpeed at the start of AlgoGas (src/SourceEuler.c:2340); in

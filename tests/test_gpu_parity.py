@@ -83,6 +83,23 @@ def test_gas_planet_fp64(nr, ns, calls):
     assert abs(go["planets"].y[0] - oo["planets"].y[0]) <= 1e-14
 
 
+# rings whose threads (one to four cells each) are no whole number of
+# wavefronts, with a planet that feels the disc: the ring reductions at their
+# remainders, the n-body step with a free planet.  The file's FP64 bars.
+@pytest.mark.parametrize("ns", [8, 63, 97, 400, 1030, 1530, 1533, 2044])
+@pytest.mark.parametrize("energy", [0, 1])
+def test_ragged_rings_fp64(ns, energy):
+    p, pl = gas_planet(nrad=12, nsec=ns, forced_circular=0, energy_equation=energy, beta_cooling=energy)
+    pl = dict(pl, feel_disk=[1])
+    o, so, d, sg = pair(p, pl)
+    n_o = o.algogas(DT)
+    d.algogas(DT)
+    assert d.status().last_call_substeps == n_o
+    errs, go, oo = compare(o, d, p, 1e-12, 1e-12, 1e-12)
+    for k in ("x", "y", "vx", "vy"):
+        assert abs(getattr(go["planets"], k)[0] - getattr(oo["planets"], k)[0]) <= 1e-13, k
+
+
 @pytest.mark.parametrize("nr,ns,calls", [(32, 96, 2), (64, 192, 1), (16, 1536, 1), (16, 3072, 1)])
 def test_energy_sg_fp64(nr, ns, calls):
     p, pl = energy_sg(nrad=nr, nsec=ns)
