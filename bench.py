@@ -38,8 +38,7 @@ def kernel_bytes_per_cell(name, w, energy, sg):
         # SubStep1 + viscosity + SubStep2: state (+ g_r, g_theta) in, new velocities (+ e) out
         "source": (ns + (2 if sg else 0)) * w + (2 + (1 if energy else 0)) * w,
         "energy": 4 * w + 1 * w,                         # rho, vr, vt, e in; e out
-        "transport_rad": ns * w + nq * w,                # state in, radially transported quantities out
-        "transport_azi": (nq + 1) * w + nq * w,          # quantities + vt in, shifted quantities out
+        "transport_azi": ns * w + nq * w,                # state in, transported quantities out
         "finish": nq * w + ns * w,                       # momenta in, state out
         "sg_rows_fwd": w + 2 * w,                        # Sigma -> complex row spectra
         # Z columns in, the two half kernel spectra ((Ns/2+1) x 2 Nrad complex

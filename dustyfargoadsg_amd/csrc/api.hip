@@ -61,9 +61,6 @@ struct dfargo_ctx {
   // capture only; default priority)
   hipStream_t stream2 = nullptr;
   hipEvent_t ev_fork = nullptr, ev_join = nullptr;
-  // the next sub-step's row transforms of self-gravity are formed by
-  // k_finish (a.sg_rows_in_finish), and once at the start of each call
-  bool sg_post = false;
   std::vector<hipEvent_t> evpool;
   std::vector<double> VthetaMed, VradMed, gcs_host;
   std::vector<float> fstage;
@@ -232,18 +229,13 @@ static bool is_sg_kernel(int id) {
          id == KID_SGZ_CONV || id == KID_SGZ_FILL;
 }
 
-// Start of an AlgoGas call on stream s: the device loop condition, the
-// sound speed of the state, and (when k_finish's partner forms them) the
-// row spectra of the state's density for the first sub-step.
+// Start of an AlgoGas call on stream s: the device loop condition and the
+// sound speed of the state.
 static void call_start(dfargo_ctx *c, double DT, hipStream_t s) {
   launch_algogas_begin(c->a, DT, s);
   if (c->p.energy_equation) {
     if (c->prec == DFARGO_FP64) launch_eos_pre<double>(c->a, s);
     else launch_eos_pre<float>(c->a, s);
-  }
-  if (c->sg_post) {
-    if (c->prec == DFARGO_FP64) launch_sg_rows_forced<double>(c->a, s);
-    else launch_sg_rows_forced<float>(c->a, s);
   }
 }
 
@@ -363,27 +355,10 @@ static int ensure_graph(dfargo_ctx *c, int level) {
 // The particles move after the planets (src/SourceEuler.c:504-531), i.e.
 // after the control kernel, and before the source terms that read their
 // feedback.
-//
-// With the full self-gravity and an edge that k_finish completes (wall or
-// open, no wave-killing zones or other boundary kernel after it), k_finish
-// can also form the row transforms for the next sub-step from the density
-// it stores (sg_post); the sub-step's self-gravity branch then starts with
-// the radial transforms.  Measured on MI355X (512x1536 energy+SG disc) the
-// ring-per-workgroup k_finish takes the row transforms' time back (21 us
-// against 9 us) and the CFL branch, which the radial transforms now meet
-// sooner, slows by as much, so the sub-step is no faster (0.172 against
-// 0.170 ms): it stays off (kSgRowsInFinish).
-static constexpr bool kSgRowsInFinish = false;
 static void build_sequence(dfargo_ctx *c) {
   c->seq.clear();
-  const bool wkz = c->p.wave_killing_zones && (c->a.wkz_n_in > 0 || c->a.wkz_i_out < c->p.nrad);
-  c->sg_post = kSgRowsInFinish && c->p.self_gravity && !c->p.sg_zero_mode &&
-               (c->p.boundary == DFARGO_BC_WALL || c->p.boundary == DFARGO_BC_OPEN) && !wkz &&
-               c->p.damp_to != DFARGO_DAMP_TO_VISCOUS;
   if (c->p.self_gravity && c->p.sg_zero_mode)
     for (int id : {KID_SGZ_MEAN, KID_SGZ_CONV, KID_SGZ_FILL}) c->seq.push_back(id);
-  else if (c->p.self_gravity && c->sg_post)
-    for (int id : {KID_SG_COLS, KID_SG_ROWS_INV}) c->seq.push_back(id);
   else if (c->p.self_gravity)
     for (int id : {KID_SG_ROWS_FWD, KID_SG_COLS, KID_SG_ROWS_INV}) c->seq.push_back(id);
   c->seq.push_back(KID_CFL);
@@ -404,10 +379,9 @@ static void build_sequence(dfargo_ctx *c) {
   if (df && c->a.df_visc)
     for (int id : {KID_DF_STRESS, KID_DF_VISC}) c->seq.push_back(id);
   if (df) c->seq.push_back(KID_DF_SUBSTEP2);
-  c->a.sg_rows_in_finish = c->sg_post ? 1 : 0;
-  for (int id : {KID_TRANSPORT_RAD, KID_TRANSPORT_AZI, KID_FINISH}) c->seq.push_back(id);
+  for (int id : {KID_TRANSPORT_AZI, KID_FINISH}) c->seq.push_back(id);
   if (df)
-    for (int id : {KID_DF_TRANSPORT_RAD, KID_DF_TRANSPORT_AZI, KID_DF_FINISH}) c->seq.push_back(id);
+    for (int id : {KID_DF_TRANSPORT_AZI, KID_DF_FINISH}) c->seq.push_back(id);
   if (c->p.boundary == DFARGO_BC_NONREFLECTING) {
     if (c->p.energy_equation) c->seq.push_back(KID_EOS_STEP);
     c->seq.push_back(KID_NONREFLECTING);
@@ -569,7 +543,7 @@ static int build_context(dfargo_ctx *c) {
   c->esz = (c->prec == DFARGO_FP64) ? sizeof(double) : sizeof(float);
   c->nfield = (size_t)(nr + 2) * ns;
   void **fields[] = {&a.rho, &a.vr, &a.vt, &a.en, &a.cs, &a.vri, &a.vti, &a.trr, &a.trp, &a.tpp,
-                     &a.divv, &a.vh, &a.t_rho, &a.t_rp, &a.t_rm, &a.t_tp, &a.t_tm, &a.t_en, &a.pot, &a.e_int,
+                     &a.divv, &a.vh, &a.pot, &a.e_int,
                      &a.z_rho, &a.z_rp, &a.z_rm, &a.z_tp, &a.z_tm, &a.z_en};
   for (void **f : fields)
     if ((rc = dalloc(c, f, c->esz * c->nfield))) return rc;
@@ -1641,7 +1615,7 @@ extern "C" int dfargo_attach_dust_fluid(dfargo_ctx *c, const dfargo_dust_fluid_p
   HIPCHK(hipSetDevice(c->dev));
   KArgs &a = c->a;
   double **grids[] = {&a.drho, &a.dvr, &a.dvt, &a.dstokes, &a.dvri, &a.dvti, &a.dtrr, &a.dtrp, &a.dtpp,
-                      &a.dt_rho, &a.dt_rp, &a.dt_rm, &a.dt_tp, &a.dt_tm, &a.dz_rho, &a.dz_rp, &a.dz_rm,
+                      &a.dz_rho, &a.dz_rp, &a.dz_rm,
                       &a.dz_tp, &a.dz_tm};
   for (double **g : grids)
     if ((rc = dalloc(c, (void **)g, sizeof(double) * c->nfield))) return rc;

@@ -16,7 +16,7 @@
 //   k_df_substep2  artificial viscosity (DVradNew), or in the
 //                  short-friction-time approximation DVradInt as it is;
 //                  the per-tile sums of the new vtheta for the FARGO mean
-//   k_transport_rad / k_transport_azi on the dust fields (Transportd)
+//   k_transport_azi on the dust fields (Transportd)
 //   k_df_finish    ComputeVelocities, Diffd, the floor, the wall,
 //                  sub-Keplerian and open-dust boundaries
 // and the wave-killing zones damp the fluid in k_evanescent.
@@ -320,11 +320,6 @@ __host__ __device__ inline KArgs df_transport_args(const KArgs &a) {
   d.rho = a.drho;
   d.vri = a.dvr;
   d.vti = a.dvt;
-  d.t_rho = a.dt_rho;
-  d.t_rp = a.dt_rp;
-  d.t_rm = a.dt_rm;
-  d.t_tp = a.dt_tp;
-  d.t_tm = a.dt_tm;
   d.z_rho = a.dz_rho;
   d.z_rp = a.dz_rp;
   d.z_rm = a.dz_rm;
@@ -442,6 +437,7 @@ __global__ void __launch_bounds__(256) k_df_finish(KArgs a) {
   if (!c->active) return;
   const int i = blockIdx.y, ns = a.ns, nr = a.nr;
   const int j = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i == nr && blockIdx.x == 0 && threadIdx.x < 64) add_lost_mass(a, a.dlost_col, &a.ctrl->lost_massd);
   if (j >= ns) return;
   const long l = (long)i * ns + j;
   if (i == nr) {
@@ -469,7 +465,7 @@ __global__ void __launch_bounds__(256) k_df_finish(KArgs a) {
 }
 
 static void launch_df_kernel(int id, const KArgs &a, hipStream_t s) {
-  const int bx = a.ns < 256 ? a.ns : 256;
+  const int bx = a.ns < 256 ? (a.ns + 63) / 64 * 64 : 256; // whole wavefronts
   const dim3 g((a.ns + bx - 1) / bx, a.nr), b(bx);
   switch (id) {
     case KID_DF_CFL: hipLaunchKernelGGL(k_df_cfl, dim3(a.nr), dim3(256), 0, s, a); break;
@@ -485,19 +481,7 @@ static void launch_df_kernel(int id, const KArgs &a, hipStream_t s) {
       hipLaunchKernelGGL(k_df_substep2, dim3(ntile, a.nr + 1), dim3(DF_SRC_COLS), 0, s, a);
       break;
     }
-    case KID_DF_TRANSPORT_RAD: {
-      const KArgs d = df_transport_args(a);
-      hipLaunchKernelGGL(k_transport_rad<double>, dim3((a.ns + RT_C - 1) / RT_C, (a.nr + RT_R - 1) / RT_R),
-                         dim3(RT_C, RT_R), 0, s, d);
-      break;
-    }
-    case KID_DF_TRANSPORT_AZI: {
-      const KArgs d = df_transport_args(a);
-      const int per = (a.tune_azi_waves == 1 || a.tune_azi_waves == 2) ? a.tune_azi_waves : 4;
-      const int nseg = (a.ns + AZ_OWN - 1) / AZ_OWN;
-      hipLaunchKernelGGL(k_transport_azi<double>, dim3((nseg + per - 1) / per, a.nr), dim3(per * AZ_LANES), 0, s, d);
-      break;
-    }
+    case KID_DF_TRANSPORT_AZI: launch_transport<double>(df_transport_args(a), s); break;
     case KID_DF_FINISH: hipLaunchKernelGGL(k_df_finish, dim3(g.x, a.nr + 1), b, 0, s, a); break;
     default: break;
   }

@@ -56,10 +56,6 @@ struct KArgs {
   // rings per workgroup of the self-gravity row transforms: 0 the default
   // (two where the rows run in place), 1 or 2
   int sg_rows_pair;
-  // with the full self-gravity: k_finish also forms the next sub-step's row
-  // spectra (one workgroup per ring), and the self-gravity branch of a
-  // sub-step starts with the radial transforms
-  int sg_rows_in_finish;
   int num_cu; // compute units of the device
   // constants
   double pm, dphi, invdphi, gamma, alpha, visc_const, floor_dens;
@@ -75,9 +71,9 @@ struct KArgs {
   const double *InvDxTheta; // 1 / (dphi Rmed[i]) per ring
   // fields (T)
   void *rho, *vr, *vt, *en, *cs, *vri, *vti, *trr, *trp, *tpp, *divv, *vh;
-  void *t_rho, *t_rp, *t_rm, *t_tp, *t_tm, *t_en, *sgr, *sgt, *pot, *e_int;
-  // the transported quantities after the azimuthal pass (the segments of a
-  // ring read t_* around their cells while others store: separate arrays)
+  void *sgr, *sgt, *pot, *e_int;
+  // the transported quantities (the transport reads the state around its
+  // cells while others store: separate arrays)
   void *z_rho, *z_rp, *z_rm, *z_tp, *z_tm, *z_en;
   // ring buffers (FP64 unless noted)
   double *vmoy, *ring_dt, *ring_part, *nu_ring, *gcs, *vmed, *lost_col;
@@ -122,12 +118,12 @@ struct KArgs {
   // the dust fluid (DUSTFLUID YES, FP64 storage): switches, grain
   // constants (internal density and radius in code units, the code-to-cgs
   // surface density factor), state, the sub-step's Stokes numbers,
-  // DVradInt / DVthetaInt, stresses, the transport's buffers (dt_*, dz_*
-  // as t_*, z_* for the gas), ring buffers and ring tables
+  // DVradInt / DVthetaInt, stresses, the transport's results (dz_* as z_*
+  // for the gas), ring buffers and ring tables
   int df_on, df_sfta, df_feel_disk, df_feedback, df_feel_sg, df_diffusion, df_visc, df_open;
   double df_rho_int, df_radius, df_to_cgs, df_diff_inn;
   double *drho, *dvr, *dvt, *dstokes, *dvri, *dvti, *dtrr, *dtrp, *dtpp;
-  double *dt_rho, *dt_rp, *dt_rm, *dt_tp, *dt_tm, *dz_rho, *dz_rp, *dz_rm, *dz_tp, *dz_tm;
+  double *dz_rho, *dz_rp, *dz_rm, *dz_tp, *dz_tm;
   double *dvmoy, *dvmed, *dvt_part, *dlost_col, *df_axisg, *df_ring_dt;
   long *dnshift;
   const double *df_cs, *df_nu, *df_sup15, *df_cavsup, *DSigmaMed, *DVthetaMed, *DVradMed;
@@ -146,11 +142,11 @@ struct KArgs {
 // launchers (step.hip, sg.hip); each enqueues on stream s
 enum KernelId {
   KID_SG_ROWS_FWD = 0, KID_SG_COLS, KID_SG_ROWS_INV,
-  KID_CFL, KID_CONTROL, KID_SOURCE, KID_ENERGY, KID_TRANSPORT_RAD, KID_TRANSPORT_AZI,
+  KID_CFL, KID_CONTROL, KID_SOURCE, KID_ENERGY, KID_TRANSPORT_AZI,
   KID_FINISH, KID_DUST_MOVE, KID_DUST_SCAN, KID_DUST_SCATTER, KID_DUST_SORT, KID_DUST_DEPOSIT, KID_DUST_REORDER,
   KID_EVANESCENT, KID_NONREFLECTING,
   KID_SGZ_MEAN, KID_SGZ_CONV, KID_SGZ_FILL, KID_EOS_STEP, KID_VISC1D,
-  KID_DF_CFL, KID_DF_AXISG, KID_DF_SOURCE, KID_DF_STRESS, KID_DF_VISC, KID_DF_SUBSTEP2, KID_DF_TRANSPORT_RAD,
+  KID_DF_CFL, KID_DF_AXISG, KID_DF_SOURCE, KID_DF_STRESS, KID_DF_VISC, KID_DF_SUBSTEP2,
   KID_DF_TRANSPORT_AZI, KID_DF_FINISH, KID_COUNT
 };
 extern const char *kKernelNames[KID_COUNT];
@@ -169,7 +165,6 @@ template <typename T> void launch_kernel(int id, const KArgs &a, hipStream_t s);
 template <typename T> void prepare_kernels(const KArgs &a);
 template <typename T> void sg_prepare(const KArgs &a);
 template <typename T> void launch_sg_kernel(int id, const KArgs &a, hipStream_t s);
-template <typename T> void launch_sg_rows_forced(const KArgs &a, hipStream_t s);
 // dust.hip: the particle kernels of a sub-step (after the control kernel),
 // and the start-up interpolation outside sub-steps
 template <typename T> void launch_dust_kernel(int id, const KArgs &a, hipStream_t s);

@@ -463,11 +463,6 @@ template <typename T> void launch_sg_accel(const KArgs &a, hipStream_t s) {
   for (int id : {KID_SG_ROWS_FWD, KID_SG_COLS, KID_SG_ROWS_INV})
     sg_pipeline<T>(id, a, s, 1);
 }
-// the row transforms of the stored density, whatever the loop condition
-// (at the start of an AlgoGas call when k_finish forms them afterwards)
-template <typename T> void launch_sg_rows_forced(const KArgs &a, hipStream_t s) {
-  sg_pipeline<T>(KID_SG_ROWS_FWD, a, s, 1);
-}
 template <typename T>
 void launch_fft_rows(void *data, int nrows, int L, const void *tw, int dir, hipStream_t s) {
   allow_lds(k_fft_rows<T>, 2 * sizeof(cx<T>) * fpsz(L));
@@ -488,8 +483,6 @@ template void sg_prepare<double>(const KArgs &);
 template void sg_prepare<float>(const KArgs &);
 template void launch_sg_kernel<double>(int, const KArgs &, hipStream_t);
 template void launch_sg_kernel<float>(int, const KArgs &, hipStream_t);
-template void launch_sg_rows_forced<double>(const KArgs &, hipStream_t);
-template void launch_sg_rows_forced<float>(const KArgs &, hipStream_t);
 template void launch_sg_accel<double>(const KArgs &, hipStream_t);
 template void launch_sg_accel<float>(const KArgs &, hipStream_t);
 template void launch_fft_rows<double>(void *, int, int, const void *, int, hipStream_t);

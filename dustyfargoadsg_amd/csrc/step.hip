@@ -15,12 +15,12 @@
 
 const char *kKernelNames[KID_COUNT] = {
     "sg_rows_fwd", "sg_cols", "sg_rows_inv",
-    "cfl_ring",    "control",        "source",  "energy",         "transport_rad",
+    "cfl_ring",    "control",        "source",  "energy",
     "transport_azi", "finish",      "dust_move",      "dust_scan",  "dust_scatter",
     "dust_sort",     "dust_deposit", "dust_reorder", "evanescent", "nonreflecting",
     "sgz_mean",      "sgz_conv",     "sgz_fill",     "eos_step",      "visc1d",
     "df_cfl",        "df_axisg",      "df_source",    "df_stress",    "df_visc",       "df_substep2",
-    "df_transport_rad", "df_transport_azi", "df_finish"};
+    "df_transport_azi", "df_finish"};
 
 // ------------------------------------------------------------------------
 // helpers
@@ -55,6 +55,12 @@ __device__ __forceinline__ unsigned mix32(unsigned x) {
 __device__ __forceinline__ unsigned sr_key(const dfargo_ctrl *c, long l, unsigned salt) {
   return mix32((unsigned)l * 0x9E3779B9U ^ mix32((unsigned)c->substeps_total * 0x85EBCA6BU + salt));
 }
+// One hash of the cell serves the quantities a kernel stores there: each takes
+// it through a multiplication of its own (a 32-bit multiplication costs four
+// issue slots, the whole hash three of them).
+__device__ __forceinline__ unsigned sr_draw(unsigned cell_key, unsigned q) {
+  return (cell_key ^ (0x9E3779B9U * (2U * q + 1U))) * 0x2C1B3C6DU;
+}
 template <typename T> __device__ __forceinline__ T sr_round(double v, unsigned key);
 template <> __device__ __forceinline__ double sr_round<double>(double v, unsigned) { return v; }
 // The 29 mantissa bits of the double below the float's last bit are the
@@ -72,11 +78,14 @@ template <typename T> __device__ __forceinline__ void st_sr(void *p, long i, dou
   ((T *)p)[i] = sr_round<T>(v, key);
 }
 // salts of the stochastically rounded stores
-enum { SR_VR = 1, SR_VT, SR_E, SR_EN, SR_RAD = 8, SR_AZI = 16, SR_EVA = 24, SR_ACC = 32, SR_FIN = 40 };
+enum { SR_VR = 1, SR_VT, SR_E, SR_EN, SR_AZI = 16, SR_EVA = 24, SR_ACC = 32, SR_FIN = 40 };
 
-// a / b from the hardware reciprocal, two Newton steps and one correction
-// of the quotient: within an ulp or two of the IEEE quotient for operands
-// well inside the exponent range (no scaling steps)
+// a / b from the hardware reciprocal, two Newton steps and one correction of
+// the quotient: the compiler's IEEE sequence without its scaling of operands
+// near the ends of the exponent range (three of eleven instructions and the
+// waits on their carry).  For the transport's operands, slopes and densities
+// far from 1e-154 and 1e154, that is the IEEE quotient; with a zero or
+// infinite divisor it is a NaN.
 __device__ __forceinline__ double div_nr(double a, double b) {
   double r = __builtin_amdgcn_rcp(b);
   double e = fma(-b, r, 1.0);
@@ -86,19 +95,6 @@ __device__ __forceinline__ double div_nr(double a, double b) {
   const double q = a * r;
   return fma(r, fma(-b, q, a), q);
 }
-
-// arithmetic type of the transport stencils for a storage type, and its
-// division: with FP64 storage the reference's IEEE double quotient; with
-// FP32 storage FP64 arithmetic whose quotients need not be correctly
-// rounded (their ulp is 2^-29 of the stored values' rounding)
-template <typename T> struct TransportArith {
-  using type = T;
-  static __device__ __forceinline__ double div(double a, double b) { return a / b; }
-};
-template <> struct TransportArith<float> {
-  using type = double;
-  static __device__ __forceinline__ double div(double a, double b) { return div_nr(a, b); }
-};
 
 __device__ __forceinline__ double dmin2(double a, double b) { return (b < a) ? b : a; }
 __device__ __forceinline__ double dmax2(double a, double b) { return (b > a) ? b : a; }
@@ -1599,144 +1595,31 @@ template <typename T, int K> __global__ void __launch_bounds__(RING_LB(K)) k_ene
 // transport
 // ------------------------------------------------------------------------
 
-// Radial transport (ComputeLRMomenta + OneWindRad, src/TransportEuler.c:
-// 89-220) on tiles of RT_R rings x RT_C columns.  The Work values
-// Q/(rho+1e-20) of the tile's rings and of two halo rings either side, then
-// the ComputeStarRad slopes, go through LDS, so each is formed once per cell
-// (plus the halo); every thread then updates one cell.  Quantity slots:
-// 0 rp, 1 rm, 2 tp, 3 tm, 4 e, 5 rho (the Work of the density itself),
-// 6 rho as its own base for RhoStar.  The arithmetic is that of the storage
-// type R (the reference's double with FP64 storage).
-#define RT_C 32
-#define RT_R 8
-
-// slope of ComputeStarRad at ring r (zero on the first and last ring)
-template <typename T, typename R = typename TransportArith<T>::type>
-__device__ __forceinline__ R rad_slope(const KArgs &a, int r, R qm, R q0, R qp) {
-  if (r <= 0 || r >= a.nr - 1) return R(0);
-  R dqm = (q0 - qm) * (R)a.InvDiffRmed[r];
-  R dqp = (qp - q0) * (R)a.InvDiffRmed[r + 1];
-  // branch-free: the quotient is formed on every lane and selected (where
-  // it is not used it may be an infinity or a NaN of a zero denominator,
-  // which the select discards; nothing traps)
-  const bool use = dqp * dqm > R(0);
-  const R d = TransportArith<T>::div(R(2) * dqp * dqm, dqp + dqm);
-  return use ? d : R(0);
-}
-// The upwind side of face r (between rings r-1 and r) for velocity v and
-// the weight of its slope in QRStar: (Rmed[r]-Rmed[r-1]-v dt)/2 from ring
-// r-1 when v > 0, else -(Rmed[r+1]-Rmed[r]+v dt)/2 from ring r (the same
-// products and sums as the reference's two branches); shared by every
-// quantity at the face.  Faces 0 and nr have no star (open = false).
-template <typename R> struct RadFace {
-  bool open, up;
-  R w;
-};
-template <typename R> __device__ __forceinline__ RadFace<R> rad_face(const KArgs &a, int r, R v, R dt) {
-  RadFace<R> f;
-  f.open = (r > 0 && r < a.nr);
-  f.up = v > R(0);
-  const int rc = f.open ? r : 1; // keeps the table reads in range on closed faces
-  const R wu = ((R)a.Rmed[rc] - (R)a.Rmed[rc - 1] - v * dt) * R(0.5);
-  const R wd = ((R)a.Rmed[rc + 1] - (R)a.Rmed[rc] + v * dt) * R(0.5);
-  f.w = f.up ? wu : -wd;
-  return f;
-}
-// QRStar at face r from the Work values of rings r-1, r and the slopes there
-template <typename R>
-__device__ __forceinline__ R rad_star(const RadFace<R> &f, R wm, R w0, R dqm, R dq0) {
-  const R s = (f.up ? wm : w0) + f.w * (f.up ? dqm : dq0);
-  return f.open ? s : R(0);
-}
-// the six transported quantities of cell (r, j) before the pass
-template <typename T, typename R>
-__device__ __forceinline__ void rad_quantities(const KArgs &a, int r, int j, R Of, R (&Q)[6]) {
-  const int ns = a.ns;
-  const int jp = (j == ns - 1) ? 0 : j + 1;
-  const T *rho = (const T *)a.rho + (long)r * ns, *vr = (const T *)a.vri + (long)r * ns;
-  const T *vt = (const T *)a.vti + (long)r * ns;
-  const R d = (R)rho[j], Rm = (R)a.Rmed[r];
-  Q[0] = d * (R)vr[j + ns];
-  Q[1] = d * (R)vr[j];
-  Q[2] = d * ((R)vt[jp] + Rm * Of) * Rm;
-  Q[3] = d * ((R)vt[j] + Rm * Of) * Rm;
-  Q[4] = a.energy ? (R)((const T *)a.en)[(long)r * ns + j] : R(0);
-  Q[5] = d;
-}
-
-template <typename T> __global__ void __launch_bounds__(RT_C * RT_R) k_transport_rad(KArgs a) {
-  using R = typename TransportArith<T>::type;
-  __shared__ R sW[7][RT_R + 4][RT_C];
-  __shared__ R sD[7][RT_R + 2][RT_C];
-  const dfargo_ctrl *c = a.ctrl;
-  if (!c->active) return;
-  const int ns = a.ns, nr = a.nr, tx = threadIdx.x, ty = threadIdx.y;
-  const int j = blockIdx.x * RT_C + tx, i0 = blockIdx.y * RT_R;
-  const int jc = (j < ns) ? j : ns - 1; // columns past the edge only fill the tile
-  const R dt = (R)c->dt, Of = (R)c->omega_frame, dtheta = (R)(a.pm / (double)ns);
-  // Work values of rings i0-2 .. i0+RT_R+1
-  for (int q = ty; q < RT_R + 4; q += RT_R) {
-    const int r = i0 - 2 + q;
-    if (r < 0 || r > nr - 1) {
-#pragma unroll
-      for (int k = 0; k < 7; k++) sW[k][q][tx] = R(0);
-      continue;
-    }
-    R Q[6];
-    rad_quantities<T, R>(a, r, jc, Of, Q);
-    // the Work values Q / (rho + 1e-20) share one reciprocal per cell
-    const R inv = TransportArith<T>::div(R(1), Q[5] + R(1e-20));
-#pragma unroll
-    for (int k = 0; k < 6; k++) sW[k][q][tx] = Q[k] * inv;
-    sW[6][q][tx] = Q[5];
-  }
-  __syncthreads();
-  // slopes at rings i0-1 .. i0+RT_R
-  for (int q = ty; q < RT_R + 2; q += RT_R) {
-    const int r = i0 - 1 + q;
-#pragma unroll
-    for (int k = 0; k < 7; k++) sD[k][q][tx] = rad_slope<T>(a, r, sW[k][q][tx], sW[k][q + 1][tx], sW[k][q + 2][tx]);
-  }
-  __syncthreads();
-  const int i = i0 + ty;
-  if (j >= ns || i >= nr) return;
-  const long l = (long)i * ns + j;
-  const R v0 = (R)((const T *)a.vri)[l], v1 = (R)((const T *)a.vri)[l + ns];
-  // stars at faces i (Work of rings i-1, i: slots ty+1, ty+2; slopes of
-  // rings i-1, i: slots ty, ty+1) and i+1
-  const RadFace<R> f0 = rad_face<R>(a, i, v0, dt), f1 = rad_face<R>(a, i + 1, v1, dt);
-  const R rs0 = rad_star<R>(f0, sW[6][ty + 1][tx], sW[6][ty + 2][tx], sD[6][ty][tx], sD[6][ty + 1][tx]);
-  const R rs1 = rad_star<R>(f1, sW[6][ty + 2][tx], sW[6][ty + 3][tx], sD[6][ty + 1][tx], sD[6][ty + 2][tx]);
-  R Q[6];
-  rad_quantities<T, R>(a, i, j, Of, Q);
-  const R fin = dt * dtheta * (R)a.Rinf[i], fout = dt * dtheta * (R)a.Rsup[i], invs = (R)a.InvSurf[i];
-  void *outp[6] = {a.t_rp, a.t_rm, a.t_tp, a.t_tm, a.t_en, a.t_rho};
-#pragma unroll
-  for (int k = 0; k < 6; k++) {
-    if (k == 4 && !a.energy) continue;
-    if (k < 4 && DF_ON(T, a) && a.tr_skip_mom) {
-      ((T *)outp[k])[l] = (T)Q[k];
-      continue;
-    }
-    const R q0 = rad_star<R>(f0, sW[k][ty + 1][tx], sW[k][ty + 2][tx], sD[k][ty][tx], sD[k][ty + 1][tx]);
-    const R q1 = rad_star<R>(f1, sW[k][ty + 2][tx], sW[k][ty + 3][tx], sD[k][ty + 1][tx], sD[k][ty + 2][tx]);
-    // VanLeerRadial (src/TransportEuler.c:205-217)
-    R varq = fin * q0 * rs0 * v0;
-    varq -= fout * q1 * rs1 * v1;
-    ((T *)outp[k])[l] = sr_round<T>((double)Q[k] + (double)(varq * invs), sr_key(c, l, SR_RAD + k));
-    if (k == 5 && i == 0) a.lost_col[j] = (double)varq;
-  }
-}
-
-// Azimuthal transport (OneWindTheta, src/TransportEuler.c:225-465) on ring
-// segments, one wavefront each: the residual and uniform passes and the
-// shift.  The ring quantities of the FARGO scheme come first, in FP64
-// whatever the storage type, from the per-tile sums k_source leaves of the
-// velocity before transport: the mean VMed
-// (ComputeAverageThetaVelocities), the integer shift Nshift and the
-// constant residual (ComputeConstantResidual, src/TransportEuler.c:292-348).
-// Every wavefront of a ring forms them from the same sums in the same
-// order, so all agree on the shift.
+// Transport (ComputeLRMomenta, OneWindRad and OneWindTheta,
+// src/TransportEuler.c:89-465): a wavefront holds 64 consecutive columns, one a
+// lane, and walks outwards through a strip of S rings.  At each ring the radial
+// pass completes the ring before, which then takes the residual and the uniform
+// azimuthal pass and the integer shift while it is still in registers.
+//
+// Radial and azimuthal pass as kernels of their own each were at the memory's
+// rate with FP64 storage (1024x3072: 86 and 72 us; five quantities written by
+// one and read by the other, 250 MB) and bound by VALU issue with FP32 storage
+// (55 and 70 us).  Together they take 104 and 97 us, bound by VALU issue: they
+// read the state and write the transported quantities once, and a value rounds
+// to storage once.  What is counted beyond
+// that is instructions: each Work value Q / (rho + 1e-20), difference, slope,
+// face value and flux is formed once (tiles in LDS formed every radial face
+// twice and 10/8 of the slopes: 90 us for the radial pass alone).  A strip
+// repeats the Work of four rings and the slopes of two at its ends, a wavefront
+// eight of its 64 columns; transport_strip picks S.  FP64 whatever the storage
+// type.
+//
+// The ring quantities of the FARGO scheme come first, from the per-tile sums
+// k_source leaves of the velocity before transport: the mean VMed
+// (ComputeAverageThetaVelocities), the integer shift Nshift and the constant
+// residual (ComputeConstantResidual, src/TransportEuler.c:292-348), two lanes
+// per ring of the strip.  Every wavefront of a ring forms them from the same
+// sums in the same order, so all agree on the shift.
 
 // The cells a wavefront owns: its 64 lanes hold 64 consecutive cells of a
 // ring, and each of the two passes leaves two fewer valid cells at either
@@ -1747,129 +1630,341 @@ template <typename T> __global__ void __launch_bounds__(RT_C * RT_R) k_transport
 #define AZ_OWN (AZ_LANES - 2 * AZ_HALO)
 
 // The neighbouring lanes' values: lane L receives lane L - 1's (prev) or
-// lane L + 1's (next); the end lanes receive their own, which only feeds
-// cells outside the valid range.  CDNA's whole-wavefront DPP shifts
-// (wave_shr:1, wave_shl:1) move each 32-bit half in one VALU operation,
-// without the LDS crossbar of a general lane permute.
+// lane L + 1's (next); the end lanes receive zeros, which only feed cells
+// outside the valid range.  CDNA's whole-wavefront DPP shifts (wave_shr:1,
+// wave_shl:1) move each 32-bit half in one VALU operation, without the LDS
+// crossbar of a general lane permute; with zeros for the end lanes the move
+// needs no copy of its destination first.
 template <int CTRL> __device__ __forceinline__ double dpp_shift(double v) {
-  const int lo = __double2loint(v), hi = __double2hiint(v);
-  return __hiloint2double(__builtin_amdgcn_update_dpp(hi, hi, CTRL, 0xf, 0xf, false),
-                          __builtin_amdgcn_update_dpp(lo, lo, CTRL, 0xf, 0xf, false));
+  return __hiloint2double(__builtin_amdgcn_update_dpp(0, __double2hiint(v), CTRL, 0xf, 0xf, true),
+                          __builtin_amdgcn_update_dpp(0, __double2loint(v), CTRL, 0xf, 0xf, true));
 }
 #define DPP_WAVE_SHL1 0x130
 #define DPP_WAVE_SHR1 0x138
 __device__ __forceinline__ double lane_prev(double v) { return dpp_shift<DPP_WAVE_SHR1>(v); }
 __device__ __forceinline__ double lane_next(double v) { return dpp_shift<DPP_WAVE_SHL1>(v); }
 
-// ComputeStarTheta (src/TransportEuler.c:419-444) at this lane's cell (the
-// face between the previous cell and this one), for the values x, the
-// velocity v of the cell and the time step dt
-template <typename T, typename R = typename TransportArith<T>::type>
-__device__ __forceinline__ R azi_star_lane(R x, R v, R dt, R dxtheta, R invdxtheta) {
-  const R xm = lane_prev(x), xp = lane_next(x);
-  const R dqm = x - xm, dqp = xp - x;
-  const R dq = (dqp * dqm > R(0)) ? TransportArith<T>::div(dqp * dqm, dqp + dqm) * invdxtheta : R(0);
-  const R dqprev = lane_prev(dq);
-  const R ksi = v * dt;
-  if (ksi > R(0)) return xm + (dxtheta - ksi) * dqprev;
-  return x - (dxtheta + ksi) * dq;
+// The operations' order.  With FP64 storage the transport keeps the
+// reference's products and sums one by one (over thousands of sub-steps of a
+// nearly steady flow another order of them drifts from it by more than 1e-12);
+// with FP32 storage, whose rounding is 2^29 times as large, products shared by
+// the quantities are formed once and accumulated by fused multiply-adds, a
+// fifth fewer instructions.
+template <typename T> constexpr bool kExactOrder = sizeof(T) == sizeof(double);
+template <typename T> __device__ __forceinline__ double mul_add(double a, double b, double c) {
+  if constexpr (kExactOrder<T>) return a * b + c;
+  else return fma(a, b, c);
+}
+
+// What an azimuthal pass shares over its quantities, for the velocity v of this
+// lane's face (between the previous cell and this one): the upwind side, and
+// the weights with which a cell's slope enters the values at its two faces
+// (ComputeStarTheta, src/TransportEuler.c:419-444): dxtheta - v dt at its right
+// face, which is the next lane's, when that one is left by this cell, and
+// -(dxtheta + v dt) at its left.
+struct AziFace {
+  bool up;
+  double wl, wr;
+};
+struct AziRing {
+  double dx, invdx, dxrad, invsurf;
+};
+template <typename T> __device__ __forceinline__ AziFace azi_face(double v, double dt, const AziRing &g) {
+  const double ksi = v * dt;
+  if constexpr (kExactOrder<T>) return {ksi > 0.0, -(g.dx + ksi), lane_next(g.dx - ksi)};
+  // the slope's 1 / dxtheta goes into the weights
+  const double x = ksi * g.invdx;
+  return {ksi > 0.0, -(1.0 + x), lane_next(1.0 - x)};
+}
+// the value at this lane's face for the cell values x; one difference per
+// face (a cell's second one is its neighbour's)
+template <typename T> __device__ __forceinline__ double azi_star_lane(double x, const AziFace &f, const AziRing &g) {
+  const double dqp = lane_next(x) - x, dqm = lane_prev(dqp);
+  // the quotient is formed on every lane and selected (where it is not used
+  // it may be a NaN of a zero sum, which the select discards)
+  const double prod = dqp * dqm;
+  double d = div_nr(prod, dqp + dqm);
+  if constexpr (kExactOrder<T>) d *= g.invdx;
+  const double dq = prod > 0.0 ? d : 0.0;
+  const double left = lane_prev(mul_add<T>(f.wr, dq, x)), right = mul_add<T>(f.wl, dq, x);
+  return f.up ? left : right;
 }
 
 // QuantitiesAdvection (src/TransportEuler.c:375-400) with velocity v: the
 // density star first, then every quantity's star, flux and update.  Q[5]
 // is the density.  The flux through this lane's face is dxrad S RS v; the
-// cell's update is its own face's flux minus the next lane's.
-template <typename T, typename R = typename TransportArith<T>::type>
-__device__ __forceinline__ void azi_pass_lane(const KArgs &a, R (&Q)[6], R v, R dt, R dxtheta, R invdxtheta,
-                                              R dxrad, R invsurf) {
-  const R RI = Q[5];
-  const R RS = azi_star_lane<T>(RI, v, dt, dxtheta, invdxtheta);
+// cell's update is its own face's flux minus the next lane's, over the surface.
+template <typename T, bool E>
+__device__ __forceinline__ void azi_pass_lane(const KArgs &a, double (&Q)[6], double v, double dt, const AziRing &g) {
+  const double RI = Q[5];
+  const AziFace f = azi_face<T>(v, dt, g);
+  const double rs = azi_star_lane<T>(RI, f, g), rsv = rs * v * (g.dxrad * g.invsurf);
   // the Work values Q / (rho + 1e-20) share one reciprocal
-  const R inv = TransportArith<T>::div(R(1), RI + R(1e-20));
+  const double inv = div_nr(1.0, RI + 1e-20);
 #pragma unroll
   for (int q = 0; q < 6; q++) {
-    if (q == 4 && !a.energy) continue;
+    if (q == 4 && !E) continue;
     if (q < 4 && DF_ON(T, a) && a.tr_skip_mom) continue;
-    const R S = azi_star_lane<T>(Q[q] * inv, v, dt, dxtheta, invdxtheta);
-    const R f = dxrad * S * RS * v;
-    const R fn = lane_next(f);
-    R varq = f;
-    varq -= fn;
-    Q[q] += varq * invsurf;
+    const double star = azi_star_lane<T>(Q[q] * inv, f, g);
+    if constexpr (kExactOrder<T>) {
+      const double flux = g.dxrad * star * rs * v;
+      Q[q] += (flux - lane_next(flux)) * g.invsurf;
+    } else {
+      const double flux = star * rsv;
+      Q[q] += flux - lane_next(flux);
+    }
   }
 }
 
-template <typename T> __global__ void __launch_bounds__(256) k_transport_azi(KArgs a) {
-  using R = typename TransportArith<T>::type;
+// the state of one cell of the newest ring, as stored, and vr at its outer face
+template <typename T> struct RadRaw {
+  T rho, vt, vtp, en, vr_out;
+};
+template <typename T, bool E>
+__device__ __forceinline__ RadRaw<T> rad_load(const KArgs &a, int r, int j, int jp) {
+  const long l = (long)r * a.ns;
+  RadRaw<T> q;
+  q.rho = ((const T *)a.rho)[l + j];
+  q.vt = ((const T *)a.vti)[l + j];
+  q.vtp = ((const T *)a.vti)[l + jp];
+  q.vr_out = ((const T *)a.vri)[l + a.ns + j];
+  q.en = E ? ((const T *)a.en)[l + j] : (T)0;
+  return q;
+}
+// lane k's value (k uniform); only where every lane is active
+__device__ __forceinline__ double lane_value(double v, int k) {
+  return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), k),
+                          __builtin_amdgcn_readlane(__double2loint(v), k));
+}
+// v plus the value of the other lane of its pair (quad_perm 1,0,3,2)
+__device__ __forceinline__ double pair_sum(double v) {
+  return v + __hiloint2double(__builtin_amdgcn_update_dpp(0, __double2hiint(v), 0xB1, 0xf, 0xf, true),
+                              __builtin_amdgcn_update_dpp(0, __double2loint(v), 0xB1, 0xf, 0xf, true));
+}
+// rings per strip, at most (two lanes per ring hold its FARGO values)
+#define TR_STRIP_MAX 32
+// wavefronts per SIMD the registers allow: 166 of them without the energy
+// equation; with it 188, which three wavefronts' budget of 168 would spill
+// (256x768 FP64: 24 us against 21)
+constexpr int tr_occupancy(bool energy) { return energy ? 2 : 3; }
+
+// Quantity slots: 0 rp, 1 rm, 2 tp, 3 tm, 4 e (E: the energy equation), 5 rho
+// (the Work of the density itself); slot 6 of the radial pass's values is rho
+// as its own base for RhoStar.
+template <typename T, bool E> __global__ void __launch_bounds__(256, tr_occupancy(E)) k_transport_azi(KArgs a, int S) {
   const dfargo_ctrl *c = a.ctrl;
   if (!c->active) return;
-  const int ns = a.ns, i = blockIdx.y, lane = threadIdx.x & (AZ_LANES - 1);
-  const int seg = blockIdx.x * (blockDim.x / AZ_LANES) + threadIdx.x / AZ_LANES;
+  const int ns = a.ns, nr = a.nr, lane = threadIdx.x & (AZ_LANES - 1), per = blockDim.x / AZ_LANES;
+  // the blocks of one XCD take neighbouring segments and strips (ring_of_block)
+  const int nb = gridDim.x * gridDim.y, b0 = blockIdx.y * gridDim.x + blockIdx.x;
+  const int b = (a.xcd_remap && nb % 8 == 0) ? (b0 % 8) * (nb / 8) + b0 / 8 : b0;
+  const int seg = __builtin_amdgcn_readfirstlane((b % gridDim.x) * per + threadIdx.x / AZ_LANES);
+  const int i0 = (b / gridDim.x) * S, i1 = (i0 + S < nr) ? i0 + S : nr;
   if (seg * AZ_OWN >= ns) return; // a whole wavefront
   int j = (seg * AZ_OWN - AZ_HALO + lane) % ns;
   if (j < 0) j += ns;
-  const long base = (long)i * ns;
-  const double dt = c->dt, invdt = 1.0 / dt;
-  // the ring's mean velocity, shift and residual
-  const int ntile = (ns + DF_SRC_COLS - 1) / DF_SRC_COLS;
-  double sum = 0.0;
-  for (int t = lane; t < ntile; t += AZ_LANES) sum += a.vt_part[(long)i * ntile + t];
-  const double vmed = wave_sum(sum) / (double)ns;
-  const double dpinvns = a.pm / (double)ns;
-  const double Ntilde = vmed * a.InvRmed[i] * dt * (double)ns / a.pm;
-  const double Nround = floor(Ntilde + 0.5);
-  const long nshift = (long)Nround;
-  const double u = (Ntilde - Nround) * a.Rmed[i] * invdt * dpinvns;
-  if (seg == 0 && lane == 0) {
-    a.vmed[i] = vmed;
-    a.nshift[i] = nshift;
-    // distance of Ntilde from the nearest rounding tie, min over the call
-    // (the gas's shift)
-    const double margin = 0.5 - fabs(Ntilde - Nround);
-    if (!(DF_ON(T, a) && a.tr_dust))
-      atomicMin(&a.ctrl->fargo_margin_bits, (unsigned long long)__double_as_longlong(margin > 0.0 ? margin : 0.0));
-  }
-  // mass through the inner edge (VanLeerRadial's LostByDisk, ring 0;
-  // LostMassd for the dust fluid)
-  if (i == 0 && seg == 0) {
-    double lost = 0.0;
-    for (int jj = lane; jj < ns; jj += AZ_LANES) lost += a.lost_col[jj];
-    lost = wave_sum(lost);
-    if (lane == 0) {
-      if (DF_ON(T, a) && a.tr_dust) a.ctrl->lost_massd += lost;
-      else a.ctrl->lost_mass += lost;
+  const int jp = (j == ns - 1) ? 0 : j + 1;
+  const double dt = c->dt, invdt = 1.0 / dt, Of = c->omega_frame, dtheta = a.pm / (double)ns;
+  const bool skip_mom = DF_ON(T, a) && a.tr_skip_mom;
+  const int rb = (i0 - 2 > 0) ? i0 - 2 : 0;
+  double v_r = (double)((const T *)a.vri)[(long)rb * ns + j]; // vr at face r
+  RadRaw<T> next = rad_load<T, E>(a, rb, j, jp);
+  // ring tables of the walk, ring rb + k in lane k: read once, ahead (a scalar
+  // load per ring would make the walk wait for each)
+  const int rt = (rb + lane < nr + 1) ? rb + lane : nr + 1;
+  const double tRmed = a.Rmed[rt], tIdr = a.InvDiffRmed[rt], tRinf = a.Rinf[rt], tInvS = a.InvSurf[rt];
+  // the FARGO scheme's ring values, ring i0 + k in the lanes 2 k and 2 k + 1
+  double gV, gU, gDx, gInvDx, gDxrad;
+  int gShift;
+  {
+    const int ntile = (ns + DF_SRC_COLS - 1) / DF_SRC_COLS;
+    const int i = (i0 + (lane >> 1) < i1) ? i0 + (lane >> 1) : i1 - 1;
+    double sum = 0.0;
+    for (int t0 = 0; t0 < ntile; t0 += 16) {
+      double x[8]; // in flight together
+#pragma unroll
+      for (int q = 0; q < 8; q++) {
+        const int t = t0 + 2 * q + (lane & 1);
+        x[q] = t < ntile ? a.vt_part[(long)i * ntile + t] : 0.0;
+      }
+#pragma unroll
+      for (int q = 0; q < 8; q++) sum += x[q];
+    }
+    gV = pair_sum(sum) / (double)ns;
+    const double Ntilde = gV * a.InvRmed[i] * dt * (double)ns / a.pm;
+    const double Nround = floor(Ntilde + 0.5);
+    const long nshift = (long)Nround;
+    gU = (Ntilde - Nround) * a.Rmed[i] * invdt * (a.pm / (double)ns);
+    gDx = a.pm / (double)ns * a.Rmed[i];
+    gInvDx = 1.0 / gDx;
+    gDxrad = (a.Rsup[i] - a.Rinf[i]) * dt;
+    long sh = nshift % ns;
+    if (sh < 0) sh += ns;
+    gShift = (int)sh;
+    if (seg == 0) {
+      // distance of Ntilde from the nearest rounding tie, min over the call
+      // (the gas's shift)
+      double margin = 0.5 - fabs(Ntilde - Nround);
+      margin = wave_min(margin > 0.0 ? margin : 0.0);
+      if ((lane & 1) == 0 && i0 + (lane >> 1) < i1) {
+        a.vmed[i] = gV;
+        a.nshift[i] = nshift;
+      }
+      if (lane == 0 && !(DF_ON(T, a) && a.tr_dust))
+        atomicMin(&a.ctrl->fargo_margin_bits, (unsigned long long)__double_as_longlong(margin));
     }
   }
-  // quantities after the radial pass: rp, rm, tp, tm, [e], rho; the
-  // results go to z_*, since other wavefronts of the ring may still read
-  // the cells this one stores
-  const void *qp[6] = {a.t_rp, a.t_rm, a.t_tp, a.t_tm, a.t_en, a.t_rho};
-  void *zp[6] = {a.z_rp, a.z_rm, a.z_tp, a.z_tm, a.z_en, a.z_rho};
-  R Q[6];
-#pragma unroll
-  for (int q = 0; q < 6; q++) Q[q] = (q == 4 && !a.energy) ? R(0) : (R)((const T *)qp[q])[base + j];
-  // the residual velocity of the cell (src/TransportEuler.c:280-290)
-  double v = (ld<T>(a.vti, base + j) * dt) * invdt - vmed;
-  if (!a.fast) v = u + v;
-  const double dxth = a.pm / (double)ns * a.Rmed[i];
-  const R dxtheta = (R)dxth, invdxtheta = (R)(1.0 / dxth);
-  const R dxrad = (R)((a.Rsup[i] - a.Rinf[i]) * dt), invsurf = (R)(1.0 / a.Surf[i]), rdt = (R)dt;
-  // residual pass (the only pass of the standard transport), then the
-  // uniform pass with the constant residual
-  azi_pass_lane<T>(a, Q, (R)v, rdt, dxtheta, invdxtheta, dxrad, invsurf);
-  if (a.fast) azi_pass_lane<T>(a, Q, (R)u, rdt, dxtheta, invdxtheta, dxrad, invsurf);
-  // AdvectSHIFT (src/TransportEuler.c:350-373): new[j] = old[j - Nshift]
   const int own = lane - AZ_HALO;
-  if (own < 0 || own >= AZ_OWN || seg * AZ_OWN + own >= ns) return;
-  long sh_mod = nshift % ns;
-  if (sh_mod < 0) sh_mod += ns;
-  long jn = j + sh_mod;
-  if (jn >= ns) jn -= ns;
+  const bool store = own >= 0 && own < AZ_OWN && seg * AZ_OWN + own < ns;
+  void *zp[6] = {a.z_rp, a.z_rm, a.z_tp, a.z_tm, a.z_en, a.z_rho};
+  // Entering step r (the newest ring read is r, q = r - 1 the one before):
+  // Qq, Wq, vtq: ring q; Qp, vtp: ring q - 1; diff: the scaled differences
+  // across face q (between rings q - 1 and q); right: the values of ring q - 1
+  // at face q; flux: through face q - 1; v: the velocity at face q.
+  double Qp[6], Qq[6], Wq[7], diff[7], right[7], flux[6], v = 0.0, vtq = 0.0, vtp = 0.0;
 #pragma unroll
-  for (int q = 0; q < 6; q++) {
-    if (q == 4 && !a.energy) continue;
-    ((T *)zp[q])[base + jn] = sr_round<T>((double)Q[q], sr_key(c, base + jn, SR_AZI + q));
+  for (int k = 0; k < 7; k++) Wq[k] = diff[k] = right[k] = 0.0;
+#pragma unroll
+  for (int k = 0; k < 6; k++) Qp[k] = Qq[k] = flux[k] = 0.0;
+  for (int r = rb; r <= i1 + 1; r++) {
+    const RadRaw<T> raw = next;
+    if (r + 1 < nr && r <= i1) next = rad_load<T, E>(a, r + 1, j, jp);
+    const int tr = r - rb; // table lane of ring r
+    // (beyond the last ring the walk repeats it, with differences of weight 0)
+    const double d = (double)raw.rho, Rm = lane_value(tRmed, tr), RO = Rm * Of, v_out = (double)raw.vr_out;
+    const double Q[6] = {d * v_out,
+                         d * v_r,
+                         d * ((double)raw.vtp + RO) * Rm,
+                         d * ((double)raw.vt + RO) * Rm,
+                         E ? (double)raw.en : 0.0,
+                         d};
+    // the Work values share one reciprocal per cell
+    const double inv = div_nr(1.0, d + 1e-20);
+    double W[7];
+#pragma unroll
+    for (int k = 0; k < 6; k++) W[k] = Q[k] * inv;
+    W[6] = d;
+    const int q = r - 1;
+    if (q >= 0) {
+      // ComputeStarRad: the slopes of ring q (zero on the first and last), the
+      // values of ring q at its lower face q and its upper face r, and with
+      // them the values at face q from the upwind side; the faces 0 and nr are
+      // closed
+      const double idr = r < nr ? lane_value(tIdr, tr) : 0.0;
+      const bool inner = q > 0 && q < nr - 1, open = q > 0 && q < nr;
+      const double gap = (inner && tr > 0) ? lane_value(tRmed, tr) - lane_value(tRmed, tr - 1) : 0.0; // q to r
+      const double wl = -0.5 * (gap + v * dt), wr = 0.5 * (gap - v_r * dt);
+      double star[7];
+#pragma unroll
+      for (int k = 0; k < 7; k++) {
+        if (k == 4 && !E) continue;
+        const double dm = diff[k];
+        const double dp = (W[k] - Wq[k]) * idr;
+        diff[k] = dp;
+        // the quotient is formed on every lane and selected (where it is not
+        // used it may be a NaN of a zero sum, which the select discards)
+        const double prod = dp * dm, x = div_nr(2.0 * prod, dp + dm);
+        const double slope = (inner && prod > 0.0) ? x : 0.0;
+        star[k] = v > 0.0 ? right[k] : mul_add<T>(wl, slope, Wq[k]);
+        right[k] = mul_add<T>(wr, slope, Wq[k]);
+      }
+      // VanLeerRadial (src/TransportEuler.c:205-217): the flux through face q,
+      // then ring q - 1's update
+      const double f0 = (open && tr > 0) ? dt * dtheta * lane_value(tRinf, tr - 1) : 0.0, f0sv = f0 * star[6] * v;
+      const int i = q - 1;
+      const bool mine = i >= i0 && i < i1;
+      const double invs = mine ? lane_value(tInvS, tr - 2) : 0.0;
+#pragma unroll
+      for (int k = 0; k < 6; k++) {
+        if (k == 4 && !E) continue;
+        const double f = kExactOrder<T> ? f0 * star[k] * star[6] * v : f0sv * star[k], varq = flux[k] - f;
+        flux[k] = f;
+        if (!(k < 4 && skip_mom)) Qp[k] = mul_add<T>(varq, invs, Qp[k]);
+        if (k == 5 && i == 0 && mine && store) a.lost_col[j] = varq;
+      }
+      if (mine) {
+        // the residual velocity of the cell (src/TransportEuler.c:280-290),
+        // the residual pass (the only pass of the standard transport) and the
+        // uniform pass with the constant residual
+        const int g = 2 * (i - i0);
+        const double vmed = lane_value(gV, g), u = lane_value(gU, g);
+        const AziRing ring = {lane_value(gDx, g), lane_value(gInvDx, g), lane_value(gDxrad, g), invs};
+        double vres = (vtp * dt) * invdt - vmed;
+        if (!a.fast) vres = u + vres;
+        azi_pass_lane<T, E>(a, Qp, vres, dt, ring);
+        if (a.fast) azi_pass_lane<T, E>(a, Qp, u, dt, ring);
+        // AdvectSHIFT (src/TransportEuler.c:350-373): new[j] = old[j - Nshift]
+        // (the shift is read while every lane is active: lane g may be one that
+        // stores nothing, and a register reloaded for the storing lanes alone
+        // would not hold its value)
+        const int shift = __builtin_amdgcn_readlane(gShift, g);
+        if (store) {
+          int jn = j + shift;
+          if (jn >= ns) jn -= ns;
+          const long l = (long)i * ns + jn;
+          const unsigned key = sr_key(c, l, SR_AZI);
+#pragma unroll
+          for (int k = 0; k < 6; k++) {
+            if (k == 4 && !E) continue;
+            ((T *)zp[k])[l] = sr_round<T>(Qp[k], sr_draw(key, k));
+          }
+        }
+      }
+    }
+#pragma unroll
+    for (int k = 0; k < 6; k++) {
+      Qp[k] = Qq[k];
+      Qq[k] = Q[k];
+    }
+#pragma unroll
+    for (int k = 0; k < 7; k++) Wq[k] = W[k];
+    vtp = vtq;
+    vtq = (double)raw.vt;
+    v = v_r;
+    v_r = v_out;
   }
+}
+
+// Rings per strip of the transport.  A strip of S rings walks S + 4, plus its
+// start (about two rings' time), and a last round of wavefronts that is nearly
+// empty costs as much as a full one: the S with the shortest walk times rounds.
+// 1024x3072 FP32: 19 rings (3024 wavefronts on 3072 places) 97 us, 16 rings
+// (3584) 105 us, 8 rings (7168) 99 us; a small grid takes 2.
+static int transport_strip(const KArgs &a, int per) {
+  const long nseg = ((a.ns + AZ_OWN - 1) / AZ_OWN + per - 1) / per * per, places = 4L * tr_occupancy(a.energy) * a.num_cu;
+  int best = 2;
+  long cost = -1;
+  for (int S = 2; S <= TR_STRIP_MAX; S++) {
+    const long t = (nseg * ((a.nr + S - 1) / S) + places - 1) / places * (S + 6);
+    if (cost < 0 || t < cost) {
+      cost = t;
+      best = S;
+    }
+  }
+  return best;
+}
+template <typename T> static void launch_transport(const KArgs &a, hipStream_t s) {
+  const int per = (a.tune_azi_waves == 1 || a.tune_azi_waves == 2) ? a.tune_azi_waves : 4;
+  const int S = transport_strip(a, per), nseg = (a.ns + AZ_OWN - 1) / AZ_OWN;
+  const dim3 g((nseg + per - 1) / per, (a.nr + S - 1) / S), b(per * AZ_LANES);
+  if (a.energy) hipLaunchKernelGGL((k_transport_azi<T, true>), g, b, 0, s, a, S);
+  else hipLaunchKernelGGL((k_transport_azi<T, false>), g, b, 0, s, a, S);
+}
+
+// The mass through the inner edge (VanLeerRadial's LostByDisk, ring 0;
+// LostMassd for the dust fluid) from the columns' fluxes the transport left:
+// one wavefront of the kernel that ends the sub-step for that fluid.
+__device__ __forceinline__ void add_lost_mass(const KArgs &a, const double *col, double *total) {
+  double lost = 0.0;
+  for (int j = threadIdx.x; j < a.ns; j += 8 * 64) {
+    double x[8]; // in flight together
+#pragma unroll
+    for (int q = 0; q < 8; q++) x[q] = j + q * 64 < a.ns ? col[j + q * 64] : 0.0;
+#pragma unroll
+    for (int q = 0; q < 8; q++) lost += x[q];
+  }
+  lost = wave_sum(lost);
+  if (threadIdx.x == 0) *total += lost;
 }
 
 // ComputeVelocities (src/TransportEuler.c:515-547) and the floors
@@ -1980,32 +2075,13 @@ template <typename T> __global__ void __launch_bounds__(256) k_finish(KArgs a) {
   // the sub-step ends here: the next one's loop condition takes effect
   if (blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) a.ctrl->go = c->go_next;
   const int i = blockIdx.y, ns = a.ns, nr = a.nr, j = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i == nr && blockIdx.x == 0 && threadIdx.x < 64) add_lost_mass(a, a.lost_col, &a.ctrl->lost_mass);
   if (j >= ns) return;
   if (i == nr) {
     finish_outer_face<T>(a, c, j);
     return;
   }
   finish_cell<T>(a, c, i, j);
-}
-
-// The same with self-gravity, one workgroup per ring: after storing its
-// ring the workgroup forms the ring's reduced densities from the values it
-// stored and transforms them (compute_fftdensity and the azimuthal FFT of
-// the next sub-step, src/sgdens.c:54-70), so that the next sub-step's
-// self-gravity starts from the radial transforms.  The workgroup of ring
-// nrad-1 also stores the outer face.
-template <typename T> __global__ void __launch_bounds__(SG_TB_MAX) k_finish_rows(KArgs a, cx<T> *zt) {
-  extern __shared__ unsigned char smem[];
-  const dfargo_ctrl *c = a.ctrl;
-  if (!c->active) return;
-  if (blockIdx.x == 0 && threadIdx.x == 0) a.ctrl->go = c->go_next;
-  const int i = ring_of_block(a), ns = a.ns, nr = a.nr;
-  cx<T> *A = (cx<T> *)smem, *B = A + fpsz(ns);
-  for (int j = threadIdx.x; j < ns; j += blockDim.x) {
-    A[fp(j)] = sg_reduced<T>(a, i, finish_cell<T>(a, c, i, j));
-    if (i == nr - 1) finish_outer_face<T>(a, c, j);
-  }
-  sg_row_transform<T>(a, i, A, B, zt);
 }
 
 // EvanescentBoundary (src/SideEuler.c:796-950) for the gas, after the
@@ -2427,9 +2503,10 @@ static dim3 cell_grid(const KArgs &a, int rings) {
 }
 static dim3 cell_block(const KArgs &a) { return dim3(a.ns < 256 ? a.ns : 256); }
 // the velocity/boundary kernel's workgroup: the tuned width, at most a ring
+// in whole wavefronts
 static int finish_bx(const KArgs &a) {
   const int w = (a.tune_finish_block == 64 || a.tune_finish_block == 128) ? a.tune_finish_block : 256;
-  return a.ns < w ? a.ns : w;
+  return a.ns < w ? (a.ns + 63) / 64 * 64 : w;
 }
 
 template <typename T> void launch_kernel(int id, const KArgs &a, hipStream_t s) {
@@ -2452,24 +2529,8 @@ template <typename T> void launch_kernel(int id, const KArgs &a, hipStream_t s) 
                          a);
       break;
     case KID_ENERGY: RING_DISPATCH(k_energy, T, a, s, 0); break;
-    case KID_TRANSPORT_RAD: {
-      dim3 g((a.ns + RT_C - 1) / RT_C, (a.nr + RT_R - 1) / RT_R);
-      hipLaunchKernelGGL(k_transport_rad<T>, g, dim3(RT_C, RT_R), 0, s, a);
-      break;
-    }
-    case KID_TRANSPORT_AZI: {
-      const int per = (a.tune_azi_waves == 1 || a.tune_azi_waves == 2) ? a.tune_azi_waves : 4;
-      const int nseg = (a.ns + AZ_OWN - 1) / AZ_OWN;
-      hipLaunchKernelGGL(k_transport_azi<T>, dim3((nseg + per - 1) / per, a.nr), dim3(per * AZ_LANES), 0, s, a);
-      break;
-    }
+    case KID_TRANSPORT_AZI: launch_transport<T>(a, s); break;
     case KID_FINISH: {
-      if (a.sg_rows_in_finish) {
-        const size_t lds = sg_rows_lds_bytes(a, sizeof(cx<T>));
-        hipLaunchKernelGGL(k_finish_rows<T>, dim3(a.nr), dim3(sg_threads(a, lds, a.nr, a.ns / 2)), lds, s, a,
-                           (cx<T> *)a.sg_z);
-        break;
-      }
       const int bx = finish_bx(a);
       hipLaunchKernelGGL(k_finish<T>, dim3((a.ns + bx - 1) / bx, a.nr + 1), dim3(bx), 0, s, a);
       break;
@@ -2486,7 +2547,6 @@ template <typename T> void launch_kernel(int id, const KArgs &a, hipStream_t s) 
     case KID_DF_STRESS:
     case KID_DF_VISC:
     case KID_DF_SUBSTEP2:
-    case KID_DF_TRANSPORT_RAD:
     case KID_DF_TRANSPORT_AZI:
     case KID_DF_FINISH:
       // the dust fluid runs with FP64 storage only (the context refuses it
@@ -2511,13 +2571,7 @@ void launch_algogas_begin(const KArgs &a, double DT, hipStream_t s) {
 }
 
 template <typename T> void prepare_kernels(const KArgs &a) {
-  if (a.sg && !a.sg_zero) {
-    sg_prepare<T>(a);
-    // dynamic LDS above 64 KiB must be requested (gfx950 has 160 KiB per CU)
-    const size_t lds = sg_rows_lds_bytes(a, sizeof(cx<T>));
-    if (lds > 65536)
-      hipFuncSetAttribute((const void *)k_finish_rows<T>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-  }
+  if (a.sg && !a.sg_zero) sg_prepare<T>(a);
 }
 template void prepare_kernels<double>(const KArgs &);
 template void prepare_kernels<float>(const KArgs &);
