@@ -270,7 +270,10 @@ __global__ void __launch_bounds__(64) k_df_substep2(KArgs a) {
   const dfargo_ctrl *c = a.ctrl;
   if (!c->active) return;
   const int i = blockIdx.y, ns = a.ns, nr = a.nr;
-  const int j = blockIdx.x * DF_SRC_COLS + threadIdx.x;
+  // the lanes of k_source's segments, so that the sums have its order; the
+  // others only take part in the sum
+  const int own = (int)threadIdx.x - AZ_HALO;
+  const int j = own >= 0 && own < AZ_OWN ? blockIdx.x * DF_SRC_COLS + own : ns;
   const double dt = c->dt, invdt = 1.0 / dt;
   const double *vr = a.dvri, *vt = a.dvti, *drho = a.drho;
   double rate = 0.0;
@@ -478,7 +481,7 @@ static void launch_df_kernel(int id, const KArgs &a, hipStream_t s) {
     case KID_DF_VISC: hipLaunchKernelGGL(k_df_visc, g, b, 0, s, a); break;
     case KID_DF_SUBSTEP2: {
       const int ntile = (a.ns + DF_SRC_COLS - 1) / DF_SRC_COLS;
-      hipLaunchKernelGGL(k_df_substep2, dim3(ntile, a.nr + 1), dim3(DF_SRC_COLS), 0, s, a);
+      hipLaunchKernelGGL(k_df_substep2, dim3(ntile, a.nr + 1), dim3(64), 0, s, a);
       break;
     }
     case KID_DF_TRANSPORT_AZI: launch_transport<double>(df_transport_args(a), s); break;

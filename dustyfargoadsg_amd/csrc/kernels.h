@@ -136,8 +136,9 @@ struct KArgs {
   void *sg_z, *sg_w, *sg_kr, *sg_kt, *tw_ns, *tw_2n;
 };
 
-// columns of a source-kernel tile: one wavefront per ring of the tile
-#define DF_SRC_COLS 64
+// columns of a ring whose vtheta the source kernels sum into one partial: those
+// a wavefront owns of the 64 it holds
+#define DF_SRC_COLS 56
 
 // launchers (step.hip, sg.hip); each enqueues on stream s
 enum KernelId {

@@ -222,20 +222,6 @@ __device__ double pot_at(const KArgs &a, const dfargo_ctrl *c, int i, int j) {
   return pot;
 }
 
-// indirect part of the potential felt by the particles (the IndPot grid of
-// FillForcesArrays, src/Pframeforce.c:60-88): the planets' term is
-// assigned, not summed, so the last planet's stands, as in the reference
-__device__ double indpot_at(const KArgs &a, const dfargo_ctrl *c, int i, int j) {
-  const double x = a.Rmed[i] * a.CosAz[j], y = a.Rmed[i] * a.SinAz[j];
-  double ip = 0.0;
-  if (a.indirect_term && a.d_feel_planets && c->nb > 0) {
-    const int k = c->nb - 1;
-    ip = DF_G * c->pot_m[k] * c->pot_invd3[k] * (x * c->pot_x[k] + y * c->pot_y[k]);
-  }
-  if (a.gas_indirect && a.d_feel_disk) ip -= c->ind_x * x + c->ind_y * y;
-  return ip;
-}
-
 // ------------------------------------------------------------------------
 // per-call and per-sub-step control
 // ------------------------------------------------------------------------
@@ -1155,351 +1141,424 @@ template <typename T> __global__ void __launch_bounds__(256) k_visc_stress(KArgs
   st<T>(a.trp, l, Trp);
 }
 
-// Source terms of one sub-step on tiles of SRC_TR rings x SRC_TC columns:
-// SubStep1 (src/SourceEuler.c:865-994, with the self-gravity kick of
-// update_sgvelocity, src/sgupdate.c:30-72), the viscous stresses and
-// velocity update (ComputeViscousTerms + UpdateVelocitiesWithViscosity,
-// src/Viscosity.c:159-378) and SubStep2 (src/SourceEuler.c:1012-1116), in
-// that order, with the intermediate VradInt / VthetaInt and stresses in
-// LDS.  Each stage is evaluated on the tile and the halo the next stage
-// reads: potential on a 4-cell halo, SubStep1 on 3, stresses on 2, the
-// viscous update on 1.  The state is read only; the post-SubStep2
-// velocities go to vri / vti and the energy to e_int (the ActualiseGas
-// copies of src/SourceEuler.c:598-630 are deferred to the end of the
-// sub-step), so no workgroup overwrites what another one still reads.
-#define SRC_TR (SrcBlock<T>::tr)
-#define SRC_TC DF_SRC_COLS
-static_assert(SRC_TC == 64, "the SubStep2 stage sums one tile ring per wavefront");
-#define SRC_PR (SRC_TR + 6)
-#define SRC_PC (SRC_TC + 6)
-#define SRC_VR (SRC_TR + 5)
-#define SRC_VC (SRC_TC + 5)
-#define SRC_SR (SRC_TR + 3)
-#define SRC_SC (SRC_TC + 3)
-#define SRC_FC (SRC_TC + 7)  // state staged on rings i0-4 .. i0+TR+1, columns j0-4 .. j0+TC+2
-// Rings (tr) and threads (n) per tile.  With FP32 storage 16 rings (78 KiB
-// of LDS, two tiles per CU) recompute fewer halo cells per tile cell than
-// 8 rings (48 KiB, three tiles): the kernel runs 11 % faster at 1024x3072.
-// FP64 storage (64 KiB at 8 rings) stays at 8 rings, where 16 measured
-// 15 % slower.  768 threads fill 24 wavefronts per CU either way; the
-// wavefronts hide the latency of the stages' LDS and global reads (256,
-// 512 and 1024 threads measured slower).  The tile shape does not change
-// the results.
-template <typename T> struct SrcBlock {
-  static constexpr int n = 768, tr = 16;
-};
-template <> struct SrcBlock<double> {
-  static constexpr int n = 768, tr = 8;
-};
+// The source and transport kernels hold a ring's cells in wavefronts: 64
+// consecutive cells a wavefront, one a lane.  The values of neighbouring cells
+// are neighbouring lanes', so each step that reads them leaves fewer valid
+// cells at either end; after the source terms (SubStep1, the stresses, the
+// viscous update, SubStep2: one cell each) and after the transport's two
+// azimuthal passes (two cells each) the middle 56 are complete, which the
+// wavefront owns.
+#define AZ_LANES 64
+#define AZ_HALO 4
+#define AZ_OWN (AZ_LANES - 2 * AZ_HALO)
+static_assert(AZ_OWN == DF_SRC_COLS, "the source kernel leaves one partial sum per wavefront");
 
-// the 1-D tables k_source reads, staged per tile
-enum { ST_IDRM, ST_RINF, ST_IRINF, ST_RMED, ST_SUPP, ST_IDXT, ST_NU, ST_RSUP, ST_IDRS, ST_IRMED, ST_N };
-__device__ __forceinline__ const double *src_table(const KArgs &a, int k) {
-  switch (k) {
-    case ST_IDRM: return a.InvDiffRmed;
-    case ST_RINF: return a.Rinf;
-    case ST_IRINF: return a.InvRinf;
-    case ST_RMED: return a.Rmed;
-    case ST_SUPP: return a.supp_torque;
-    case ST_IDXT: return a.InvDxTheta;
-    case ST_NU: return a.nu_ring;
-    case ST_RSUP: return a.Rsup;
-    case ST_IDRS: return a.InvDiffRsup;
-    default: return a.InvRmed;
-  }
+// The neighbouring lanes' values: lane L receives lane L - 1's (prev) or
+// lane L + 1's (next); the end lanes receive zeros, which only feed cells
+// outside the valid range.  CDNA's whole-wavefront DPP shifts (wave_shr:1,
+// wave_shl:1) move each 32-bit half in one VALU operation, without the LDS
+// crossbar of a general lane permute; with zeros for the end lanes the move
+// needs no copy of its destination first.
+template <int CTRL> __device__ __forceinline__ double dpp_shift(double v) {
+  return __hiloint2double(__builtin_amdgcn_update_dpp(0, __double2hiint(v), CTRL, 0xf, 0xf, true),
+                          __builtin_amdgcn_update_dpp(0, __double2loint(v), CTRL, 0xf, 0xf, true));
+}
+#define DPP_WAVE_SHL1 0x130
+#define DPP_WAVE_SHR1 0x138
+__device__ __forceinline__ double lane_prev(double v) { return dpp_shift<DPP_WAVE_SHR1>(v); }
+__device__ __forceinline__ double lane_next(double v) { return dpp_shift<DPP_WAVE_SHL1>(v); }
+
+// The operations' order.  With FP64 storage the source terms and the
+// transport keep the reference's products and sums one by one (over thousands of sub-steps of a
+// nearly steady flow another order of them drifts from it by more than 1e-12);
+// with FP32 storage, whose rounding is 2^29 times as large, products shared by
+// the quantities are formed once and accumulated by fused multiply-adds, a
+// fifth fewer instructions.
+template <typename T> constexpr bool kExactOrder = sizeof(T) == sizeof(double);
+template <typename T> __device__ __forceinline__ double mul_add(double a, double b, double c) {
+  if constexpr (kExactOrder<T>) return a * b + c;
+  else return fma(a, b, c);
 }
 
-template <typename T> __device__ __forceinline__ double src_press(const KArgs &a, long l, int i) {
-  if (!a.energy) {
-    const double cs = (double)(T)a.cs_iso[i];
-    return ld<T>(a.rho, l) * cs * cs;
-  }
-  return (a.gamma - 1.0) * ld<T>(a.en, l);
+// 1 / b to within an ulp, and with it the quotients a / b of that divisor: div_nr's
+// steps, shared where several quotients have one divisor; with FP32 storage
+// the products
+__device__ __forceinline__ double rcp_nr(double b) {
+  double r = __builtin_amdgcn_rcp(b);
+  r = fma(r, fma(-b, r, 1.0), r);
+  return fma(r, fma(-b, r, 1.0), r);
+}
+template <typename T> __device__ __forceinline__ double quotient(double a, double b, double r) {
+  const double q = a * r;
+  if constexpr (!kExactOrder<T>) return q;
+  return fma(r, fma(-b, q, a), q);
+}
+// m / sqrt(x) for the potential: square root and quotient, with FP32 storage
+// from the reciprocal square root
+template <typename T> __device__ __forceinline__ double over_sqrt(double m, double x) {
+  if constexpr (kExactOrder<T>) return div_nr(m, sqrt(x));
+  double y = __builtin_amdgcn_rsq(x);
+  y = fma(0.5 * y, fma(-x * y, y, 1.0), y);
+  return m * fma(0.5 * y, fma(-x * y, y, 1.0), y);
 }
 
-template <typename T> __global__ void __launch_bounds__(SrcBlock<T>::n) k_source(KArgs a) {
-  __shared__ double sPot[SRC_PR][SRC_PC];
-  // VradInt / VthetaInt in FP64 whatever the storage type: their sub-step
-  // increments are kept in full until the final, unbiased rounding
-  __shared__ double sVr[SRC_VR][SRC_VC], sVt[SRC_VR][SRC_VC];
-  __shared__ T sTrr[SRC_SR][SRC_SC], sTpp[SRC_SR][SRC_SC], sTrp[SRC_SR][SRC_SC];
-  // the state the stages read, staged once: density and vtheta as stored,
-  // pressure in FP64 (slot = V slot + 1 = S slot + 2 in both directions)
-  __shared__ T sRho[SRC_PR][SRC_FC], sVth[SRC_PR][SRC_FC];
-  __shared__ double sP[SRC_PR][SRC_FC];
-  __shared__ int sCol[SRC_FC];
-  // the 1-D tables on the staged rings (zero outside the grid)
-  __shared__ double sTab[ST_N][SRC_PR];
-  const dfargo_ctrl *c = a.ctrl;
-  if (!c->active) return;
-  constexpr int TB = SrcBlock<T>::n;
-  const int ns = a.ns, nr = a.nr, tid = threadIdx.x;
-  const int j0 = blockIdx.x * SRC_TC, i0 = blockIdx.y * SRC_TR;
-  const double dt = c->dt;
-#define STAB(k, i) sTab[k][(i) - i0 + 4]
-  // the particles of this sub-step were re-sorted into the other set
-  if (a.d_on && blockIdx.x == 0 && blockIdx.y == 0 && tid == 0) a.ctrl->pset ^= 1;
-  // The global values stage 1 reads at its cells (rings i0-3 .. i0+SRC_TR+1,
-  // columns j0-3 .. j0+SRC_TC+1): loaded first, so that their latency
-  // overlaps the staging below.
-  constexpr int S1_N = SRC_VR * SRC_VC, S1_IT = (S1_N + TB - 1) / TB;
-  T pf_vr[S1_IT], pf_sgr[S1_IT], pf_sgrm[S1_IT], pf_sgt[S1_IT], pf_sgtm[S1_IT];
-#pragma unroll
-  for (int it = 0; it < S1_IT; it++) {
-    const int idx = tid + it * TB, q = idx / SRC_VC, p = idx - q * SRC_VC, i = i0 - 3 + q;
-    pf_vr[it] = pf_sgr[it] = pf_sgrm[it] = pf_sgt[it] = pf_sgtm[it] = (T)0;
-    if (idx < S1_N && i >= 0 && i <= nr - 1) {
-      int j = (j0 - 3 + p) % ns, jm = (j0 - 4 + p) % ns;
-      j = (j < 0) ? j + ns : j;
-      jm = (jm < 0) ? jm + ns : jm;
-      const long l = (long)i * ns + j;
-      if (i >= 1) {
-        pf_vr[it] = ((const T *)a.vr)[l];
-        if (a.sg) {
-          pf_sgr[it] = ((const T *)a.sgr)[l];
-          pf_sgrm[it] = ((const T *)a.sgr)[l - ns];
-        }
-      }
-      if (a.sg) {
-        pf_sgt[it] = ((const T *)a.sgt)[l];
-        pf_sgtm[it] = ((const T *)a.sgt)[(long)i * ns + jm];
-      }
+// lane k's value (k uniform); only where every lane is active
+__device__ __forceinline__ double lane_value(double v, int k) {
+  return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), k),
+                          __builtin_amdgcn_readlane(__double2loint(v), k));
+}
+// Source terms of one sub-step: SubStep1 (src/SourceEuler.c:865-994, with the
+// self-gravity kick of update_sgvelocity, src/sgupdate.c:30-72), the viscous
+// stresses and velocity update (ComputeViscousTerms +
+// UpdateVelocitiesWithViscosity, src/Viscosity.c:159-378) and SubStep2
+// (src/SourceEuler.c:1012-1116), in that order.  A wavefront walks outwards
+// through a strip of S rings with one column a lane: having read ring r it forms
+// VradInt / VthetaInt of ring r, the stresses and the viscous update of VradInt
+// of ring r - 1, and the viscous update of VthetaInt and SubStep2 of ring r - 2,
+// whose inputs are then complete.  Every value is formed once per column, is
+// kept in registers as long as the rings above need it, and comes from the
+// neighbouring columns by lane moves.  The state is read only; the
+// post-SubStep2 velocities go to vri / vti and the energy to e_int (the
+// ActualiseGas copies of src/SourceEuler.c:598-630 are deferred to the end of
+// the sub-step), so no wavefront overwrites what another one still reads.
+//
+// Bound by VALU issue.  As tiles in LDS with a halo per stage the potential
+// was formed 1.9 times a cell (8 rings, FP64) and every operand went through
+// LDS behind a barrier: 118 us at 1024x3072 FP64, 95 us FP32 with
+// self-gravity.  The quotients by the sums of neighbouring densities (six a
+// cell) share two reciprocals.
+//
+// Rings at a strip's ends take only the stages that its own rings need.
+//
+// X: the less used terms, SRC_FRAME a corotating frame and the dust fluid's drag
+// on the gas, SRC_DUST particles (and a frame), whose switches and grids
+// otherwise take the scalar registers of every disc's loop; E: the energy
+// equation.
+enum { SRC_PLAIN = 0, SRC_FRAME = 1, SRC_DUST = 2 };
+#define SRC_STRIP_MAX 32
+// wavefronts per SIMD: the registers of all but the plainest kernel exceed a
+// fourth wavefront's budget of 128
+constexpr int src_occupancy(bool fp64, bool E, int X) { return (fp64 || E || X != SRC_PLAIN) ? 3 : 4; }
+
+// the state of one cell of the newest ring, as stored; x: the particles'
+// feedback accelerations, or the dust fluid's Stokes number, density and
+// velocities where it drags the gas
+template <typename T> struct SrcRaw {
+  T rho, vt, vr, en, sgr, sgt, x[4];
+};
+template <typename T, bool E, int X> __device__ __forceinline__ SrcRaw<T> src_load(const KArgs &a, int r, int j) {
+  const long l = (long)r * a.ns + j;
+  SrcRaw<T> q;
+  q.rho = ((const T *)a.rho)[l];
+  q.vt = ((const T *)a.vt)[l];
+  q.vr = ((const T *)a.vr)[l];
+  q.en = E ? ((const T *)a.en)[l] : (T)0;
+  q.sgr = q.sgt = (T)0;
+  if (a.sg) {
+    q.sgr = ((const T *)a.sgr)[l];
+    q.sgt = ((const T *)a.sgt)[l];
+  }
+  q.x[0] = q.x[1] = q.x[2] = q.x[3] = (T)0;
+  if constexpr (X == SRC_DUST) {
+    if (a.d_feedback) {
+      q.x[0] = ((const T *)a.radfbacc)[l];
+      q.x[1] = ((const T *)a.azifbacc)[l];
     }
   }
-  // columns j0-4 .. j0+SRC_TC+2 of the staged region, wrapped
-  for (int p = tid; p < SRC_FC; p += TB) {
-    int jj = (j0 - 4 + p) % ns;
-    sCol[p] = (jj < 0) ? jj + ns : jj;
+  if constexpr (X == SRC_FRAME) {
+    if (DF_ON(T, a) && a.df_feedback) {
+      q.x[0] = (T)a.dstokes[l];
+      q.x[1] = (T)a.drho[l];
+      q.x[2] = (T)a.dvr[l];
+      q.x[3] = (T)a.dvt[l];
+    }
   }
-  for (int idx = tid; idx < ST_N * SRC_PR; idx += TB) {
-    const int k = idx / SRC_PR, q = idx - k * SRC_PR, r = i0 - 4 + q;
-    sTab[k][q] = (r >= 0 && r <= nr - 1) ? src_table(a, k)[r] : 0.0;
-  }
-  __syncthreads();
-  // stage 0: the state of rings i0-4 .. i0+SRC_TR+1 into LDS, and the
-  // potential there (rings outside the grid hold zeros no valid cell reads)
-  const bool frame_trip = a.d_on && a.d_np > 0 && c->omega_prev != 0.0;
-  for (int idx = tid; idx < SRC_PR * SRC_FC; idx += TB) {
-    const int q = idx / SRC_FC, p = idx - q * SRC_FC, r = i0 - 4 + q;
-    const bool in = (r >= 0 && r <= nr - 1);
-    const long l = (long)r * ns + sCol[p];
-    sRho[q][p] = in ? ((const T *)a.rho)[l] : (T)0;
-    if (in && frame_trip) {
+  return q;
+}
+// the ring tables: ring rb + k in lane k (zero outside the grid), and one ring's
+struct SrcTab {
+  double idrm, rinf, irinf, rmed, supp, idxt, nu, rsup, idrs, irmed, cs, r15;
+};
+__device__ __forceinline__ SrcTab src_tables(const KArgs &a, int i, bool in) {
+  const int k = in ? i : 0;
+  SrcTab t = {a.InvDiffRmed[k], a.Rinf[k], a.InvRinf[k],      a.Rmed[k],    a.supp_torque[k], a.InvDxTheta[k],
+              a.nu_ring[k],     a.Rsup[k], a.InvDiffRsup[k], a.InvRmed[k], a.cs_iso[k],      a.r15[k]};
+  if (!in) t = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
+  return t;
+}
+__device__ __forceinline__ SrcTab src_table_of(const SrcTab &t, int k) {
+  return {lane_value(t.idrm, k), lane_value(t.rinf, k), lane_value(t.irinf, k), lane_value(t.rmed, k),
+          lane_value(t.supp, k), lane_value(t.idxt, k), lane_value(t.nu, k),    lane_value(t.rsup, k),
+          lane_value(t.idrs, k), lane_value(t.irmed, k), lane_value(t.cs, k),   lane_value(t.r15, k)};
+}
+
+template <typename T, bool E, int X>
+__global__ void __launch_bounds__(256, src_occupancy(sizeof(T) == 8, E, X)) k_source(KArgs a, int S) {
+  const dfargo_ctrl *c = a.ctrl;
+  if (!c->active) return;
+  const int ns = a.ns, nr = a.nr, lane = threadIdx.x & (AZ_LANES - 1), per = blockDim.x / AZ_LANES;
+  // the particles of this sub-step were re-sorted into the other set
+  if (X == SRC_DUST && blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) a.ctrl->pset ^= 1;
+  // the blocks of one XCD take neighbouring segments and strips (ring_of_block)
+  const int nb = gridDim.x * gridDim.y, b0 = blockIdx.y * gridDim.x + blockIdx.x;
+  const int b = (a.xcd_remap && nb % 8 == 0) ? (b0 % 8) * (nb / 8) + b0 / 8 : b0;
+  const int seg = __builtin_amdgcn_readfirstlane((b % gridDim.x) * per + threadIdx.x / AZ_LANES);
+  const int i0 = (b / gridDim.x) * S, i1 = (i0 + S < nr) ? i0 + S : nr;
+  if (seg * AZ_OWN >= ns) return; // a whole wavefront
+  int j = (seg * AZ_OWN - AZ_HALO + lane) % ns;
+  if (j < 0) j += ns;
+  const int own = lane - AZ_HALO;
+  const bool store = own >= 0 && own < AZ_OWN && seg * AZ_OWN + own < ns;
+  const int rb = (i0 - 3 > 0) ? i0 - 3 : 0;
+  SrcRaw<T> next = src_load<T, E, X>(a, rb, j);
+  const SrcTab tabs = src_tables(a, rb + lane, rb + lane < nr);
+  const double cosj = a.CosAz[j], sinj = a.SinAz[j];
+  // the planets, planet k in lane k
+  const int npl = c->nb, lp = lane < npl ? lane : 0;
+  const double pX = c->pot_x[lp], pY = c->pot_y[lp], pM = c->pot_m[lp], pS = c->pot_smooth[lp], pI = c->pot_invd3[lp];
+  const double dt = c->dt, invdt = 1.0 / dt, Of = c->omega_frame, ind_x = c->ind_x, ind_y = c->ind_y;
+  const double invdphi = a.invdphi, g1 = a.gamma - 1.0, C2 = DF_CVNR * DF_CVNR, onethird = 1.0 / 3.0;
+  const bool frame_trip = X == SRC_DUST && a.d_np > 0 && c->omega_prev != 0.0;
+  // the change of the corotating frame's rate this sub-step
+  const bool frame = X != SRC_PLAIN && a.frame;
+  const double omega_prev = c->omega_prev, dom = frame ? c->domega : 0.0;
+  const int ntile = (ns + DF_SRC_COLS - 1) / DF_SRC_COLS;
+  const SrcTab zero_tab = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
+  // ring s = r - 1: the state, its density to the left, the reciprocals of the
+  // density sums across its inner and left face, VradInt, VthetaInt
+  double s_rho = 1.0, s_rhojm = 1.0, s_rr = 0.0, s_rt = 0.0, s_vr = 0.0, s_vt = 0.0, s_en = 0.0;
+  double s_p = 0.0, s_pot = 0.0, s_ip = 0.0, s_vt0 = 0.0, s_vtn0 = 0.0, s_sgr = 0.0;
+  SrcTab ts = zero_tab;
+  // ring t = r - 2: the same, VradInt after viscosity, the stresses, SubStep2's
+  // radial pressure of ring t - 1
+  double t_rho = 1.0, t_rhojm = 1.0, t_rr = 0.0, t_rt = 0.0, t_vr = 0.0, t_vt = 0.0, t_en = 0.0;
+  double t_trr = 0.0, t_tpp = 0.0, t_trp = 0.0, u_rho = 1.0, u_qr = 0.0;
+  SrcTab tt = zero_tab;
+  for (int r = rb; r <= i1 + 1; r++) {
+    const SrcRaw<T> raw = next;
+    if (r + 1 < nr && r <= i1) next = src_load<T, E, X>(a, r + 1, j);
+    const SrcTab tr = src_table_of(tabs, r - rb);
+    const int s = r - 1, t = r - 2;
+    // SubStep1 at ring r (VradInt and VthetaInt of ring nrad are zero, as in
+    // the reference where they are never set)
+    const double rho = (double)raw.rho, rhojm = lane_prev(rho), en = (double)raw.en;
+    const double sum_r = rho + s_rho, sum_t = rho + rhojm;
+    const double rr = rcp_nr(sum_r), rt = rcp_nr(sum_t);
+    double vt0 = (double)raw.vt;
+    if (frame_trip) {
       // the particles' interpolation holds vt + Rmed OmegaFrame in the gas
       // grid and subtracts it again (src/Dsys.c:316,1082): SubStep1 reads
       // the round trip's result
-      const double rw = sTab[ST_RMED][q] * c->omega_prev;
-      sVth[q][p] = (T)((ld<T>(a.vt, l) + rw) - rw);
-    } else {
-      sVth[q][p] = in ? ((const T *)a.vt)[l] : (T)0;
+      const double rw = tr.rmed * omega_prev;
+      vt0 = (double)(T)((vt0 + rw) - rw);
     }
-    sP[q][p] = in ? src_press<T>(a, l, r) : 0.0;
-    if (p < SRC_PC) sPot[q][p] = in ? pot_at(a, c, r, sCol[p]) : 0.0;
-  }
-  __syncthreads();
-  // the change of the corotating frame's rate this sub-step
-  const double dom = a.frame ? c->domega : 0.0;
-  // stage 1: SubStep1 on rings i0-3 .. i0+SRC_TR+1 (VradInt and VthetaInt
-  // of ring nrad are zero, as in the reference where they are never set)
-#pragma unroll
-  for (int it = 0; it < S1_IT; it++) {
-    const int idx = tid + it * TB;
-    if (idx >= S1_N) break;
-    const int q = idx / SRC_VC, p = idx - q * SRC_VC, i = i0 - 3 + q, j = sCol[p + 1];
-    if (i < 0 || i > nr - 1) {
-      sVr[q][p] = 0.0;
-      sVt[q][p] = 0.0;
-      continue;
-    }
-    const long l = (long)i * ns + j;
-    const double rl = (double)sRho[q + 1][p + 1], pl = sP[q + 1][p + 1], potl = sPot[q + 1][p + 1];
-    // the particles' grids (pressure gradients, indirect and self-gravity
-    // accelerations, src/SourceEuler.c:893-948) on the tile's own cells
-    const int jt = j0 - 3 + p;
-    const bool dgrid = a.d_on && q >= 3 && q < 3 + SRC_TR && jt >= j0 && jt < j0 + SRC_TC && jt < ns;
-    double vri = 0.0;
-    if (i >= 1) {
-      const double plim = sP[q][p + 1], idrm = STAB(ST_IDRM, i);
-      double gradp = (pl - plim) * 2.0 / (rl + (double)sRho[q][p + 1]) * idrm;
-      double gradphi = (potl - sPot[q][p + 1]) * idrm;
-      double vt2;
-      if (a.frame) {
-        // CorrectVtheta (src/SideEuler.c:1133-1148) on the values read
-        const double ci = dom * STAB(ST_RMED, i), cim = dom * STAB(ST_RMED, i - 1);
-        vt2 = ((double)sVth[q + 1][p + 1] - ci) + ((double)sVth[q + 1][p + 2] - ci) +
-              ((double)sVth[q][p + 1] - cim) + ((double)sVth[q][p + 2] - cim);
-      } else {
-        vt2 = (double)sVth[q + 1][p + 1] + (double)sVth[q + 1][p + 2] + (double)sVth[q][p + 1] +
-              (double)sVth[q][p + 2];
+    const double vtn0 = lane_next(vt0), sgr = (double)raw.sgr;
+    const double cs = (double)(T)tr.cs, p = E ? g1 * en : rho * cs * cs;
+    // the potential (pot_at)
+    double pot = 0.0, ip = 0.0;
+    {
+      const double x = tr.rmed * cosj, y = tr.rmed * sinj;
+      for (int k = 0; k < npl; k++) {
+        const double xp = lane_value(pX, k), yp = lane_value(pY, k), mp = lane_value(pM, k);
+        const double distance = (x - xp) * (x - xp) + (y - yp) * (y - yp);
+        double pk = over_sqrt<T>(-DF_G * mp, distance + lane_value(pS, k));
+        if (a.indirect_term) pk += DF_G * mp * lane_value(pI, k) * (x * xp + y * yp);
+        pot += pk;
       }
-      vt2 = vt2 / 4.0 + STAB(ST_RINF, i) * c->omega_frame;
-      vt2 = vt2 * vt2;
-      vri = (double)pf_vr[it] + dt * (-gradp - gradphi + vt2 * STAB(ST_IRINF, i));
-      if (a.d_on && a.d_feedback) vri += dt * ld<T>(a.radfbacc, l);
-      if (DF_ON(T, a) && a.df_feedback) {
-        // the dust fluid's drag on the gas, implicit (src/SourceEuler.c:915-921)
-        const double ts = a.dstokes[l] * a.r15[i], eps = a.drho[l] / rl;
-        vri = (vri * ts + eps * a.dvr[l] * dt) / (ts + dt * eps);
+      double ps = -DF_G * 1.0 * tr.irmed;
+      const double gi = ind_x * x + ind_y * y;
+      if (a.gas_indirect) ps -= gi;
+      pot += ps;
+      // its indirect part as the particles feel it (the IndPot grid of
+      // FillForcesArrays, src/Pframeforce.c:60-88): the planets' term is
+      // assigned, not summed, so the last planet's stands, as in the reference
+      if (X == SRC_DUST) {
+        if (a.indirect_term && a.d_feel_planets && npl > 0)
+          ip = DF_G * lane_value(pM, npl - 1) * lane_value(pI, npl - 1) *
+               (x * lane_value(pX, npl - 1) + y * lane_value(pY, npl - 1));
+        if (a.gas_indirect && a.d_feel_disk) ip -= gi;
+      }
+    }
+    const double ipjm = X == SRC_DUST ? lane_prev(ip) : 0.0;
+    double vr1 = 0.0, vt1 = 0.0;
+    const double pljm = lane_prev(p), potjm = lane_prev(pot), sgtjm = a.sg ? lane_prev((double)raw.sgt) : 0.0;
+    if (r < nr && r >= i0 - 2) {
+      const long l = (long)r * ns + j;
+      // the particles' grids (pressure gradients, indirect and self-gravity
+      // accelerations, src/SourceEuler.c:893-948) on the wavefront's own cells
+      const bool dgrid = X == SRC_DUST && store && r >= i0 && r < i1;
+      if (r >= 1) {
+        const double gradp = quotient<T>((p - s_p) * 2.0, sum_r, rr) * tr.idrm;
+        const double gradphi = (pot - s_pot) * tr.idrm;
+        double vt2;
+        if (frame) {
+          // CorrectVtheta (src/SideEuler.c:1133-1148) on the values read
+          const double ci = dom * tr.rmed, cim = dom * ts.rmed;
+          vt2 = (vt0 - ci) + (vtn0 - ci) + (s_vt0 - cim) + (s_vtn0 - cim);
+        } else {
+          vt2 = vt0 + vtn0 + s_vt0 + s_vtn0;
+        }
+        vt2 = vt2 / 4.0 + tr.rinf * Of;
+        vt2 = vt2 * vt2;
+        vr1 = (double)raw.vr + dt * (-gradp - gradphi + vt2 * tr.irinf);
+        if (X == SRC_DUST && a.d_feedback) vr1 += dt * (double)raw.x[0];
+        if (X == SRC_FRAME && DF_ON(T, a) && a.df_feedback) {
+          // the dust fluid's drag on the gas, implicit (src/SourceEuler.c:915-921)
+          const double st = (double)raw.x[0] * tr.r15, eps = div_nr((double)raw.x[1], rho);
+          vr1 = div_nr(vr1 * st + eps * (double)raw.x[2] * dt, st + dt * eps);
+        }
+        if (dgrid) {
+          st<T>(a.radgradp, l, (p - s_p) * tr.idrm);
+          if (a.indirect_term)
+            st<T>(a.radindacc, l, -(ip - s_ip) * tr.idrm);
+        }
+        if (a.sg) {
+          const double radsgacc = ((tr.rinf - ts.rmed) * sgr + (tr.rmed - tr.rinf) * s_sgr) * tr.idrm;
+          if (dgrid) st<T>(a.radsgacc, l, radsgacc);
+          vr1 = vr1 + dt * radsgacc;
+        }
+      }
+      const double gradp = quotient<T>((p - pljm) * 2.0, sum_t, rt) * tr.idxt;
+      const double gradphi = (pot - potjm) * tr.idxt;
+      vt1 = vt0;
+      if (frame) vt1 = vt1 - dom * tr.rmed;
+      vt1 = vt1 - dt * (gradp + gradphi);
+      vt1 += dt * tr.supp;
+      if (X == SRC_DUST && a.d_feedback) vt1 += dt * (double)raw.x[1];
+      if (X == SRC_FRAME && DF_ON(T, a) && a.df_feedback) {
+        // src/SourceEuler.c:991-997, with the dust's vtheta after CorrectVtheta
+        const double st = (double)raw.x[0] * tr.r15, eps = div_nr((double)raw.x[1], rho);
+        const double dvtl = frame ? (double)raw.x[3] - dom * tr.rmed : (double)raw.x[3];
+        vt1 = div_nr(vt1 * st + eps * dvtl * dt, st + dt * eps);
       }
       if (dgrid) {
-        st<T>(a.radgradp, l, (pl - plim) * idrm);
+        st<T>(a.azigradp, l, (p - pljm) * tr.idxt);
         if (a.indirect_term)
-          st<T>(a.radindacc, l, -(indpot_at(a, c, i, j) - indpot_at(a, c, i - 1, j)) * idrm);
+          st<T>(a.aziindacc, l, -(ip - ipjm) * tr.idxt);
       }
       if (a.sg) {
-        double radsgacc = ((STAB(ST_RINF, i) - STAB(ST_RMED, i - 1)) * (double)pf_sgr[it] +
-                           (STAB(ST_RMED, i) - STAB(ST_RINF, i)) * (double)pf_sgrm[it]) * idrm;
-        if (dgrid) st<T>(a.radsgacc, l, radsgacc);
-        vri = vri + dt * radsgacc;
+        const double azisgacc = 0.5 * ((double)raw.sgt + sgtjm);
+        if (dgrid) st<T>(a.azisgacc, l, azisgacc);
+        vt1 = vt1 + dt * azisgacc;
       }
     }
-    const double invdxtheta = STAB(ST_IDXT, i);
-    const double pljm = sP[q + 1][p];
-    double gradp = (pl - pljm) * 2.0 / (rl + (double)sRho[q + 1][p]) * invdxtheta;
-    double gradphi = (potl - sPot[q + 1][p]) * invdxtheta;
-    double vti = (double)sVth[q + 1][p + 1];
-    if (a.frame) vti = vti - dom * STAB(ST_RMED, i);
-    vti = vti - dt * (gradp + gradphi);
-    vti += dt * STAB(ST_SUPP, i);
-    if (a.d_on && a.d_feedback) vti += dt * ld<T>(a.azifbacc, l);
-    if (DF_ON(T, a) && a.df_feedback) {
-      // src/SourceEuler.c:991-997, with the dust's vtheta after CorrectVtheta
-      const double ts = a.dstokes[l] * a.r15[i], eps = a.drho[l] / rl;
-      const double dvtl = a.frame ? a.dvt[l] - dom * STAB(ST_RMED, i) : a.dvt[l];
-      vti = (vti * ts + eps * dvtl * dt) / (ts + dt * eps);
-    }
-    if (dgrid) {
-      st<T>(a.azigradp, l, (pl - pljm) * invdxtheta);
-      if (a.indirect_term)
-        st<T>(a.aziindacc, l, -(indpot_at(a, c, i, j) - indpot_at(a, c, i, sCol[p])) * invdxtheta);
-    }
-    if (a.sg) {
-      const double azisgacc = 0.5 * ((double)pf_sgt[it] + (double)pf_sgtm[it]);
-      if (dgrid) st<T>(a.azisgacc, l, azisgacc);
-      vti = vti + dt * azisgacc;
-    }
-    sVr[q][p] = vri;
-    sVt[q][p] = vti;
-  }
-  __syncthreads();
-  if (a.visc_on) {
-    // stage 2: stresses on rings i0-2 .. i0+SRC_TR (V slot = S slot + 1)
-    const double onethird = 1.0 / 3.0;
-    for (int idx = tid; idx < SRC_SR * SRC_SC; idx += TB) {
-      const int q = idx / SRC_SC, p = idx - q * SRC_SC, i = i0 - 2 + q, j = sCol[p + 2];
-      if (i < 0 || i > nr - 1) {
-        sTrr[q][p] = sTpp[q][p] = sTrp[q][p] = (T)0;
-        continue;
+    // the stresses of ring s, then VradInt of ring s and VthetaInt of ring t
+    double trr = 0.0, tpp = 0.0, trp = 0.0, vs = s_vr, vtt = t_vt;
+    if (a.visc_on) {
+      if (s >= 0 && s >= i0 - 2 && s < nr) {
+        const double vtnx = lane_next(s_vt);
+        double dv = (vr1 * ts.rsup - s_vr * ts.rinf) * ts.idrs * ts.irmed;
+        dv += (vtnx - s_vt) * invdphi * ts.irmed;
+        const double Drr = (vr1 - s_vr) * ts.idrs;
+        const double Dpp = (vtnx - s_vt) * invdphi * ts.irmed + 0.5 * (vr1 + s_vr) * ts.irmed;
+        trr = 2.0 * s_rho * ts.nu * (Drr - onethird * dv);
+        tpp = 2.0 * s_rho * ts.nu * (Dpp - onethird * dv);
+        if (s >= 1) {
+          const double Drp = 0.5 * (ts.rinf * (s_vt * ts.irmed - t_vt * tt.irmed) * ts.idrm +
+                                    (s_vr - lane_prev(s_vr)) * invdphi * ts.irinf);
+          trp = 2.0 * 0.25 * (s_rho + t_rho + s_rhojm + t_rhojm) * ts.nu * Drp;
+        }
       }
-      const double nu = STAB(ST_NU, i), irm = STAB(ST_IRMED, i), idrs = STAB(ST_IDRS, i);
-      const double vrl = (double)sVr[q + 1][p + 1], vrp = (double)sVr[q + 2][p + 1];
-      const double vtl = (double)sVt[q + 1][p + 1], vtp = (double)sVt[q + 1][p + 2];
-      double dv = (vrp * STAB(ST_RSUP, i) - vrl * STAB(ST_RINF, i)) * idrs * irm;
-      dv += (vtp - vtl) * a.invdphi * irm;
-      const double Drr = (vrp - vrl) * idrs;
-      const double Dpp = (vtp - vtl) * a.invdphi * irm + 0.5 * (vrp + vrl) * irm;
-      const double rho = (double)sRho[q + 2][p + 2];
-      sTrr[q][p] = (T)(2.0 * rho * nu * (Drr - onethird * dv));
-      sTpp[q][p] = (T)(2.0 * rho * nu * (Dpp - onethird * dv));
-      double Trp = 0.0;
-      if (i >= 1) {
-        const double Drp = 0.5 * (STAB(ST_RINF, i) * (vtl * irm - (double)sVt[q][p + 1] * STAB(ST_IRMED, i - 1)) *
-                                      STAB(ST_IDRM, i) +
-                                  (vrl - (double)sVr[q + 1][p]) * a.invdphi * STAB(ST_IRINF, i));
-        Trp = 2.0 * 0.25 *
-              (rho + (double)sRho[q + 1][p + 2] + (double)sRho[q + 2][p + 1] + (double)sRho[q + 1][p + 1]) * nu *
-              Drp;
+      if (s >= 1 && s >= i0 - 1 && s < nr) {
+        const double trpn = lane_next(trp);
+        const double num = dt * ts.irinf *
+                           ((ts.rmed * trr - tt.rmed * t_trr) * ts.idrm + (trpn - trp) * invdphi - 0.5 * (tpp + t_tpp));
+        vs += 2.0 * quotient<T>(num, s_rho + t_rho, s_rr);
       }
-      sTrp[q][p] = (T)Trp;
-    }
-    __syncthreads();
-    // stage 3: the viscous update in place, VthetaInt on rings i0 ..
-    // i0+SRC_TR-1 x columns j0-1 .. j0+SRC_TC, VradInt on rings i0-1 ..
-    // i0+SRC_TR x columns j0 .. j0+SRC_TC-1 (S slot = V slot - 1)
-    for (int idx = tid; idx < SRC_TR * (SRC_TC + 2); idx += TB) {
-      const int q = idx / (SRC_TC + 2), p = idx - q * (SRC_TC + 2), i = i0 + q;
-      const int qv = q + 3, pv = p + 2, qs = qv - 1, ps = pv - 1;
-      if (i >= 1 && i < nr - 1) {
-        const double rho = (double)sRho[qv + 1][pv + 1];
-        const double trpl = (double)sTrp[qs][ps], trpp = (double)sTrp[qs + 1][ps];
-        double v = (double)sVt[qv][pv];
-        v += dt * STAB(ST_IRMED, i) *
-             ((STAB(ST_RSUP, i) * trpp - STAB(ST_RINF, i) * trpl) * STAB(ST_IDRS, i) +
-              ((double)sTpp[qs][ps] - (double)sTpp[qs][ps - 1]) * a.invdphi + 0.5 * (trpl + trpp)) /
-             (0.5 * (rho + (double)sRho[qv + 1][pv]));
-        sVt[qv][pv] = v;
+      if (t >= 1 && t >= i0 && t < nr - 1) {
+        const double tppjm = lane_prev(t_tpp);
+        const double num = dt * tt.irmed *
+                           ((tt.rsup * trp - tt.rinf * t_trp) * tt.idrs + (t_tpp - tppjm) * invdphi + 0.5 * (t_trp + trp));
+        vtt += 2.0 * quotient<T>(num, t_rho + t_rhojm, t_rt);
       }
     }
-    for (int idx = tid; idx < (SRC_TR + 2) * SRC_TC; idx += TB) {
-      const int q = idx / SRC_TC, p = idx - q * SRC_TC, i = i0 - 1 + q;
-      const int qv = q + 2, pv = p + 3, qs = qv - 1, ps = pv - 1;
-      if (i >= 1 && i <= nr - 1) {
-        const double rho = (double)sRho[qv + 1][pv + 1];
-        double v = (double)sVr[qv][pv];
-        v += dt * STAB(ST_IRINF, i) *
-             ((STAB(ST_RMED, i) * (double)sTrr[qs][ps] - STAB(ST_RMED, i - 1) * (double)sTrr[qs - 1][ps]) *
-                  STAB(ST_IDRM, i) +
-              ((double)sTrp[qs][ps + 1] - (double)sTrp[qs][ps]) * a.invdphi -
-              0.5 * ((double)sTpp[qs][ps] + (double)sTpp[qs - 1][ps])) /
-             (0.5 * (rho + (double)sRho[qv][pv + 1]));
-        sVr[qv][pv] = v;
+    // SubStep2 at ring t, and the wavefront's sum of the elongation rates
+    // vt dt / dt of the stored vtheta (ComputeThetaElongations and
+    // ComputeAverageThetaVelocities, src/TransportEuler.c:249-290), from which
+    // the transport forms the ring mean
+    double dv = vs - t_vr;
+    const double qr = (dv < 0.0) ? C2 * t_rho * dv * dv : 0.0;
+    if (t >= i0 && t < i1) {
+      const double dvt = lane_next(vtt) - vtt;
+      const double qt = (dvt < 0.0) ? C2 * t_rho * dvt * dvt : 0.0, qtm = lane_prev(qt);
+      const double step = dt * 2.0;
+      double rate = 0.0;
+      if (store) {
+        const long l = (long)t * ns + j;
+        const unsigned key = sizeof(T) == sizeof(float) ? sr_key(c, l, SR_VR) : 0u;
+        double vrn = 0.0;
+        if (t >= 1) vrn = t_vr - quotient<T>(step, t_rho + u_rho, t_rr) * (qr - u_qr) * tt.idrm;
+        const double vtn = vtt - quotient<T>(step, t_rho + t_rhojm, t_rt) * (qt - qtm) * tt.idxt;
+        ((T *)a.vri)[l] = sr_round<T>(vrn, sr_draw(key, 0));
+        const T vts = sr_round<T>(vtn, sr_draw(key, 1));
+        ((T *)a.vti)[l] = vts;
+        rate = ((double)vts * dt) * invdt;
+        if (E) {
+          const double e = t_en - dt * qr * dv * tt.idrs - dt * qt * dvt * tt.idxt;
+          ((T *)a.e_int)[l] = sr_round<T>(e, sr_draw(key, 2));
+        }
+        if (t == nr - 1) {
+          // vr and vt of ring nrad are zero after ActualiseGas
+          st<T>(a.vr, l + ns, 0.0);
+          st<T>(a.vt, l + ns, 0.0);
+        }
       }
+      rate = wave_sum(rate);
+      if (lane == 0) a.vt_part[(long)t * ntile + seg] = rate;
     }
-    __syncthreads();
-  }
-  // stage 4: SubStep2 on the tile (V slot = tile slot + 3).  Each
-  // wavefront holds one ring of the tile (SRC_TC = 64 columns) and leaves
-  // the tile's sum of the elongation rates vt dt / dt of the stored vtheta
-  // (ComputeThetaElongations and ComputeAverageThetaVelocities,
-  // src/TransportEuler.c:249-290), from which the azimuthal transport forms
-  // the ring mean.
-  const double C2 = DF_CVNR * DF_CVNR, invdt = 1.0 / dt;
-  const int ntile = (ns + SRC_TC - 1) / SRC_TC;
-  for (int b0 = 0; b0 < SRC_TR * SRC_TC; b0 += TB) {
-    const int idx = b0 + tid;
-    const int q = idx / SRC_TC, p = idx - q * SRC_TC, i = i0 + q, jt = j0 + p;
-    double rate = 0.0;
-    if (idx < SRC_TR * SRC_TC && i <= nr - 1 && jt < ns) {
-      const int qv = q + 3, pv = p + 3, j = sCol[pv + 1];
-      const long l = (long)i * ns + j;
-      const double rho = (double)sRho[qv + 1][pv + 1];
-      const double vrl = (double)sVr[qv][pv], vrp = (double)sVr[qv + 1][pv];
-      const double vtl = (double)sVt[qv][pv], vtp = (double)sVt[qv][pv + 1], vtm = (double)sVt[qv][pv - 1];
-      double dv = vrp - vrl;
-      const double qr = (dv < 0.0) ? C2 * rho * dv * dv : 0.0;
-      dv = vtp - vtl;
-      const double qt = (dv < 0.0) ? C2 * rho * dv * dv : 0.0;
-      const double rhojm = (double)sRho[qv + 1][pv];
-      dv = vtl - vtm;
-      const double qtm = (dv < 0.0) ? C2 * rhojm * dv * dv : 0.0;
-      double vrn = 0.0;
-      if (i >= 1) {
-        const double rhoim = (double)sRho[qv][pv + 1];
-        dv = vrl - (double)sVr[qv - 1][pv];
-        const double qrm = (dv < 0.0) ? C2 * rhoim * dv * dv : 0.0;
-        vrn = vrl - dt * 2.0 / (rho + rhoim) * (qr - qrm) * STAB(ST_IDRM, i);
-      }
-      const double invdxtheta = STAB(ST_IDXT, i);
-      st_sr<T>(a.vri, l, vrn, sr_key(c, l, SR_VR));
-      const T vts = sr_round<T>(vtl - dt * 2.0 / (rho + rhojm) * (qt - qtm) * invdxtheta, sr_key(c, l, SR_VT));
-      ((T *)a.vti)[l] = vts;
-      rate = ((double)vts * dt) * invdt;
-      if (a.energy) {
-        double e = ld<T>(a.en, l);
-        e = e - dt * qr * (vrp - vrl) * STAB(ST_IDRS, i) - dt * qt * (vtp - vtl) * invdxtheta;
-        st_sr<T>(a.e_int, l, e, sr_key(c, l, SR_E));
-      }
-      if (i == nr - 1) {
-        // vr and vt of ring nrad are zero after ActualiseGas
-        st<T>(a.vr, l + ns, 0.0);
-        st<T>(a.vt, l + ns, 0.0);
-      }
-    }
-    rate = wave_sum(rate);
-    if ((tid & 63) == 0 && idx < SRC_TR * SRC_TC && i <= nr - 1) a.vt_part[(long)i * ntile + blockIdx.x] = rate;
+    u_rho = t_rho; u_qr = qr;
+    t_rho = s_rho; t_rhojm = s_rhojm; t_rr = s_rr; t_rt = s_rt; t_vr = vs; t_vt = s_vt; t_en = s_en;
+    t_trr = trr; t_tpp = tpp; t_trp = trp;
+    tt = ts;
+    s_rho = rho; s_rhojm = rhojm; s_rr = rr; s_rt = rt; s_vr = vr1; s_vt = vt1; s_en = en;
+    s_p = p; s_pot = pot; s_ip = ip; s_vt0 = vt0; s_vtn0 = vtn0; s_sgr = sgr;
+    ts = tr;
   }
 }
-#undef STAB
+
+// Rings per strip of a walk of S + extra rings' time, for `columns` wavefronts a
+// ring and a kernel of which `occupancy` wavefronts share a SIMD.  On a small
+// grid a SIMD has at most one wavefront, which is alone with its own latency:
+// the shortest strips for which that holds, up to four rings (64x192 FP32
+// transport: 1 ring 10.5 us, 2 rings 12.0; 200x400 FP64: 2 rings, 800 wavefronts,
+// 14.4, 1 ring, 1600, 15.9).  On larger ones the shortest walk times rounds of
+// wavefronts, since a last round that is nearly empty costs as much as a full
+// one (1024x3072 FP32 transport: 19 rings, 2970 wavefronts on 3072 places, 97 us;
+// 16 rings, 3520, 105; 28 rings, two wavefronts a SIMD on average but not
+// evenly, 114).
+static int strip_rings(const KArgs &a, int columns, int occupancy, int extra, int most) {
+  const long simds = 4L * a.num_cu;
+  for (int S = 1; S <= 4; S++)
+    if ((long)columns * ((a.nr + S - 1) / S) <= simds) return S;
+  int best = 2;
+  long cost = -1;
+  for (int S = 2; S <= most; S++) {
+    const long t = ((long)columns * ((a.nr + S - 1) / S) + occupancy * simds - 1) / (occupancy * simds) * (S + extra);
+    if (cost < 0 || t < cost) {
+      cost = t;
+      best = S;
+    }
+  }
+  return best;
+}
+template <typename T> static void launch_source(const KArgs &a, hipStream_t s) {
+  const int nseg = (a.ns + AZ_OWN - 1) / AZ_OWN, per = 4, bx = (nseg + per - 1) / per;
+  // a strip of S rings walks S + 5, plus its start
+  const int x = a.d_on ? SRC_DUST : (a.frame || (DF_ON(T, a) && a.df_feedback)) ? SRC_FRAME : SRC_PLAIN;
+  const int S = strip_rings(a, nseg, src_occupancy(sizeof(T) == 8, a.energy, x), 7, SRC_STRIP_MAX);
+  const dim3 g(bx, (a.nr + S - 1) / S), b(per * AZ_LANES);
+#define SRC_LAUNCH(X)                                                                        \
+  if (a.energy) hipLaunchKernelGGL((k_source<T, true, X>), g, b, 0, s, a, S);                \
+  else hipLaunchKernelGGL((k_source<T, false, X>), g, b, 0, s, a, S)
+  if (x == SRC_DUST) {
+    SRC_LAUNCH(SRC_DUST);
+  } else if (x == SRC_FRAME) {
+    SRC_LAUNCH(SRC_FRAME);
+  } else {
+    SRC_LAUNCH(SRC_PLAIN);
+  }
+#undef SRC_LAUNCH
+}
 
 // Energy source terms, per ring: ComputeDivergenceVelocity
 // (src/SourceEuler.c:2373-2411), the stresses and ComputeViscousHeating
@@ -1611,7 +1670,7 @@ template <typename T, int K> __global__ void __launch_bounds__(RING_LB(K)) k_ene
 // face value and flux is formed once (tiles in LDS formed every radial face
 // twice and 10/8 of the slopes: 90 us for the radial pass alone).  A strip
 // repeats the Work of four rings and the slopes of two at its ends, a wavefront
-// eight of its 64 columns; transport_strip picks S.  FP64 whatever the storage
+// eight of its 64 columns; strip_rings picks S.  FP64 whatever the storage
 // type.
 //
 // The ring quantities of the FARGO scheme come first, from the per-tile sums
@@ -1620,41 +1679,6 @@ template <typename T, int K> __global__ void __launch_bounds__(RING_LB(K)) k_ene
 // residual (ComputeConstantResidual, src/TransportEuler.c:292-348), two lanes
 // per ring of the strip.  Every wavefront of a ring forms them from the same
 // sums in the same order, so all agree on the shift.
-
-// The cells a wavefront owns: its 64 lanes hold 64 consecutive cells of a
-// ring, and each of the two passes leaves two fewer valid cells at either
-// end (a cell's update reads its neighbours up to two cells away), so the
-// middle 56 are complete after both.
-#define AZ_LANES 64
-#define AZ_HALO 4
-#define AZ_OWN (AZ_LANES - 2 * AZ_HALO)
-
-// The neighbouring lanes' values: lane L receives lane L - 1's (prev) or
-// lane L + 1's (next); the end lanes receive zeros, which only feed cells
-// outside the valid range.  CDNA's whole-wavefront DPP shifts (wave_shr:1,
-// wave_shl:1) move each 32-bit half in one VALU operation, without the LDS
-// crossbar of a general lane permute; with zeros for the end lanes the move
-// needs no copy of its destination first.
-template <int CTRL> __device__ __forceinline__ double dpp_shift(double v) {
-  return __hiloint2double(__builtin_amdgcn_update_dpp(0, __double2hiint(v), CTRL, 0xf, 0xf, true),
-                          __builtin_amdgcn_update_dpp(0, __double2loint(v), CTRL, 0xf, 0xf, true));
-}
-#define DPP_WAVE_SHL1 0x130
-#define DPP_WAVE_SHR1 0x138
-__device__ __forceinline__ double lane_prev(double v) { return dpp_shift<DPP_WAVE_SHR1>(v); }
-__device__ __forceinline__ double lane_next(double v) { return dpp_shift<DPP_WAVE_SHL1>(v); }
-
-// The operations' order.  With FP64 storage the transport keeps the
-// reference's products and sums one by one (over thousands of sub-steps of a
-// nearly steady flow another order of them drifts from it by more than 1e-12);
-// with FP32 storage, whose rounding is 2^29 times as large, products shared by
-// the quantities are formed once and accumulated by fused multiply-adds, a
-// fifth fewer instructions.
-template <typename T> constexpr bool kExactOrder = sizeof(T) == sizeof(double);
-template <typename T> __device__ __forceinline__ double mul_add(double a, double b, double c) {
-  if constexpr (kExactOrder<T>) return a * b + c;
-  else return fma(a, b, c);
-}
 
 // What an azimuthal pass shares over its quantities, for the velocity v of this
 // lane's face (between the previous cell and this one): the upwind side, and
@@ -1730,11 +1754,6 @@ __device__ __forceinline__ RadRaw<T> rad_load(const KArgs &a, int r, int j, int 
   q.vr_out = ((const T *)a.vri)[l + a.ns + j];
   q.en = E ? ((const T *)a.en)[l + j] : (T)0;
   return q;
-}
-// lane k's value (k uniform); only where every lane is active
-__device__ __forceinline__ double lane_value(double v, int k) {
-  return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), k),
-                          __builtin_amdgcn_readlane(__double2loint(v), k));
 }
 // v plus the value of the other lane of its pair (quad_perm 1,0,3,2)
 __device__ __forceinline__ double pair_sum(double v) {
@@ -1925,28 +1944,12 @@ template <typename T, bool E> __global__ void __launch_bounds__(256, tr_occupanc
   }
 }
 
-// Rings per strip of the transport.  A strip of S rings walks S + 4, plus its
-// start (about two rings' time), and a last round of wavefronts that is nearly
-// empty costs as much as a full one: the S with the shortest walk times rounds.
-// 1024x3072 FP32: 19 rings (3024 wavefronts on 3072 places) 97 us, 16 rings
-// (3584) 105 us, 8 rings (7168) 99 us; a small grid takes 2.
-static int transport_strip(const KArgs &a, int per) {
-  const long nseg = ((a.ns + AZ_OWN - 1) / AZ_OWN + per - 1) / per * per, places = 4L * tr_occupancy(a.energy) * a.num_cu;
-  int best = 2;
-  long cost = -1;
-  for (int S = 2; S <= TR_STRIP_MAX; S++) {
-    const long t = (nseg * ((a.nr + S - 1) / S) + places - 1) / places * (S + 6);
-    if (cost < 0 || t < cost) {
-      cost = t;
-      best = S;
-    }
-  }
-  return best;
-}
 template <typename T> static void launch_transport(const KArgs &a, hipStream_t s) {
   const int per = (a.tune_azi_waves == 1 || a.tune_azi_waves == 2) ? a.tune_azi_waves : 4;
-  const int S = transport_strip(a, per), nseg = (a.ns + AZ_OWN - 1) / AZ_OWN;
-  const dim3 g((nseg + per - 1) / per, (a.nr + S - 1) / S), b(per * AZ_LANES);
+  const int nseg = (a.ns + AZ_OWN - 1) / AZ_OWN, bx = (nseg + per - 1) / per;
+  // a strip of S rings walks S + 4, plus its start
+  const int S = strip_rings(a, nseg, tr_occupancy(a.energy), 6, TR_STRIP_MAX);
+  const dim3 g(bx, (a.nr + S - 1) / S), b(per * AZ_LANES);
   if (a.energy) hipLaunchKernelGGL((k_transport_azi<T, true>), g, b, 0, s, a, S);
   else hipLaunchKernelGGL((k_transport_azi<T, false>), g, b, 0, s, a, S);
 }
@@ -2495,6 +2498,14 @@ static int wide_k(int ns) {
     }                                                                                       \
   } while (0)
 
+template <typename T> __device__ __forceinline__ double src_press(const KArgs &a, long l, int i) {
+  if (!a.energy) {
+    const double cs = (double)(T)a.cs_iso[i];
+    return ld<T>(a.rho, l) * cs * cs;
+  }
+  return (a.gamma - 1.0) * ld<T>(a.en, l);
+}
+
 #include "dust_fluid.h"
 
 static dim3 cell_grid(const KArgs &a, int rings) {
@@ -2525,8 +2536,7 @@ template <typename T> void launch_kernel(int id, const KArgs &a, hipStream_t s) 
       hipLaunchKernelGGL(k_evanescent<T>, dim3(a.wkz_n_in + (a.nr - a.wkz_i_out)), dim3(EV_TB), 0, s, a);
       break;
     case KID_SOURCE:
-      hipLaunchKernelGGL(k_source<T>, dim3((a.ns + SRC_TC - 1) / SRC_TC, (a.nr + SRC_TR - 1) / SRC_TR), dim3(SrcBlock<T>::n), 0, s,
-                         a);
+      launch_source<T>(a, s);
       break;
     case KID_ENERGY: RING_DISPATCH(k_energy, T, a, s, 0); break;
     case KID_TRANSPORT_AZI: launch_transport<T>(a, s); break;
