@@ -61,21 +61,20 @@ def kernel_bytes_per_launch(name, w, energy, sg, cells, npart):
             "dust_move": 5 * 8 + 10 * 8 + 12 * 8 + 4 + 4,
             "dust_scan": 0,
             "dust_scatter": 4 + 4 + 4,             # cell, slot in; bucket entry out
-            "dust_sort": 0,
-            # bucket entry, r, th, cell, drag x2, four weights per stencil (+ t_s,
-            # |dv|^2 with the energy equation)
-            "dust_deposit": 8 + 4 + 4 + 16 + 8 * 8 + (16 if energy else 0),
-            # bucket entry in; seven FP64 fields and the id read and written
-            "dust_reorder": 8 + 2 * (7 * 8 + 4),
+            # cell, first nodes, bucket entry in, entry out; seven FP64 fields and
+            # the id read and written
+            "dust_rank": 4 + 4 + 8 + 8 + 2 * (7 * 8 + 4),
+            # bucket entry, drag x2, four weights per stencil (+ t_s, |dv|^2 with
+            # the energy equation)
+            "dust_deposit": 8 + 16 + 8 * 8 + (16 if energy else 0),
         }[name]
         per_cell = {
             "dust_move": 0,
             "dust_scan": 4 + 4,                    # counts in, ring-local starts out
             "dust_scatter": 4,                     # ring-local start of the particle's cell
-            "dust_sort": 4 + 4 + 4,                # local start, count in; start out
+            "dust_rank": 4 + 4,                    # local start, count in
             # starts, counts, rho in; two feedback grids (+ FBedot) out
             "dust_deposit": 8 + w + 2 * w + (w if energy else 0),
-            "dust_reorder": 0,
         }[name]
         return per_particle * npart + per_cell * cells
     return kernel_bytes_per_cell(name, w, energy, sg) * cells

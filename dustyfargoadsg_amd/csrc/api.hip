@@ -365,8 +365,7 @@ static void build_sequence(dfargo_ctx *c) {
   if (c->a.df_on) c->seq.push_back(KID_DF_CFL);
   c->seq.push_back(KID_CONTROL);
   if (c->dust_on)
-    for (int id : {KID_DUST_MOVE, KID_DUST_SCAN, KID_DUST_SCATTER, KID_DUST_SORT, KID_DUST_DEPOSIT,
-                   KID_DUST_REORDER})
+    for (int id : {KID_DUST_MOVE, KID_DUST_SCAN, KID_DUST_SCATTER, KID_DUST_RANK, KID_DUST_DEPOSIT})
       c->seq.push_back(id);
   const bool df = c->a.df_on != 0;
   // the dust fluid's source step starts from the state the sub-step starts
@@ -1518,14 +1517,16 @@ extern "C" int dfargo_attach_dust(dfargo_ctx *c, const dfargo_dust_params *d, co
   double **pd[] = {&a.p_raddrag, &a.p_azidrag, &a.p_ts, &a.p_dv2};
   for (double **q : pd)
     if ((rc = dalloc(c, (void **)q, sizeof(double) * np))) return rc;
-  if ((rc = dalloc(c, (void **)&a.p_sorted, sizeof(unsigned long long) * np))) return rc;
+  if ((rc = dalloc(c, (void **)&a.p_sorted, sizeof(unsigned long long) * np)) ||
+      (rc = dalloc(c, (void **)&a.p_entry, sizeof(unsigned long long) * np)))
+    return rc;
   if ((rc = dalloc(c, (void **)&a.p_w, sizeof(double) * 18 * np)) ||
       (rc = dalloc(c, (void **)&a.p_tsmin, sizeof(unsigned long long) * ((np + 255) / 256))))
     return rc;
-  int **pi[] = {&a.p_cell, &a.p_slot, &a.p_base, &a.out_list};
+  int **pi[] = {&a.p_cell, &a.p_slot, &a.p_base};
   for (int **q : pi)
     if ((rc = dalloc(c, (void **)q, sizeof(int) * np))) return rc;
-  int **ci[] = {&a.cell_count, &a.cell_local, &a.cell_start};
+  int **ci[] = {&a.cell_count, &a.cell_local};
   for (int **q : ci)
     if ((rc = dalloc(c, (void **)q, sizeof(int) * ncell))) return rc;
   if ((rc = dalloc(c, (void **)&a.ring_tot, sizeof(int) * (size_t)(nr + 1))) ||

@@ -96,12 +96,12 @@ struct KArgs {
   // per particle the separable stencil weights of its three stencils:
   // p_w[(kind * 6 + q) * np + k], q < 3 radial, 3 + q azimuthal
   double *p_w;
-  // buckets: particle cell and slot in it, per-cell counts and starts
-  // (ring-local, then global), per-ring totals and offsets (ring_off[nr]:
-  // the particles inside the grid); bucket entries are (id << 32 | position)
-  int *p_cell, *p_slot, *cell_count, *cell_local, *cell_start, *ring_tot, *ring_off;
-  unsigned long long *p_sorted;
-  int *out_list; // positions of the particles outside the grid
+  // buckets: particle cell and slot in it, per-cell counts and ring-local
+  // starts, per-ring totals and offsets (ring_off[nr]: the particles inside
+  // the grid); bucket entries are (id << 32 | position), and ordered by id
+  // (first nodes of the stencils << 32 | position)
+  int *p_cell, *p_slot, *cell_count, *cell_local, *ring_tot, *ring_off;
+  unsigned long long *p_sorted, *p_entry;
   // first node of each stencil relative to the particle's cell, 2 + 2 bits
   // per stencil (ring, column; offset + 1)
   int *p_base;
@@ -144,7 +144,7 @@ struct KArgs {
 enum KernelId {
   KID_SG_ROWS_FWD = 0, KID_SG_COLS, KID_SG_ROWS_INV,
   KID_CFL, KID_CONTROL, KID_SOURCE, KID_ENERGY, KID_TRANSPORT_AZI,
-  KID_FINISH, KID_DUST_MOVE, KID_DUST_SCAN, KID_DUST_SCATTER, KID_DUST_SORT, KID_DUST_DEPOSIT, KID_DUST_REORDER,
+  KID_FINISH, KID_DUST_MOVE, KID_DUST_SCAN, KID_DUST_SCATTER, KID_DUST_RANK, KID_DUST_DEPOSIT,
   KID_EVANESCENT, KID_NONREFLECTING,
   KID_SGZ_MEAN, KID_SGZ_CONV, KID_SGZ_FILL, KID_EOS_STEP, KID_VISC1D,
   KID_DF_CFL, KID_DF_AXISG, KID_DF_SOURCE, KID_DF_STRESS, KID_DF_VISC, KID_DF_SUBSTEP2,

@@ -17,7 +17,7 @@ const char *kKernelNames[KID_COUNT] = {
     "sg_rows_fwd", "sg_cols", "sg_rows_inv",
     "cfl_ring",    "control",        "source",  "energy",
     "transport_azi", "finish",      "dust_move",      "dust_scan",  "dust_scatter",
-    "dust_sort",     "dust_deposit", "dust_reorder", "evanescent", "nonreflecting",
+    "dust_rank",     "dust_deposit", "evanescent", "nonreflecting",
     "sgz_mean",      "sgz_conv",     "sgz_fill",     "eos_step",      "visc1d",
     "df_cfl",        "df_axisg",      "df_source",    "df_stress",    "df_visc",       "df_substep2",
     "df_transport_azi", "df_finish"};
@@ -2548,9 +2548,8 @@ template <typename T> void launch_kernel(int id, const KArgs &a, hipStream_t s) 
     case KID_DUST_MOVE:
     case KID_DUST_SCAN:
     case KID_DUST_SCATTER:
-    case KID_DUST_SORT:
-    case KID_DUST_DEPOSIT:
-    case KID_DUST_REORDER: launch_dust_kernel<T>(id, a, s); break;
+    case KID_DUST_RANK:
+    case KID_DUST_DEPOSIT: launch_dust_kernel<T>(id, a, s); break;
     case KID_DF_CFL:
     case KID_DF_AXISG:
     case KID_DF_SOURCE:
