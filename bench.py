@@ -57,8 +57,8 @@ def kernel_bytes_per_launch(name, w, energy, sg, cells, npart):
     if name.startswith("dust_"):
         per_particle = {
             # r, th, vr, vth, size in; r, th, vr, vth, l, St, drag x2, t_s,
-            # |dv|^2, the CIC/TSC weights (12-18 doubles) out; cell and slot
-            "dust_move": 5 * 8 + 10 * 8 + 12 * 8 + 4 + 4,
+            # |dv|^2, the CIC/TSC weights (8-12 doubles) out; cell and slot
+            "dust_move": 5 * 8 + 10 * 8 + 8 * 8 + 4 + 4,
             "dust_scan": 0,
             "dust_scatter": 4 + 4 + 4,             # cell, slot in; bucket entry out
             # cell, first nodes, bucket entry in, entry out; seven FP64 fields and

@@ -1520,7 +1520,7 @@ extern "C" int dfargo_attach_dust(dfargo_ctx *c, const dfargo_dust_params *d, co
   if ((rc = dalloc(c, (void **)&a.p_sorted, sizeof(unsigned long long) * np)) ||
       (rc = dalloc(c, (void **)&a.p_entry, sizeof(unsigned long long) * np)))
     return rc;
-  if ((rc = dalloc(c, (void **)&a.p_w, sizeof(double) * 18 * np)) ||
+  if ((rc = dalloc(c, (void **)&a.p_w, sizeof(double) * 12 * np)) ||
       (rc = dalloc(c, (void **)&a.p_tsmin, sizeof(unsigned long long) * ((np + 255) / 256))))
     return rc;
   int **pi[] = {&a.p_cell, &a.p_slot, &a.p_base};

@@ -94,7 +94,7 @@ struct KArgs {
   // |dv|^2 for the heating
   double *p_raddrag, *p_azidrag, *p_ts, *p_dv2;
   // per particle the separable stencil weights of its three stencils:
-  // p_w[(kind * 6 + q) * np + k], q < 3 radial, 3 + q azimuthal
+  // p_w[(3 * set + q) * np + k], the sets as dust.hip numbers them
   double *p_w;
   // buckets: particle cell and slot in it, per-cell counts and ring-local
   // starts, per-ring totals and offsets (ring_off[nr]: the particles inside

@@ -1047,8 +1047,12 @@ __device__ void control_wave(const KArgs &a, dfargo_ctrl *c, const double *sums,
       // the particles of this sub-step feel the planets where the n-body
       // step left them (src/SourceEuler.c:504-513 come before RotatePsys)
       if (a.d_on) {
-        c->dust_pl_x[lane] = b.x;
-        c->dust_pl_y[lane] = b.y;
+        // distance, azimuth and smoothing length, once for all particles
+        const double rpl = sqrt(b.x * b.x + b.y * b.y);
+        c->dust_pl_r[lane] = rpl;
+        c->dust_pl_t[lane] = atan2(b.y, b.x);
+        c->dust_pl_eps[lane] = a.thickness_smoothing * a.aspect_ratio * pow(0.5 * rpl, 1.0 + a.flaring) *
+                               pow(2.0, 1.0 + a.flaring);
       }
       // RotatePsys (src/Psys.c:352-370)
       const double angle = omega_frame * dt;

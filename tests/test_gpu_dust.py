@@ -103,6 +103,19 @@ def test_startup_interpolation(interp):
     compare_grids(o, g, p, ("dust_density", "fb_accr", "fb_acct"), 1e-12)
 
 
+# the deposit's wavefronts of 60 columns and strips of 2 or 4 rings at their
+# remainders, buckets on both sides of the 24 particles from which a whole
+# wavefront sums one.  Sums of n <= 100 terms of like sign: n eps, far inside
+# the bar of the start-up interpolation.
+@pytest.mark.parametrize("interp", list(INTERPS))
+@pytest.mark.parametrize("nr,ns,nbpart", [(16, 8, 3000), (17, 59, 3000), (18, 60, 3000), (19, 61, 20000), (33, 122, 3000),
+                                          (515, 1920, 20000)])
+def test_deposit_edges(nr, ns, nbpart, interp):
+    p, d, o, g = setup(gas_planet, nr, ns, nbpart, interpolation=INTERPS[interp])
+    compare_particles(o, g, 0.0, 1e-12)
+    compare_grids(o, g, p, ("dust_density", "fb_accr", "fb_acct"), 1e-12)
+
+
 @pytest.mark.parametrize("interp", list(INTERPS))
 def test_dust_substeps_fp64(interp):
     """Two AlgoGas calls with particles feeling the disc, the planet and the

@@ -100,6 +100,19 @@ def test_ragged_rings_fp64(ns, energy):
         assert abs(getattr(go["planets"], k)[0] - getattr(oo["planets"], k)[0]) <= 1e-13, k
 
 
+# strips of more than one ring, the last of them shorter, on either side of
+# the size from which the wavefronts outnumber the SIMDs.  The file's bars.
+@pytest.mark.parametrize("nr", [41, 100])
+@pytest.mark.parametrize("energy", [0, 1])
+def test_strips_of_rings_fp64(nr, energy):
+    p, pl = gas_planet(nrad=nr, nsec=3072, energy_equation=energy, beta_cooling=energy)
+    o, so, d, sg = pair(p, pl)
+    n_o = o.algogas(DT / 20)
+    d.algogas(DT / 20)
+    assert d.status().last_call_substeps == n_o
+    compare(o, d, p, 1e-12, 1e-12, 1e-12)
+
+
 @pytest.mark.parametrize("nr,ns,calls", [(32, 96, 2), (64, 192, 1), (16, 1536, 1), (16, 3072, 1)])
 def test_energy_sg_fp64(nr, ns, calls):
     p, pl = energy_sg(nrad=nr, nsec=ns)
