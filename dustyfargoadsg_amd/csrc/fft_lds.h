@@ -1,7 +1,5 @@
 // fft_lds.h -- complex transforms in LDS (Stockham radix 8/4/3/2, one
-// workgroup per transform) shared by the self-gravity kernels (sg.hip) and
-// the end-of-sub-step kernel that forms the next sub-step's row spectra
-// (step.hip).
+// workgroup per transform) of the self-gravity kernels (sg.hip).
 #ifndef DFARGO_FFT_LDS_H
 #define DFARGO_FFT_LDS_H
 

@@ -10,7 +10,6 @@
 #include <hip/hip_runtime.h>
 #include <math.h>
 
-#include "fft_lds.h"
 #include "kernels.h"
 
 const char *kKernelNames[KID_COUNT] = {

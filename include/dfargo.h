@@ -432,7 +432,7 @@ int dfargo_read_planet_config(const char *path, const dfargo_params *p, dfargo_p
 /* ---- launch shapes and batched discs -------------------------------------- */
 
 /* Launch shapes of the sub-step kernels that do not change results: the
- * ring kernels' XCD-contiguous block order, the azimuthal transport's
+ * ring kernels' XCD-contiguous block order, the transport's
  * wavefronts per workgroup, the velocity/boundary kernel's workgroup
  * width, the LDS buffers of the self-gravity transforms and their rings
  * per workgroup.  No
