@@ -51,14 +51,13 @@ __device__ __forceinline__ unsigned mix32(unsigned x) {
   x ^= x >> 16;
   return x;
 }
-__device__ __forceinline__ unsigned sr_key(const dfargo_ctrl *c, long l, unsigned salt) {
-  return mix32((unsigned)l * 0x9E3779B9U ^ mix32((unsigned)c->substeps_total * 0x85EBCA6BU + salt));
+// (the part of the key that is the same in every cell, and a cell's key from it)
+__device__ __forceinline__ unsigned sr_field(const dfargo_ctrl *c, unsigned salt) {
+  return mix32((unsigned)c->substeps_total * 0x85EBCA6BU + salt);
 }
-// One hash of the cell serves the quantities a kernel stores there: each takes
-// it through a multiplication of its own (a 32-bit multiplication costs four
-// issue slots, the whole hash three of them).
-__device__ __forceinline__ unsigned sr_draw(unsigned cell_key, unsigned q) {
-  return (cell_key ^ (0x9E3779B9U * (2U * q + 1U))) * 0x2C1B3C6DU;
+__device__ __forceinline__ unsigned sr_cell(long l, unsigned field) { return mix32((unsigned)l * 0x9E3779B9U ^ field); }
+__device__ __forceinline__ unsigned sr_key(const dfargo_ctrl *c, long l, unsigned salt) {
+  return sr_cell(l, sr_field(c, salt));
 }
 template <typename T> __device__ __forceinline__ T sr_round(double v, unsigned key);
 template <> __device__ __forceinline__ double sr_round<double>(double v, unsigned) { return v; }
@@ -77,7 +76,7 @@ template <typename T> __device__ __forceinline__ void st_sr(void *p, long i, dou
   ((T *)p)[i] = sr_round<T>(v, key);
 }
 // salts of the stochastically rounded stores
-enum { SR_VR = 1, SR_VT, SR_E, SR_EN, SR_AZI = 16, SR_EVA = 24, SR_ACC = 32, SR_FIN = 40 };
+enum { SR_VR = 1, SR_VT, SR_E, SR_EN, SR_RAD = 8, SR_AZI = 16, SR_EVA = 24, SR_ACC = 32, SR_FIN = 40 };
 
 // a / b from the hardware reciprocal, two Newton steps and one correction of
 // the quotient: the compiler's IEEE sequence without its scaling of operands
@@ -1171,38 +1170,25 @@ template <int CTRL> __device__ __forceinline__ double dpp_shift(double v) {
 __device__ __forceinline__ double lane_prev(double v) { return dpp_shift<DPP_WAVE_SHR1>(v); }
 __device__ __forceinline__ double lane_next(double v) { return dpp_shift<DPP_WAVE_SHL1>(v); }
 
-// The operations' order.  With FP64 storage the source terms and the
-// transport keep the reference's products and sums one by one (over thousands of sub-steps of a
-// nearly steady flow another order of them drifts from it by more than 1e-12);
-// with FP32 storage, whose rounding is 2^29 times as large, products shared by
-// the quantities are formed once and accumulated by fused multiply-adds, a
-// fifth fewer instructions.
-template <typename T> constexpr bool kExactOrder = sizeof(T) == sizeof(double);
-template <typename T> __device__ __forceinline__ double mul_add(double a, double b, double c) {
-  if constexpr (kExactOrder<T>) return a * b + c;
-  else return fma(a, b, c);
-}
+// The operations' order is that of the reference, whatever the storage type.
+// Over thousands of sub-steps of a nearly steady flow another order of the
+// products and sums drifts from it by more than 1e-12; and particles that read
+// the nearest cell turn a single FP32 cell that rounds the other way into a
+// different run (a grain by an edge reads another cell, and its drag acts on
+// that one).  Three groups of operations are not the reference's own: a Work
+// value is Q times 1 / (rho + 1e-20), an elongation (vt dt) (1 / dt), an
+// azimuthal slope a product with 1 / dxtheta; and a division is div_nr.
 
-// 1 / b to within an ulp, and with it the quotients a / b of that divisor: div_nr's
-// steps, shared where several quotients have one divisor; with FP32 storage
-// the products
+// 1 / b to within an ulp, and with it the quotients a / b of that divisor:
+// div_nr's steps, shared where several quotients have one divisor
 __device__ __forceinline__ double rcp_nr(double b) {
   double r = __builtin_amdgcn_rcp(b);
   r = fma(r, fma(-b, r, 1.0), r);
   return fma(r, fma(-b, r, 1.0), r);
 }
-template <typename T> __device__ __forceinline__ double quotient(double a, double b, double r) {
+__device__ __forceinline__ double quotient(double a, double b, double r) {
   const double q = a * r;
-  if constexpr (!kExactOrder<T>) return q;
   return fma(r, fma(-b, q, a), q);
-}
-// m / sqrt(x) for the potential: square root and quotient, with FP32 storage
-// from the reciprocal square root
-template <typename T> __device__ __forceinline__ double over_sqrt(double m, double x) {
-  if constexpr (kExactOrder<T>) return div_nr(m, sqrt(x));
-  double y = __builtin_amdgcn_rsq(x);
-  y = fma(0.5 * y, fma(-x * y, y, 1.0), y);
-  return m * fma(0.5 * y, fma(-x * y, y, 1.0), y);
 }
 
 // lane k's value (k uniform); only where every lane is active
@@ -1227,8 +1213,8 @@ __device__ __forceinline__ double lane_value(double v, int k) {
 //
 // Bound by VALU issue.  As tiles in LDS with a halo per stage the potential
 // was formed 1.9 times a cell (8 rings, FP64) and every operand went through
-// LDS behind a barrier: 118 us at 1024x3072 FP64, 95 us FP32 with
-// self-gravity.  The quotients by the sums of neighbouring densities (six a
+// LDS behind a barrier: 121 us at 1024x3072 FP64, 98 us FP32 with
+// self-gravity; now 64 and 71 us.  The quotients by the sums of neighbouring densities (six a
 // cell) share two reciprocals.
 //
 // Rings at a strip's ends take only the stages that its own rings need.
@@ -1326,6 +1312,7 @@ __global__ void __launch_bounds__(256, src_occupancy(sizeof(T) == 8, E, X)) k_so
   const bool frame = X != SRC_PLAIN && a.frame;
   const double omega_prev = c->omega_prev, dom = frame ? c->domega : 0.0;
   const int ntile = (ns + DF_SRC_COLS - 1) / DF_SRC_COLS;
+  const unsigned f_vr = sr_field(c, SR_VR), f_vt = sr_field(c, SR_VT), f_e = sr_field(c, SR_E);
   const SrcTab zero_tab = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
   // ring s = r - 1: the state, its density to the left, the reciprocals of the
   // density sums across its inner and left face, VradInt, VthetaInt
@@ -1364,7 +1351,7 @@ __global__ void __launch_bounds__(256, src_occupancy(sizeof(T) == 8, E, X)) k_so
       for (int k = 0; k < npl; k++) {
         const double xp = lane_value(pX, k), yp = lane_value(pY, k), mp = lane_value(pM, k);
         const double distance = (x - xp) * (x - xp) + (y - yp) * (y - yp);
-        double pk = over_sqrt<T>(-DF_G * mp, distance + lane_value(pS, k));
+        double pk = div_nr(-DF_G * mp, sqrt(distance + lane_value(pS, k)));
         if (a.indirect_term) pk += DF_G * mp * lane_value(pI, k) * (x * xp + y * yp);
         pot += pk;
       }
@@ -1391,7 +1378,7 @@ __global__ void __launch_bounds__(256, src_occupancy(sizeof(T) == 8, E, X)) k_so
       // accelerations, src/SourceEuler.c:893-948) on the wavefront's own cells
       const bool dgrid = X == SRC_DUST && store && r >= i0 && r < i1;
       if (r >= 1) {
-        const double gradp = quotient<T>((p - s_p) * 2.0, sum_r, rr) * tr.idrm;
+        const double gradp = quotient((p - s_p) * 2.0, sum_r, rr) * tr.idrm;
         const double gradphi = (pot - s_pot) * tr.idrm;
         double vt2;
         if (frame) {
@@ -1421,7 +1408,7 @@ __global__ void __launch_bounds__(256, src_occupancy(sizeof(T) == 8, E, X)) k_so
           vr1 = vr1 + dt * radsgacc;
         }
       }
-      const double gradp = quotient<T>((p - pljm) * 2.0, sum_t, rt) * tr.idxt;
+      const double gradp = quotient((p - pljm) * 2.0, sum_t, rt) * tr.idxt;
       const double gradphi = (pot - potjm) * tr.idxt;
       vt1 = vt0;
       if (frame) vt1 = vt1 - dom * tr.rmed;
@@ -1454,25 +1441,27 @@ __global__ void __launch_bounds__(256, src_occupancy(sizeof(T) == 8, E, X)) k_so
         dv += (vtnx - s_vt) * invdphi * ts.irmed;
         const double Drr = (vr1 - s_vr) * ts.idrs;
         const double Dpp = (vtnx - s_vt) * invdphi * ts.irmed + 0.5 * (vr1 + s_vr) * ts.irmed;
-        trr = 2.0 * s_rho * ts.nu * (Drr - onethird * dv);
-        tpp = 2.0 * s_rho * ts.nu * (Dpp - onethird * dv);
+        // the stresses round to storage, as the grids of them that are read
+        // between sub-steps do
+        trr = (double)(T)(2.0 * s_rho * ts.nu * (Drr - onethird * dv));
+        tpp = (double)(T)(2.0 * s_rho * ts.nu * (Dpp - onethird * dv));
         if (s >= 1) {
           const double Drp = 0.5 * (ts.rinf * (s_vt * ts.irmed - t_vt * tt.irmed) * ts.idrm +
                                     (s_vr - lane_prev(s_vr)) * invdphi * ts.irinf);
-          trp = 2.0 * 0.25 * (s_rho + t_rho + s_rhojm + t_rhojm) * ts.nu * Drp;
+          trp = (double)(T)(2.0 * 0.25 * (s_rho + t_rho + s_rhojm + t_rhojm) * ts.nu * Drp);
         }
       }
       if (s >= 1 && s >= i0 - 1 && s < nr) {
         const double trpn = lane_next(trp);
         const double num = dt * ts.irinf *
                            ((ts.rmed * trr - tt.rmed * t_trr) * ts.idrm + (trpn - trp) * invdphi - 0.5 * (tpp + t_tpp));
-        vs += 2.0 * quotient<T>(num, s_rho + t_rho, s_rr);
+        vs += 2.0 * quotient(num, s_rho + t_rho, s_rr);
       }
       if (t >= 1 && t >= i0 && t < nr - 1) {
         const double tppjm = lane_prev(t_tpp);
         const double num = dt * tt.irmed *
                            ((tt.rsup * trp - tt.rinf * t_trp) * tt.idrs + (t_tpp - tppjm) * invdphi + 0.5 * (t_trp + trp));
-        vtt += 2.0 * quotient<T>(num, t_rho + t_rhojm, t_rt);
+        vtt += 2.0 * quotient(num, t_rho + t_rhojm, t_rt);
       }
     }
     // SubStep2 at ring t, and the wavefront's sum of the elongation rates
@@ -1488,17 +1477,16 @@ __global__ void __launch_bounds__(256, src_occupancy(sizeof(T) == 8, E, X)) k_so
       double rate = 0.0;
       if (store) {
         const long l = (long)t * ns + j;
-        const unsigned key = sizeof(T) == sizeof(float) ? sr_key(c, l, SR_VR) : 0u;
         double vrn = 0.0;
-        if (t >= 1) vrn = t_vr - quotient<T>(step, t_rho + u_rho, t_rr) * (qr - u_qr) * tt.idrm;
-        const double vtn = vtt - quotient<T>(step, t_rho + t_rhojm, t_rt) * (qt - qtm) * tt.idxt;
-        ((T *)a.vri)[l] = sr_round<T>(vrn, sr_draw(key, 0));
-        const T vts = sr_round<T>(vtn, sr_draw(key, 1));
+        if (t >= 1) vrn = t_vr - quotient(step, t_rho + u_rho, t_rr) * (qr - u_qr) * tt.idrm;
+        const double vtn = vtt - quotient(step, t_rho + t_rhojm, t_rt) * (qt - qtm) * tt.idxt;
+        ((T *)a.vri)[l] = sr_round<T>(vrn, sr_cell(l, f_vr));
+        const T vts = sr_round<T>(vtn, sr_cell(l, f_vt));
         ((T *)a.vti)[l] = vts;
         rate = ((double)vts * dt) * invdt;
         if (E) {
           const double e = t_en - dt * qr * dv * tt.idrs - dt * qt * dvt * tt.idxt;
-          ((T *)a.e_int)[l] = sr_round<T>(e, sr_draw(key, 2));
+          ((T *)a.e_int)[l] = sr_round<T>(e, sr_cell(l, f_e));
         }
         if (t == nr - 1) {
           // vr and vt of ring nrad are zero after ActualiseGas
@@ -1663,12 +1651,14 @@ template <typename T, int K> __global__ void __launch_bounds__(RING_LB(K)) k_ene
 // pass completes the ring before, which then takes the residual and the uniform
 // azimuthal pass and the integer shift while it is still in registers.
 //
-// Radial and azimuthal pass as kernels of their own each were at the memory's
-// rate with FP64 storage (1024x3072: 86 and 72 us; five quantities written by
-// one and read by the other, 250 MB) and bound by VALU issue with FP32 storage
-// (55 and 70 us).  Together they take 104 and 97 us, bound by VALU issue: they
-// read the state and write the transported quantities once, and a value rounds
-// to storage once.  What is counted beyond
+// Radial and azimuthal pass as kernels of their own took 87 + 76 us at 1024x3072
+// with FP64 storage (five quantities written by one and read by the other, 250
+// MB) and 78 + 75 us with FP32 storage.  Together they take 104 and 113 us: they
+// read the state and write the transported quantities once.  With FP32 storage
+// the radially transported quantities still round to it between the passes,
+// each by its own draw, as where a grid held them (97 us without that rounding
+// and with products shared across the quantities, but other values: see the
+// operations' order above).  What is counted beyond
 // that is instructions: each Work value Q / (rho + 1e-20), difference, slope,
 // face value and flux is formed once (tiles in LDS formed every radial face
 // twice and 10/8 of the slopes: 90 us for the radial pass alone).  A strip
@@ -1696,24 +1686,19 @@ struct AziFace {
 struct AziRing {
   double dx, invdx, dxrad, invsurf;
 };
-template <typename T> __device__ __forceinline__ AziFace azi_face(double v, double dt, const AziRing &g) {
+__device__ __forceinline__ AziFace azi_face(double v, double dt, const AziRing &g) {
   const double ksi = v * dt;
-  if constexpr (kExactOrder<T>) return {ksi > 0.0, -(g.dx + ksi), lane_next(g.dx - ksi)};
-  // the slope's 1 / dxtheta goes into the weights
-  const double x = ksi * g.invdx;
-  return {ksi > 0.0, -(1.0 + x), lane_next(1.0 - x)};
+  return {ksi > 0.0, -(g.dx + ksi), lane_next(g.dx - ksi)};
 }
 // the value at this lane's face for the cell values x; one difference per
 // face (a cell's second one is its neighbour's)
-template <typename T> __device__ __forceinline__ double azi_star_lane(double x, const AziFace &f, const AziRing &g) {
+__device__ __forceinline__ double azi_star_lane(double x, const AziFace &f, const AziRing &g) {
   const double dqp = lane_next(x) - x, dqm = lane_prev(dqp);
   // the quotient is formed on every lane and selected (where it is not used
   // it may be a NaN of a zero sum, which the select discards)
   const double prod = dqp * dqm;
-  double d = div_nr(prod, dqp + dqm);
-  if constexpr (kExactOrder<T>) d *= g.invdx;
-  const double dq = prod > 0.0 ? d : 0.0;
-  const double left = lane_prev(mul_add<T>(f.wr, dq, x)), right = mul_add<T>(f.wl, dq, x);
+  const double d = div_nr(prod, dqp + dqm) * g.invdx, dq = prod > 0.0 ? d : 0.0;
+  const double left = lane_prev(x + f.wr * dq), right = x + f.wl * dq;
   return f.up ? left : right;
 }
 
@@ -1724,22 +1709,17 @@ template <typename T> __device__ __forceinline__ double azi_star_lane(double x, 
 template <typename T, bool E>
 __device__ __forceinline__ void azi_pass_lane(const KArgs &a, double (&Q)[6], double v, double dt, const AziRing &g) {
   const double RI = Q[5];
-  const AziFace f = azi_face<T>(v, dt, g);
-  const double rs = azi_star_lane<T>(RI, f, g), rsv = rs * v * (g.dxrad * g.invsurf);
+  const AziFace f = azi_face(v, dt, g);
+  const double rs = azi_star_lane(RI, f, g);
   // the Work values Q / (rho + 1e-20) share one reciprocal
   const double inv = div_nr(1.0, RI + 1e-20);
 #pragma unroll
   for (int q = 0; q < 6; q++) {
     if (q == 4 && !E) continue;
     if (q < 4 && DF_ON(T, a) && a.tr_skip_mom) continue;
-    const double star = azi_star_lane<T>(Q[q] * inv, f, g);
-    if constexpr (kExactOrder<T>) {
-      const double flux = g.dxrad * star * rs * v;
-      Q[q] += (flux - lane_next(flux)) * g.invsurf;
-    } else {
-      const double flux = star * rsv;
-      Q[q] += flux - lane_next(flux);
-    }
+    const double star = azi_star_lane(Q[q] * inv, f, g);
+    const double flux = g.dxrad * star * rs * v;
+    Q[q] += (flux - lane_next(flux)) * g.invsurf;
   }
 }
 
@@ -1839,6 +1819,12 @@ template <typename T, bool E> __global__ void __launch_bounds__(256, tr_occupanc
   const int own = lane - AZ_HALO;
   const bool store = own >= 0 && own < AZ_OWN && seg * AZ_OWN + own < ns;
   void *zp[6] = {a.z_rp, a.z_rm, a.z_tp, a.z_tm, a.z_en, a.z_rho};
+  unsigned f_rad[6], f_azi[6];
+#pragma unroll
+  for (int k = 0; k < 6; k++) {
+    f_rad[k] = sr_field(c, SR_RAD + k);
+    f_azi[k] = sr_field(c, SR_AZI + k);
+  }
   // Entering step r (the newest ring read is r, q = r - 1 the one before):
   // Qq, Wq, vtq: ring q; Qp, vtp: ring q - 1; diff: the scaled differences
   // across face q (between rings q - 1 and q); right: the values of ring q - 1
@@ -1887,22 +1873,24 @@ template <typename T, bool E> __global__ void __launch_bounds__(256, tr_occupanc
         // used it may be a NaN of a zero sum, which the select discards)
         const double prod = dp * dm, x = div_nr(2.0 * prod, dp + dm);
         const double slope = (inner && prod > 0.0) ? x : 0.0;
-        star[k] = v > 0.0 ? right[k] : mul_add<T>(wl, slope, Wq[k]);
-        right[k] = mul_add<T>(wr, slope, Wq[k]);
+        star[k] = v > 0.0 ? right[k] : Wq[k] + wl * slope;
+        right[k] = Wq[k] + wr * slope;
       }
       // VanLeerRadial (src/TransportEuler.c:205-217): the flux through face q,
       // then ring q - 1's update
-      const double f0 = (open && tr > 0) ? dt * dtheta * lane_value(tRinf, tr - 1) : 0.0, f0sv = f0 * star[6] * v;
+      const double f0 = (open && tr > 0) ? dt * dtheta * lane_value(tRinf, tr - 1) : 0.0;
       const int i = q - 1;
       const bool mine = i >= i0 && i < i1;
       const double invs = mine ? lane_value(tInvS, tr - 2) : 0.0;
 #pragma unroll
       for (int k = 0; k < 6; k++) {
         if (k == 4 && !E) continue;
-        const double f = kExactOrder<T> ? f0 * star[k] * star[6] * v : f0sv * star[k], varq = flux[k] - f;
+        const double f = f0 * star[k] * star[6] * v, varq = flux[k] - f;
         flux[k] = f;
-        if (!(k < 4 && skip_mom)) Qp[k] = mul_add<T>(varq, invs, Qp[k]);
+        if (!(k < 4 && skip_mom)) Qp[k] = Qp[k] + varq * invs;
         if (k == 5 && i == 0 && mine && store) a.lost_col[j] = varq;
+        // the radially transported quantities round to storage
+        if (!(k < 4 && skip_mom)) Qp[k] = (double)sr_round<T>(Qp[k], sr_cell((long)i * ns + j, f_rad[k]));
       }
       if (mine) {
         // the residual velocity of the cell (src/TransportEuler.c:280-290),
@@ -1924,11 +1912,10 @@ template <typename T, bool E> __global__ void __launch_bounds__(256, tr_occupanc
           int jn = j + shift;
           if (jn >= ns) jn -= ns;
           const long l = (long)i * ns + jn;
-          const unsigned key = sr_key(c, l, SR_AZI);
 #pragma unroll
           for (int k = 0; k < 6; k++) {
             if (k == 4 && !E) continue;
-            ((T *)zp[k])[l] = sr_round<T>(Qp[k], sr_draw(key, k));
+            ((T *)zp[k])[l] = sr_round<T>(Qp[k], sr_cell(l, f_azi[k]));
           }
         }
       }
