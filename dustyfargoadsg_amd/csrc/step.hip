@@ -455,8 +455,11 @@ template <typename T, int K> __global__ void __launch_bounds__(RING_LB(K)) k_cfl
   double vsum = 0.0;
   for (int w = 0; w < nw; w++) vsum += sh[w * M];
   const double vmoy = vsum / (double)ns;
+  // The threads past the ring take no part in the minimum: beyond six cells a
+  // thread cs is read here, and the thread that owns a cell replaces it below
+  // with no barrier between, so each thread may only read its own cells.
   double dtmin = 1e30;
-  if (i >= 1) {
+  if (i >= 1 && on) {
     const double viscosity = a.nu_ring[i];
     const double dxrad = a.Rsup[i] - a.Rinf[i];
     const double dxtheta = a.Rmed[i] * a.pm / (double)ns;
@@ -499,7 +502,6 @@ template <typename T, int K> __global__ void __launch_bounds__(RING_LB(K)) k_cfl
                        invdt6 * invdt6;
       smax = (S > smax) ? S : smax;
     }
-    // threads past the ring repeat its first cell, which changes no minimum
     dtmin = DF_CFLSECURITY / sqrt(smax);
   }
   dtmin = wave_min(dtmin);

@@ -100,6 +100,36 @@ def test_ragged_rings_fp64(ns, energy):
         assert abs(getattr(go["planets"], k)[0] - getattr(oo["planets"], k)[0]) <= 1e-13, k
 
 
+# Rings of 8, 12 and 16 cells a thread whose threads are no whole number of
+# wavefronts, with the energy equation: there the CFL kernel reads the previous
+# sound speed after its reduction and replaces it, each thread in its own cells
+# alone.  Hot columns pass through column 0, the cell of which a thread past the
+# ring would take the sound speed from either side of the replacement.  Twice,
+# bit for bit, and the time steps, their number and the fields against the
+# oracle with the file's bars.
+@pytest.mark.parametrize("ns", [2056, 2080, 3200, 4104, 6176])
+def test_ragged_wide_rings_fp64(ns):
+    p, pl = gas_planet(nrad=8, nsec=ns, rmin=0.9, rmax=1.1, energy_equation=1, beta_cooling=1)
+    o, so, d, sg = pair(p, pl)
+    for st in (so, sg):
+        e, vt = st["energy"].reshape(-1, ns), st["vt"].reshape(-1, ns)
+        e[:, -8:] *= np.linspace(1.5, 4.0, 8)
+        vt[:, -4:] += 0.01
+    o.set_state(so)
+    got = []
+    for _ in range(2):
+        d.set_state(sg)
+        d.algogas(DT / 10)
+        st = d.state()
+        got.append((d.status().last_call_substeps, d.status().mindt, st["rho"], st["vr"], st["vt"], st["energy"]))
+    n_o = o.algogas(DT / 10)
+    assert got[0][0] == got[1][0] == n_o and n_o >= 3
+    for a, b in zip(got[0][1:], got[1][1:]):
+        assert np.array_equal(a, b)
+    assert abs(got[0][1] - o.status().mindt) <= 1e-12 * o.status().mindt
+    compare(o, d, p, 1e-12, 1e-12, 1e-12)
+
+
 # strips of more than one ring, the last of them shorter, on either side of
 # the size from which the wavefronts outnumber the SIMDs.  The file's bars.
 @pytest.mark.parametrize("nr", [41, 100])
