@@ -32,9 +32,9 @@
 // Sub-steps per launched graph.  The kernels of one graph follow each other
 // without a gap, two graphs on a stream lie 8 us apart (measured between the
 // last kernel of a sub-step and the first of the next, 200x400 and 1024x3072):
-// a sub-step of the smaller discs takes 40-80 us, so a call's sub-steps are
-// launched in runs.  Longer runs are instantiated when a call first needs one.
-static constexpr int kRunLength[3] = {1, 4, 16};
+// a sub-step of the smaller discs takes 30-60 us, so a call's sub-steps are
+// launched in runs, the longer ones once they pay (dfargo_run_level).
+static constexpr int kRunLength[DF_RUN_LEVELS] = DF_RUN_LENGTHS;
 
 struct dfargo_ctx {
   dfargo_params p;
@@ -48,7 +48,8 @@ struct dfargo_ctx {
   std::vector<int> seq; // kernel ids of one sub-step
   // the sub-step as a graph, and executables of runs of kRunLength[k] of it
   hipGraph_t graph = nullptr;
-  hipGraphExec_t gexec[3] = {nullptr, nullptr, nullptr};
+  hipGraphExec_t gexec[DF_RUN_LEVELS] = {};
+  long taken = 0; // sub-steps launched since the graphs were last dropped
   // sub-steps and length of the last AlgoGas call: how many to enqueue before
   // the next call first reads the control block back
   double last_DT = 0.0;
@@ -176,6 +177,7 @@ static int drop_graph(dfargo_ctx *c) {
     HIPCHK(hipGraphDestroy(c->graph));
     c->graph = nullptr;
   }
+  c->taken = 0;
   c->graph_version++;
   return DFARGO_OK;
 }
@@ -266,14 +268,14 @@ static int profiled_substep(dfargo_ctx *c) {
   return DFARGO_OK;
 }
 
-// the longest run of at most n sub-steps, launched; returns how many in *done
+// a run of at most n sub-steps, launched; returns how many in *done
 static int launch_run(dfargo_ctx *c, int n, int *done) {
-  int level = 2;
-  while (level > 0 && kRunLength[level] > n) level--;
+  const int level = dfargo_run_level((int)c->seq.size(), c->taken, n);
   int rc = ensure_graph(c, level);
   if (rc) return rc;
   HIPCHK(hipGraphLaunch(c->gexec[level], c->stream));
   *done = kRunLength[level];
+  c->taken += *done;
   return DFARGO_OK;
 }
 static int run_substeps(dfargo_ctx *c, int n) {

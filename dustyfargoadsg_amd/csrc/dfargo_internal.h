@@ -38,6 +38,12 @@ void dfargo_free_tables(dfargo_tables *t);
 double dfargo_sigma_profile(const dfargo_params *p, double r);
 double dfargo_energy_profile(const dfargo_params *p, double r);
 int dfargo_fft_length_ok(int n);
+/* Sub-steps per launched graph, and which of the lengths is launched next by a
+ * disc whose sub-step has `kernels` kernels, which has taken `taken` sub-steps
+ * since its sub-step was last captured and has `left` of them to enqueue. */
+#define DF_RUN_LEVELS 3
+#define DF_RUN_LENGTHS {1, 4, 16}
+int dfargo_run_level(int kernels, long taken, int left);
 int dfargo_set_error(int code, const char *fmt, ...);
 
 #ifdef __cplusplus

@@ -102,6 +102,24 @@ int dfargo_check_params(const dfargo_params *p) {
   return DFARGO_OK;
 }
 
+/* A longer run is captured inside the call that first launches it, so it must
+ * pay: a disc makes one once it has taken as many sub-steps without it as win
+ * its cost back.  Two graphs on a stream lie 8 us apart, so runs of 4 save 6 us
+ * a sub-step, runs of 16 a further 1.5 us.  Capture, instantiation and first
+ * launch cost, for runs of 4 and 16: 100 and 320 us at 64x192 (5 kernels), 400
+ * and 630 us at 512x1536 with the energy equation and self-gravity (9 kernels,
+ * two branches), 230 and 480 us with particles (10 kernels): won back after 17,
+ * 66, 38 and 210, 420, 320 sub-steps.  A disc that stops at any point has spent
+ * at most twice the gaps of single sub-steps on both together.  Made in the
+ * first call that could use it, a run of 16 cost 20 sub-steps at 512x1536 0.019
+ * ms each (0.188 ms, now 0.168). */
+int dfargo_run_level(int kernels, long taken, int left) {
+  static const int length[DF_RUN_LEVELS] = DF_RUN_LENGTHS, after[DF_RUN_LEVELS] = {0, 6, 48};
+  int level = DF_RUN_LEVELS - 1;
+  while (level > 0 && (length[level] > left || taken < (long)after[level] * kernels)) level--;
+  return level;
+}
+
 int dfargo_fft_length_ok(int n) {
   if (n < 1 || n > 4096) return 0;
   while (n % 2 == 0) n /= 2;

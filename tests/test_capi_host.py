@@ -240,3 +240,27 @@ def test_orbital_elements_match_oracle(lib):
         assert np.array_equal(a, b) or np.allclose(a, b, rtol=0, atol=0, equal_nan=True)
     with pytest.raises(Exception):
         orbital_elements(1.0, 0.0, 0.0, 1.0, 0.0, lib=lib)
+
+
+@pytest.mark.parametrize("kernels,cost", [(5, (0, 100, 320)), (9, (0, 400, 630)), (10, (0, 230, 480))])
+@pytest.mark.parametrize("call", [1, 3, 5, 12, 20, 37])
+def test_runs_of_substeps_pay_for_themselves(lib, kernels, cost, call):
+    """However early a disc stops, launching its sub-steps in runs (with the
+    measured costs of making one, us, and 8 us between two graphs) takes no more
+    than twice what single sub-steps take in gaps, and nothing more before the
+    first 6 sub-steps per kernel; a long-lived disc with calls of 20 and more
+    sub-steps ends up on runs of 16.  Runs made in the first call that could use
+    one fail it."""
+    length, made, taken, spent, last = (1, 4, 16), {0}, 0, 0.0, 0
+    while taken < 5000:
+        left = call
+        while left > 0:
+            last = lib.dfargo_run_level(kernels, taken, left)
+            assert length[last] <= left
+            spent += 8.0 + (0.0 if last in made else cost[last])
+            made.add(last)
+            taken += length[last]
+            left -= length[last]
+            single = 8.0 * taken
+            assert spent <= (single if taken < 6 * kernels else 2.0 * single), (taken, spent)
+    assert max(made) == (2 if call >= 16 else 1 if call >= 4 else 0)
