@@ -438,9 +438,12 @@ __device__ DfCell df_cell(const KArgs &a, const dfargo_ctrl *c, int i, int j) {
 __global__ void __launch_bounds__(256) k_df_finish(KArgs a) {
   const dfargo_ctrl *c = a.ctrl;
   if (!c->active) return;
-  const int i = blockIdx.y, ns = a.ns, nr = a.nr;
+  const int i = (int)blockIdx.y - 1, ns = a.ns, nr = a.nr;
   const int j = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i == nr && blockIdx.x == 0 && threadIdx.x < 64) add_lost_mass(a, a.dlost_col, &a.ctrl->lost_massd);
+  if (i < 0) { // as in k_finish
+    if (blockIdx.x == 0 && threadIdx.x < 64) add_lost_mass(a, a.dlost_col, &a.ctrl->lost_massd);
+    return;
+  }
   if (j >= ns) return;
   const long l = (long)i * ns + j;
   if (i == nr) {
@@ -485,7 +488,7 @@ static void launch_df_kernel(int id, const KArgs &a, hipStream_t s) {
       break;
     }
     case KID_DF_TRANSPORT_AZI: launch_transport<double>(df_transport_args(a), s); break;
-    case KID_DF_FINISH: hipLaunchKernelGGL(k_df_finish, dim3(g.x, a.nr + 1), b, 0, s, a); break;
+    case KID_DF_FINISH: hipLaunchKernelGGL(k_df_finish, dim3(g.x, a.nr + 2), b, 0, s, a); break;
     default: break;
   }
 }

@@ -2002,10 +2002,8 @@ template <typename T> __device__ CellState vel_cell(const KArgs &a, const dfargo
 // every boundary type (src/SideEuler.c:1110-1112).  Each cell of the edge
 // rings takes the values the boundary routines would copy into it from the
 // rings they read (2, 3 and nrad-2), recomputed here from the momenta.
-// Stores cell (i, j) of rings 0 .. nrad-1 and returns its density as
-// stored.
-template <typename T> __device__ __forceinline__ double finish_cell(const KArgs &a, const dfargo_ctrl *c, int i,
-                                                                    int j) {
+// Stores cell (i, j) of rings 0 .. nrad-1.
+template <typename T> __device__ __forceinline__ void finish_cell(const KArgs &a, const dfargo_ctrl *c, int i, int j) {
   const int nr = a.nr;
   const long l = (long)i * a.ns + j;
   CellState s = vel_cell<T>(a, c, i, j);
@@ -2056,21 +2054,26 @@ template <typename T> __device__ __forceinline__ double finish_cell(const KArgs 
   st<T>(a.vr, l, s.vr);
   st<T>(a.vt, l, s.vt);
   if (a.energy) st<T>(a.en, l, s.e);
-  return (double)(T)s.rho;
 }
 // the wall's radial velocity at the outer face (ring nrad)
 template <typename T> __device__ __forceinline__ void finish_outer_face(const KArgs &a, const dfargo_ctrl *c, int j) {
   if (a.bc == DFARGO_BC_WALL) st<T>(a.vr, (long)a.nr * a.ns + j, -vel_cell<T>(a, c, a.nr - 2, j).vr);
 }
 
-// Rings 0 .. nrad, the last only for the wall's vr at the outer face.
+// One row of blocks for the mass through the inner edge, then rings 0 .. nrad,
+// the last only for the wall's vr at the outer face.  The mass comes first since
+// it is a chain of loads and lane sums: in the last ring's row that was the
+// launch's tail (512x1536 FP32 9.7 us, now 9.0; 1024x3072 20.8 and 19.9).
 template <typename T> __global__ void __launch_bounds__(256) k_finish(KArgs a) {
   const dfargo_ctrl *c = a.ctrl;
   if (!c->active) return;
   // the sub-step ends here: the next one's loop condition takes effect
   if (blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) a.ctrl->go = c->go_next;
-  const int i = blockIdx.y, ns = a.ns, nr = a.nr, j = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i == nr && blockIdx.x == 0 && threadIdx.x < 64) add_lost_mass(a, a.lost_col, &a.ctrl->lost_mass);
+  const int i = (int)blockIdx.y - 1, ns = a.ns, nr = a.nr, j = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < 0) {
+    if (blockIdx.x == 0 && threadIdx.x < 64) add_lost_mass(a, a.lost_col, &a.ctrl->lost_mass);
+    return;
+  }
   if (j >= ns) return;
   if (i == nr) {
     finish_outer_face<T>(a, c, j);
@@ -2534,7 +2537,7 @@ template <typename T> void launch_kernel(int id, const KArgs &a, hipStream_t s) 
     case KID_TRANSPORT_AZI: launch_transport<T>(a, s); break;
     case KID_FINISH: {
       const int bx = finish_bx(a);
-      hipLaunchKernelGGL(k_finish<T>, dim3((a.ns + bx - 1) / bx, a.nr + 1), dim3(bx), 0, s, a);
+      hipLaunchKernelGGL(k_finish<T>, dim3((a.ns + bx - 1) / bx, a.nr + 2), dim3(bx), 0, s, a);
       break;
     }
     case KID_DUST_MOVE:
