@@ -116,6 +116,44 @@ def test_deposit_edges(nr, ns, nbpart, interp):
     compare_grids(o, g, p, ("dust_density", "fb_accr", "fb_acct"), 1e-12)
 
 
+# 150 to 400 particles a bucket: a wavefront passes over one several times, and a
+# particle's rank goes through many blocks of four.  At start-up sums of n <= 1600
+# terms of like sign, n eps < 1e-12; after a call the bars of the sub-steps.
+@pytest.mark.parametrize("interp", list(INTERPS))
+@pytest.mark.parametrize("energy", [0, 1])
+def test_crowded_buckets(interp, energy):
+    def disc(nrad, nsec):
+        return gas_planet(nrad=nrad, nsec=nsec, energy_equation=energy, beta_cooling=energy)
+    p, d, o, g = setup(disc, 16, 8, 20000, interpolation=INTERPS[interp])
+    compare_particles(o, g, 0.0, 1e-12)
+    compare_grids(o, g, p, ("dust_density", "fb_accr", "fb_acct"), 1e-12)
+    n_o = o.algogas(DT / 4)
+    g.algogas(DT / 4)
+    assert g.status().last_call_substeps == n_o
+    compare_particles(o, g, 1e-11, 1e-11)
+    compare_grids(o, g, p, ("dust_density", "fb_accr", "fb_acct") + (("fb_edot",) if energy else ()), 1e-10)
+
+
+# strips of two rings in the source and transport walks, the last of them shorter,
+# with particles and their feedback, in a frame that follows the planet
+@pytest.mark.parametrize("energy", [0, 1])
+def test_strips_of_rings_with_particles(energy):
+    def disc(nrad, nsec):
+        return gas_planet(nrad=nrad, nsec=nsec, energy_equation=energy, beta_cooling=energy, forced_circular=0,
+                          corotating=_capi.FRAME_COROTATING, omega_frame=math.sqrt(1 + 1e-3))
+    p, d, o, g = setup(disc, 41, 1536, 5000)
+    n_o = o.algogas(DT / 20)
+    g.algogas(DT / 20)
+    assert g.status().last_call_substeps == n_o
+    compare_particles(o, g, 1e-11, 1e-11)
+    go, oo = g.state(), o.state()
+    n = p.nrad * p.nsec
+    for k in ("rho", "vt") + (("energy",) if energy else ()):
+        assert relmax(go[k][:n], oo[k][:n]) <= 1e-11, k
+    assert np.abs(go["vr"][:n] - oo["vr"][:n]).max() <= 1e-11 * np.abs(oo["vt"][:n]).max()
+    compare_grids(o, g, p, ("dust_density", "fb_accr", "fb_acct"), 1e-10)
+
+
 @pytest.mark.parametrize("interp", list(INTERPS))
 def test_dust_substeps_fp64(interp):
     """Two AlgoGas calls with particles feeling the disc, the planet and the

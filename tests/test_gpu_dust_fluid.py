@@ -92,6 +92,21 @@ def test_feedback(sfta):
     run_pair(p, pl, fp)
 
 
+@pytest.mark.parametrize("frame", [0, 1])
+def test_feedback_strips_of_rings(frame):
+    """The drag on the gas where k_source and both transports walk strips of
+    two rings, the last of them shorter, without and with a rotating frame."""
+    over = dict(forced_circular=0, corotating=_capi.FRAME_COROTATING) if frame else {}
+    p, pl = gas_planet(nrad=41, nsec=1536, **over)
+    fp = _capi.dust_fluid_default_params(sfta=0, dust_feedback=1, dust_to_gas_density_ratio=0.1, sizepart=1e-2)
+    o, so, d, sg = df_pair(p, pl, fp)
+    n_o = o.algogas(DT / 20)
+    d.algogas(DT / 20)
+    assert d.status().last_call_substeps == n_o
+    compare(o, d, p, 1e-12, 1e-12, 1e-12)
+    compare_dust(o, d, p, 1e-12)
+
+
 def test_alpha_viscosities_open_edge():
     p, pl = gas_planet(nrad=32, nsec=96, viscosity=0.0, alpha_viscosity=1e-3, boundary=_capi.BC_OPEN)
     fp = _capi.dust_fluid_default_params(sfta=0, sizepart=1e-2, dalpha_viscosity=1e-4, dust_diffusion=1)

@@ -59,6 +59,20 @@ def test_frames_fp64(name):
             assert abs(getattr(go, k)[i] - getattr(oo, k)[i]) <= 1e-13, (k, i)
 
 
+# strips of two rings in the source and transport walks, the last of them shorter
+@pytest.mark.parametrize("energy", [0, 1])
+def test_frame_strips_of_rings_fp64(energy):
+    p, pl = gas_planet(nrad=41, nsec=1536, forced_circular=0, corotating=_capi.FRAME_COROTATING,
+                       energy_equation=energy, beta_cooling=energy)
+    pl = dict(pl, feel_disk=[1], feel_others=[1])
+    o, so, d, sg = pair(p, pl)
+    n_o = o.algogas(DT / 20)
+    d.algogas(DT / 20)
+    assert d.status().last_call_substeps == n_o
+    assert np.array_equal(d.fargo_shift()[0], o.fargo_shift()[0])
+    compare(o, d, p, 1e-12, 1e-12, 1e-12)
+
+
 def _wkz_case(name):
     zones = dict(wave_killing_zones=1, wkz_rmin=0.55, wkz_rmax=2.2)
     if name == "axi":
