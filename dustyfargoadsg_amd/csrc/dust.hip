@@ -235,10 +235,10 @@ __device__ __forceinline__ bool dust_deposit_needed(const KArgs &a, const dfargo
 // given time step.  The gas vtheta is read in the fixed frame, vt + Rmed
 // OmegaFrame per cell (src/Dsys.c:316), with the frame rate before this
 // sub-step's frame update.  A particle outside the grid keeps its state
-// and has no cell (p_cell = -1).  Bound by its FP64 instructions, the logs and
-// divisions of the weights first (10^6 particles, CIC: 118 us; 176 us when each
-// stencil formed both its factors, in 213 registers instead of 126, and each
-// particle the planet's azimuth and smoothing length).
+// and has no cell (p_cell = -1).  Bound by the latency of its gathers (VALU busy
+// 40 %) at the four wavefronts a SIMD that 126 registers allow (10^6 particles,
+// CIC: 118 us; 176 us when each stencil formed both its factors, in 213
+// registers, and each particle the planet's azimuth and smoothing length).
 template <typename T, int S>
 __global__ void __launch_bounds__(256) k_dust_move(KArgs a, int startup, double timestep0) {
   dfargo_ctrl *c = a.ctrl;
@@ -765,7 +765,7 @@ template <typename T, int S> static void dust_launch_s(int id, const KArgs &a, h
   // the strips of the crowded rings (1024 x 3072, 10^6 grains gathered at the
   // gap's edges: 133 us with strips of 2, 131 of 4, 150 of 8, 203 of 16)
   const int segs = (a.ns + DEP_OWN - 1) / DEP_OWN;
-  const int strip = (long)a.nr * segs / 4 < 4096 ? 2 : 4;
+  const int strip = (long)a.nr * segs / 4 < 16L * a.num_cu ? 2 : 4;
   switch (id) {
     case KID_DUST_MOVE:
       if (np > 0) hipLaunchKernelGGL((k_dust_move<T, S>), dim3(pb), dim3(256), 0, s, a, force, timestep);

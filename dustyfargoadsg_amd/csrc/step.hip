@@ -1213,11 +1213,12 @@ __device__ __forceinline__ double lane_value(double v, int k) {
 // ActualiseGas copies of src/SourceEuler.c:598-630 are deferred to the end of
 // the sub-step), so no wavefront overwrites what another one still reads.
 //
-// Bound by VALU issue.  As tiles in LDS with a halo per stage the potential
-// was formed 1.9 times a cell (8 rings, FP64) and every operand went through
-// LDS behind a barrier: 121 us at 1024x3072 FP64, 98 us FP32 with
-// self-gravity; now 64 and 71 us.  The quotients by the sums of neighbouring densities (six a
-// cell) share two reciprocals.
+// VALU issue bounds it first (66-76 % of the time at 1024x3072), then the latency
+// that three or four wavefronts a SIMD leave uncovered.  As tiles in LDS with a
+// halo per stage the potential was formed 1.9 times a cell (8 rings, FP64) and
+// every operand went through LDS behind a barrier: 121 us at 1024x3072 FP64, 98 us
+// FP32 with self-gravity; now 64 and 71 us.  The quotients by the sums of
+// neighbouring densities (six a cell) share two reciprocals.
 //
 // Rings at a strip's ends take only the stages that its own rings need.
 //
@@ -1513,12 +1514,12 @@ __global__ void __launch_bounds__(256, src_occupancy(sizeof(T) == 8, E, X)) k_so
 // ring and a kernel of which `occupancy` wavefronts share a SIMD.  On a small
 // grid a SIMD has at most one wavefront, which is alone with its own latency:
 // the shortest strips for which that holds, up to four rings (64x192 FP32
-// transport: 1 ring 10.5 us, 2 rings 12.0; 200x400 FP64: 2 rings, 800 wavefronts,
-// 14.4, 1 ring, 1600, 15.9).  On larger ones the shortest walk times rounds of
+// transport: 1 ring 8.8 us, 2 rings 10.3; 200x400 FP64: 2 rings, 800 wavefronts,
+// 12.2, 1 ring, 1600, 13.3).  On larger ones the shortest walk times rounds of
 // wavefronts, since a last round that is nearly empty costs as much as a full
-// one (1024x3072 FP32 transport: 19 rings, 2970 wavefronts on 3072 places, 97 us;
-// 16 rings, 3520, 105; 28 rings, two wavefronts a SIMD on average but not
-// evenly, 114).
+// one (1024x3072 FP32 transport: 19 rings, 2970 wavefronts on 3072 places, 109 us;
+// 16 rings, 3520, 121; 28 rings, two wavefronts a SIMD on average but not
+// evenly, 127).
 static int strip_rings(const KArgs &a, int columns, int occupancy, int extra, int most) {
   const long simds = 4L * a.num_cu;
   for (int S = 1; S <= 4; S++)
@@ -1656,17 +1657,18 @@ template <typename T, int K> __global__ void __launch_bounds__(RING_LB(K)) k_ene
 // Radial and azimuthal pass as kernels of their own took 87 + 76 us at 1024x3072
 // with FP64 storage (five quantities written by one and read by the other, 250
 // MB) and 78 + 75 us with FP32 storage.  Together they take 104 and 113 us: they
-// read the state and write the transported quantities once.  With FP32 storage
-// the radially transported quantities still round to it between the passes,
-// each by its own draw, as where a grid held them (97 us without that rounding
-// and with products shared across the quantities, but other values: see the
-// operations' order above).  What is counted beyond
-// that is instructions: each Work value Q / (rho + 1e-20), difference, slope,
-// face value and flux is formed once (tiles in LDS formed every radial face
-// twice and 10/8 of the slopes: 90 us for the radial pass alone).  A strip
-// repeats the Work of four rings and the slopes of two at its ends, a wavefront
-// eight of its 64 columns; strip_rings picks S.  FP64 whatever the storage
-// type.
+// read the state and write the transported quantities once.  VALU issue bounds
+// them first (75 and 81 % of the time), then the latency that three wavefronts a
+// SIMD leave uncovered.  With FP32 storage the radially transported quantities
+// still round to it between the passes, each by its own draw, as where a grid
+// held them (97 us without that rounding and with products shared across the
+// quantities, but other values: see the operations' order above).  What is
+// counted beyond the memory's traffic is instructions: each Work value
+// Q / (rho + 1e-20), difference, slope, face value and flux is formed once (tiles
+// in LDS formed every radial face twice and 10/8 of the slopes: 90 us for the
+// radial pass alone).  A strip repeats the Work of four rings and the slopes of
+// two at its ends, a wavefront eight of its 64 columns; strip_rings picks S.
+// FP64 whatever the storage type.
 //
 // The ring quantities of the FARGO scheme come first, from the per-tile sums
 // k_source leaves of the velocity before transport: the mean VMed
