@@ -97,10 +97,39 @@ __device__ __forceinline__ double div_nr(double a, double b) {
 __device__ __forceinline__ double dmin2(double a, double b) { return (b < a) ? b : a; }
 __device__ __forceinline__ double dmax2(double a, double b) { return (b > a) ? b : a; }
 
-// Sum and minimum over a wavefront, the same in every lane, in a fixed order:
-// four row shifts and two row broadcasts by DPP (VALU moves) leave the total
-// in lane 63.  A shuffle butterfly goes through the LDS crossbar twelve times
-// for a double, each step waiting for the one before.
+// Sum and minimum over a wavefront, the same in every lane, in a fixed order, by
+// VALU moves: a shuffle butterfly goes through the LDS crossbar twelve times for
+// a double, each step waiting for the one before.
+//
+// The sum adds the halves, then quarters, ... then neighbours, a shuffle tree's
+// order (32, 16, 8, 4, 2, 1): a sum of the ring (the cooling time's mean
+// vtheta) enters every cell of it, so its last bit decides how single FP32 values
+// are stored, and self-gravitating discs let those grow (128x512 with cooling: 4e-5
+// after forty calls).  Halves and rows meet by gfx950's lane swaps, which given
+// one value twice leave both partners' in every lane; lanes within a row by
+// rotations (row_ror 8, 4, 2, 1 = 0x128, 0x124, 0x122, 0x121).
+template <int CTRL> __device__ __forceinline__ double row_rotate(double v) {
+  return __hiloint2double(__builtin_amdgcn_update_dpp(0, __double2hiint(v), CTRL, 0xf, 0xf, true),
+                          __builtin_amdgcn_update_dpp(0, __double2loint(v), CTRL, 0xf, 0xf, true));
+}
+__device__ __forceinline__ double wave_sum(double v) {
+  const unsigned l0 = (unsigned)__double2loint(v), h0 = (unsigned)__double2hiint(v);
+  const auto l1 = __builtin_amdgcn_permlane32_swap(l0, l0, false, false);
+  const auto h1 = __builtin_amdgcn_permlane32_swap(h0, h0, false, false);
+  v = __hiloint2double((int)h1[0], (int)l1[0]) + __hiloint2double((int)h1[1], (int)l1[1]);
+  const unsigned l2 = (unsigned)__double2loint(v), h2 = (unsigned)__double2hiint(v);
+  const auto l3 = __builtin_amdgcn_permlane16_swap(l2, l2, false, false);
+  const auto h3 = __builtin_amdgcn_permlane16_swap(h2, h2, false, false);
+  v = __hiloint2double((int)h3[0], (int)l3[0]) + __hiloint2double((int)h3[1], (int)l3[1]);
+  v += row_rotate<0x128>(v);
+  v += row_rotate<0x124>(v);
+  v += row_rotate<0x122>(v);
+  v += row_rotate<0x121>(v);
+  return v;
+}
+// row_shr:1, 2, 4, 8 = 0x111, 0x112, 0x114, 0x118; row_bcast:15, :31 = 0x142,
+// 0x143 (into the rows 1 and 3, then 2 and 3); lanes without a source keep their
+// own value; the total is in lane 63
 template <int CTRL, int ROWS> __device__ __forceinline__ double dpp_row(double v, double other) {
   const int lo = __double2loint(v), hi = __double2hiint(v);
   return __hiloint2double(__builtin_amdgcn_update_dpp(__double2hiint(other), hi, CTRL, ROWS, 0xf, false),
@@ -109,18 +138,6 @@ template <int CTRL, int ROWS> __device__ __forceinline__ double dpp_row(double v
 __device__ __forceinline__ double lane63(double v) {
   return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), 63),
                           __builtin_amdgcn_readlane(__double2loint(v), 63));
-}
-// row_shr:1, 2, 4, 8 = 0x111, 0x112, 0x114, 0x118; row_bcast:15, :31 = 0x142,
-// 0x143 (into the rows 1 and 3, then 2 and 3); lanes without a source take
-// the neutral value
-__device__ __forceinline__ double wave_sum(double v) {
-  v += dpp_row<0x111, 0xf>(v, 0.0);
-  v += dpp_row<0x112, 0xf>(v, 0.0);
-  v += dpp_row<0x114, 0xf>(v, 0.0);
-  v += dpp_row<0x118, 0xf>(v, 0.0);
-  v += dpp_row<0x142, 0xa>(v, 0.0);
-  v += dpp_row<0x143, 0xc>(v, 0.0);
-  return lane63(v);
 }
 __device__ __forceinline__ double wave_min(double v) {
   v = dmin2(v, dpp_row<0x111, 0xf>(v, v));
