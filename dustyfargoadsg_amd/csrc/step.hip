@@ -398,11 +398,15 @@ __global__ void __launch_bounds__(64) k_algogas_begin(KArgs a, double DT) {
 // microseconds on its own whatever the grid, so everything the ring mean of
 // vt does not enter shares the first reduction with it and the fields are
 // loaded before that reduction waits (up to six cells per thread; beyond, the
-// registers do not hold them).  The star's force needs no sum of its own: its
-// cells lie at one distance from it, so it is the barycentre sum times a
-// factor of the ring.
-template <typename T, int K> __global__ void __launch_bounds__(RING_LB(K)) k_cfl_ring(KArgs a) {
-  constexpr int M = 7;
+// registers do not hold them).  The star's force needs no sum of its own: the
+// ring's cells lie at one distance from it, so it is the barycentre sum times a
+// factor of the ring.  SG: with self-gravity it is summed cell by cell all the
+// same.  The two differ in the last bits, which through the indirect term enter
+// the potential of every cell; a cell whose vr passes zero then stores another
+// FP32 value, and gravity spreads it (128x384 and 128x512 with cooling: 4e-5 after
+// forty calls).  1024x3072 FP32 374 -> 381 us a sub-step, 512x1536 154.6 -> 155.6.
+template <typename T, int K, bool SG> __device__ __forceinline__ void cfl_ring(const KArgs &a) {
+  constexpr int M = SG ? 9 : 7;
   __shared__ double sh[16 * M];
   __shared__ double shmin[16], shf[16 * 4];
   const dfargo_ctrl *c = a.ctrl;
@@ -438,9 +442,10 @@ template <typename T, int K> __global__ void __launch_bounds__(RING_LB(K)) k_cfl
   double *part = a.ring_part + i;
   T cs_new[K];
   {
-    CSum m = {0, 0}, xb = {0, 0}, yb = {0, 0};
+    CSum m = {0, 0}, xb = {0, 0}, yb = {0, 0}, fx = {0, 0}, fy = {0, 0};
     double s = 0.0, css = 0.0;
     int crd = 0, cre = 0;
+    const double rsm = c->tg_rsm[0];
     const double g = a.gamma;
 #pragma unroll
     for (int k = 0; k < K; k++) {
@@ -456,11 +461,17 @@ template <typename T, int K> __global__ void __launch_bounds__(RING_LB(K)) k_cfl
         css += (double)cs_new[k];
       }
       const double cm = a.Surf[i] * dens;
+      const double xc = a.Rmed[i] * a.CosAz[j], yc = a.Rmed[i] * a.SinAz[j];
       m.add(cm);
-      xb.add(cm * (a.Rmed[i] * a.CosAz[j]));
-      yb.add(cm * (a.Rmed[i] * a.SinAz[j]));
+      xb.add(cm * xc);
+      yb.add(cm * yc);
+      if (SG) {
+        const double dist2 = (xc * xc + yc * yc) + rsm * rsm, inv3 = 1.0 / dist2 / sqrt(dist2);
+        fx.add(DF_G * cm * xc * inv3);
+        fy.add(DF_G * cm * yc * inv3);
+      }
     }
-    double v[M] = {s, (double)crd, (double)cre, m.value(), xb.value(), yb.value(), css};
+    const double v[9] = {s, (double)crd, (double)cre, m.value(), xb.value(), yb.value(), css, fx.value(), fy.value()};
 #pragma unroll
     for (int q = 0; q < M; q++) {
       if ((q == 2 || q == 6) && !a.energy) continue;
@@ -548,7 +559,7 @@ template <typename T, int K> __global__ void __launch_bounds__(RING_LB(K)) k_cfl
       a.ring_dt[i] = d;
     } else if (t < 6) {
       part[(long)(t - 1) * nr] = s;
-      if (t >= 4) {
+      if (t >= 4 && !SG) {
         // target 0, the star: G cellmass dx / d^3 with d one value on the ring
         // (no cell lies in its Hill radius, 1e-15)
         const double rsm = c->tg_rsm[0], dist2 = a.Rmed[i] * a.Rmed[i] + rsm * rsm;
@@ -557,6 +568,10 @@ template <typename T, int K> __global__ void __launch_bounds__(RING_LB(K)) k_cfl
         g[0] = f;
         if (hill) g[nr] = f;
       }
+    } else if (SG && t >= 7) {
+      double *g = part + (long)(5 + 2 * (t - 7)) * nr;
+      g[0] = s;
+      if (hill) g[nr] = s;
     } else {
       const double gcs = s / (double)ns;
       a.gcs[i] = gcs;
@@ -607,6 +622,12 @@ template <typename T, int K> __global__ void __launch_bounds__(RING_LB(K)) k_cfl
       if (t == 0) { g[0] = v[0]; g[2 * (long)nr] = v[1]; }
     }
   }
+}
+template <typename T, int K> __global__ void __launch_bounds__(RING_LB(K)) k_cfl_ring(KArgs a) {
+  cfl_ring<T, K, false>(a);
+}
+template <typename T, int K> __global__ void __launch_bounds__(RING_LB(K)) k_cfl_ring_sg(KArgs a) {
+  cfl_ring<T, K, true>(a);
 }
 
 // Cash-Karp RK5 of the star+planet problem (src/RungeKunta.c:14-91), a planet
@@ -2536,7 +2557,10 @@ static int finish_bx(const KArgs &a) {
 
 template <typename T> void launch_kernel(int id, const KArgs &a, hipStream_t s) {
   switch (id) {
-    case KID_CFL: RING_DISPATCH_K(wide_k(a.ns), k_cfl_ring, T, a, s, 0); break;
+    case KID_CFL:
+      if (a.sg) RING_DISPATCH_K(wide_k(a.ns), k_cfl_ring_sg, T, a, s, 0);
+      else RING_DISPATCH_K(wide_k(a.ns), k_cfl_ring, T, a, s, 0);
+      break;
     case KID_CONTROL:
       if (a.accrete) hipLaunchKernelGGL((k_control<T, true>), dim3(1), dim3(CtrlBlock<true>::n), 0, s, a);
       else hipLaunchKernelGGL((k_control<T, false>), dim3(1), dim3(CtrlBlock<false>::n), 0, s, a);
