@@ -3,7 +3,7 @@
  *
  * TEST INFRASTRUCTURE ONLY.  Nothing in the product links or loads this
  * code; only tests/, __graft_entry__.smoke() and bench.py's cpu_baseline
- * leg use it, as the checker the HIP path is compared against.
+ * leg use it, as what the HIP path is compared with.
  *
  * The reference cannot be built here: its sources include headers that
  * src/varparser.pl generates at build time (param.h, global_ex.h, sg_ex.h),

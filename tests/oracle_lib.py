@@ -1,7 +1,7 @@
 """numpy wrapper of oracle/liboracle.so (the FP64 CPU restatement).
 
 Test infrastructure: used only by tests/, __graft_entry__.smoke() and
-bench.py's cpu_baseline leg, always as the checker.
+bench.py's cpu_baseline leg, always as what results are compared with.
 """
 import ctypes
 import os
